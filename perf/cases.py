@@ -1,0 +1,551 @@
+"""Measured workloads of the engine, through its Python entry points.
+
+A case is a dict of plain values; ``kind`` names what a pass does:
+
+  run      ``steps`` steps of one system, then its state read back (and, with
+           ``props``, its energies and virials): what a run script does
+           between two samples or frames
+  batch    the same for an ensemble of independent replicas stepped together
+  forces   an outer driver (a minimiser, a Newton-Krylov solver): positions
+           set, forces read, one Hessian-vector product
+  sample   ``steps`` steps, then the elastomers' observables: unfolded
+           positions, centres of mass, cluster virial
+  adjoint  one evaluation of a fit: the initial state restored, ``steps``
+           steps and the gradient of a loss with respect to every element's
+           modulus and the pair potential's parameters
+
+``system`` names what is simulated, ``n`` the solvent particles it is sized
+by (the sheet: solvent and elements both scale with it), ``skin`` 0 the
+per-step cell walk.  Inputs are seeded; positions and parameters are the
+float32 values that the engine holds.
+
+``exact`` integrates the same inputs in float64 with plain torch.
+"""
+from __future__ import annotations
+
+import math
+
+import numpy as np
+import torch
+
+from femmd_old_amd import Batch, System, configs
+
+RC = configs.RC_LJ
+
+
+# ---------------------------------------------------------------------------
+# cases
+# ---------------------------------------------------------------------------
+def listed():
+    return [
+        # one time step per call (an outer program advancing a small liquid by
+        # itself): latency and launches
+        dict(name="one step, 256 liquid", kind="run", system="liquid", n=256, steps=1, skin=0.6),
+        # the small hybrid of the tests between two samples of a script
+        dict(name="hybrid 4k, 20 steps", kind="run", system="disk", n=4000, steps=20, skin=0.6),
+        # a typed mixture of unequal particles, its energies sampled
+        dict(name="mixture 30k, 50 steps", kind="run", system="mixture", n=30011, steps=50, skin=0.6,
+             props=True),
+        # the headline system at a tenth of its size and in full
+        dict(name="hybrid 114k, 50 steps", kind="run", system="hybrid", n=104858, steps=50, skin=0.6),
+        dict(name="hybrid 1.1M, 100 steps", kind="run", system="hybrid", n=1048576, steps=100,
+             skin=0.6),
+        # the same forces with the cells walked every step
+        dict(name="cell walk 114k, 50 steps", kind="run", system="hybrid", n=104858, steps=50,
+             skin=0.0, props=True),
+        # elements and bonds as the larger part of the work
+        dict(name="bonded 1.1M, 50 steps", kind="run", system="bonded", n=600000, steps=50, skin=0.6),
+        # an ensemble of uneven replicas.  (Batch.tune is left out: its choice
+        # hangs on timings and changes no result)
+        dict(name="512 replicas, 100 steps", kind="batch", replicas=512, n_min=256, n_max=32768,
+             steps=100),
+        dict(name="forces and HVP, 57k", kind="forces", system="hybrid", n=52429, skin=0.6),
+        dict(name="sample elastomers, 56k", kind="sample", system="bonded", n=30000, steps=10,
+             skin=0.6),
+        # gradients: the trajectory stored, and the full sheet with checkpoints
+        dict(name="adjoint 23k, stored", kind="adjoint", n=20000, steps=50, ckpt=0),
+        dict(name="adjoint 233k, checkpoints", kind="adjoint", n=200000, steps=200, ckpt=20),
+    ]
+
+
+def _log(rng, lo, hi):
+    return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+
+def draw(rng):
+    kind = rng.choice(["run"] * 5 + ["batch", "forces", "sample", "adjoint"])
+    if kind == "run":
+        system = rng.choice(["liquid", "disk", "hybrid", "mixture", "bonded"])
+        lo, hi = {"liquid": (256, 1048576), "disk": (600, 60000), "hybrid": (4000, 1048576),
+                  "mixture": (400, 200000), "bonded": (3000, 600000)}[system]
+        n = _log(rng, lo, hi)
+        c = dict(kind=kind, system=system, n=n, steps=_log(rng, 1, 100),
+                 skin=rng.choice([0.6, 0.6, 0.6, 0.4, 0.0]))
+        if system == "mixture" or c["skin"] == 0.0:
+            c["props"] = True
+        return c
+    if kind == "batch":
+        n_min = _log(rng, 256, 2048)
+        return dict(kind=kind, replicas=_log(rng, 2, 300), n_min=n_min,
+                    n_max=_log(rng, n_min + 64, 16384), steps=_log(rng, 5, 100))
+    if kind == "forces":
+        return dict(kind=kind, system=rng.choice(["liquid", "disk", "hybrid", "bonded"]),
+                    n=_log(rng, 3000, 60000), skin=rng.choice([0.6, 0.4, 0.0]))
+    if kind == "sample":
+        return dict(kind=kind, system=rng.choice(["hybrid", "bonded"]), n=_log(rng, 4000, 200000),
+                    steps=_log(rng, 1, 30), skin=0.6)
+    return dict(kind=kind, n=_log(rng, 1500, 100000), steps=_log(rng, 5, 60),
+                ckpt=rng.choice([0, 7, 20]))
+
+
+# ---------------------------------------------------------------------------
+# inputs
+# ---------------------------------------------------------------------------
+def _grid(rng, n, spacing, jitter):
+    """n of the sites of a square lattice over a periodic box, jittered."""
+    m = math.ceil(math.sqrt(n))
+    L = m * spacing
+    g = (np.arange(m) + 0.5) * spacing
+    X, Y = np.meshgrid(g, g)
+    pick = np.sort(rng.permutation(m * m)[:n])
+    x = X.ravel()[pick] + rng.uniform(-jitter, jitter, n)
+    y = Y.ravel()[pick] + rng.uniform(-jitter, jitter, n)
+    return L, x, y
+
+
+def _liquid(n, seed):
+    rng = np.random.default_rng(seed)
+    L, x, y = _grid(rng, n, 1.118, 0.1)  # density 0.8
+    vx, vy = configs.maxwell(rng, n, 1.0, np.ones(n))
+    return configs.Workload("liquid", L, L, 0.005, x, y, vx, vy, np.ones(n), np.ones(n), seed=seed)
+
+
+def _stirred(w, seed):
+    """A workload whose sizes come from the case alone (disk radii, replica
+    sizes), with velocities, moduli and solvent displacements of the seed."""
+    rng = np.random.default_rng(seed)
+    n, k = w.n_total, w.n_solvent
+    free = np.ones(k, bool)
+    if w.bonds is not None:
+        free[w.bonds[0]] = False  # anchors stay at their bonds' rest length
+    w.x = np.mod(w.x + free * rng.uniform(-0.03, 0.03, k), w.Lx)
+    w.y = np.mod(w.y + free * rng.uniform(-0.03, 0.03, k), w.Ly)
+    vx, vy = configs.maxwell(rng, n, w.T, np.ones(n))
+    w.vx, w.vy, w._node_v = vx[:k], vy[:k], (vx[k:], vy[k:])
+    for el in w.elastomers:
+        el.E = el.E * rng.uniform(0.8, 1.2, len(el.E))
+    return w
+
+
+def _mixture(n, seed):
+    """Six types with symmetric tables and sigmas in [0.9, 1.1]."""
+    rng = np.random.default_rng(seed)
+    L, x, y = _grid(rng, n, 1.2, 0.08)
+    nt = 6
+
+    def table(lo, hi):
+        a = rng.uniform(lo, hi, (nt, nt))
+        return ((a + a.T) / 2).astype(np.float32).ravel()
+
+    w = configs.Workload("mixture", L, L, 0.004, x, y, rng.normal(0, 0.7, n), rng.normal(0, 0.7, n),
+                         rng.choice([1.0, 1.5], n), rng.uniform(0.9, 1.1, n), seed=seed)
+    w.tables = (table(0.5, 1.5), table(1.6, 2.6), table(-0.05, 0.05))
+    w.types = rng.integers(0, nt, n).astype(np.int32)
+    return w
+
+
+def _workload(case, seed):
+    n, system = case["n"], case.get("system", "sheet")
+    if system == "liquid":
+        return _liquid(n, seed)
+    if system == "disk":
+        return configs.c2(seed=seed, n_solvent=n, n_disks=1, radius=10.0)
+    if system == "mixture":
+        return _mixture(n, seed)
+    if system == "hybrid":
+        return configs.c2(seed=seed, scale=n / 1048576)
+    if system == "bonded":
+        return _stirred(configs.c3(scale=n / 600000), seed)
+    return configs.c5(seed=seed, scale=n / 200000)
+
+
+def _replicas(case, seed):
+    ws = configs.c4(n_replicas=case["replicas"], n_min=case["n_min"], n_max=case["n_max"])
+    return [_stirred(w, seed * 1009 + r) for r, w in enumerate(ws)]
+
+
+def _build(w, skin, commit=True):
+    if not hasattr(w, "tables"):
+        return configs.build_system(w, commit=commit, skin=skin)
+    s = System(w.Lx, w.Ly, dt=w.dt)
+    s.set_skin(skin)
+    s.set_pair_potential(*w.tables)
+    s.add_particles(w.x, w.y, w.vx, w.vy, w.mass, w.sigma, w.types)
+    s.allocate_cuda()
+    return s
+
+
+def _moved(case, seed, w):
+    """Positions an outer driver proposes, and a direction: float32."""
+    rng = np.random.default_rng(seed + 1)
+    ga = w.global_arrays()
+    n = w.n_total
+    x = np.mod(ga["x"] + rng.normal(0, 0.01, n), w.Lx).astype(np.float32)
+    y = np.mod(ga["y"] + rng.normal(0, 0.01, n), w.Ly).astype(np.float32)
+    x[x >= np.float32(w.Lx)] = 0.0
+    y[y >= np.float32(w.Ly)] = 0.0
+    d = rng.normal(0, 1, (2, n)).astype(np.float32)
+    return x, y, d[0], d[1]
+
+
+def _fit(w):
+    """The sheet's free nodes and the shape they are fitted to: the sheet bent
+    by one smooth mode."""
+    m = w.global_arrays()["mass"]
+    ids = np.arange(w.n_solvent, w.n_total)
+    ids = ids[np.isfinite(m[ids])].astype(np.int32)
+    ga = w.global_arrays()
+    x, y = ga["x"][ids], ga["y"][ids]
+    b = 0.05 * np.sin(2 * np.pi * y / w.Ly)
+    return ids, np.stack([x + b, y - 0.5 * b], 1).astype(np.float32)
+
+
+def prepare(case, seed):
+    if case["kind"] == "batch":
+        systems = [configs.build_system(w, commit=False) for w in _replicas(case, seed)]
+        return dict(case=case, batch=Batch(systems), systems=systems)
+    w = _workload(case, seed)
+    st = dict(case=case, sys=_build(w, case.get("skin", 0.6)))
+    if case["kind"] == "forces":
+        st["at"] = _moved(case, seed, w)
+    if case["kind"] == "adjoint":
+        st["start"] = st["sys"].get_state()
+        st["fit"] = _fit(w)
+    return st
+
+
+# ---------------------------------------------------------------------------
+# one pass
+# ---------------------------------------------------------------------------
+_PROPS = ("ke", "u_lj", "w_lj", "u_fea", "w_fea")
+
+
+def run(state):
+    case = state["case"]
+    kind = case["kind"]
+    if kind == "batch":
+        b = state["batch"]
+        b.run(case["steps"])
+        got = [b.get_state(r) for r in range(len(b))]
+        return [np.concatenate(v) for v in zip(*got)]
+    s = state["sys"]
+    if kind == "run":
+        s.run(case["steps"])
+        out = dict(state=s.get_state())
+        if case.get("props"):
+            e = s.energies()
+            out["props"] = [e[k] for k in _PROPS]
+        return out
+    if kind == "sample":
+        s.run(case["steps"])
+        c = s.cluster_props(unfolded=True)
+        return dict(c, virial=s.cluster_virial())
+    if kind == "forces":
+        x, y, dx, dy = state["at"]
+        s.set_state(x, y)
+        fx, fy = s.get_forces()
+        jx, jy, dE, deps, dsigma = s.force_jvp(dx, dy)
+        return dict(f=(fx, fy), j=(jx, jy), dE=dE, deps=deps, dsigma=dsigma)
+    s.set_state(*state["start"])
+    ids, target = state["fit"]
+    return s.adjoint(case["steps"], ids, target, ckpt=case["ckpt"])
+
+
+# ---------------------------------------------------------------------------
+# work a pass cannot do without
+# ---------------------------------------------------------------------------
+def _sizes(case):
+    """particles, elements, bonds, interacting pairs (each once)."""
+    def of(n_solvent, nodes, tri, bonds, rho, rc):
+        n = n_solvent + nodes
+        return n, tri, bonds, 0.5 * n * rho * math.pi * rc * rc
+
+    kind = case["kind"]
+    if kind == "batch":
+        lo, hi = case["n_min"], case["n_max"]
+        mean = (hi - lo) / math.log(hi / lo)
+        return of(case["replicas"] * mean, 182 * case["replicas"], 320 * case["replicas"], 0, 0.75, RC)
+    n, system = case["n"], case.get("system", "sheet")
+    if system == "hybrid":
+        return of(n, n * 93184 / 1048576, n * 153600 / 1048576, 0, 0.8, RC)
+    if system == "bonded":
+        return of(n, n * 512572 / 600000, n * 866616 / 600000, n * 32768 / 600000, 0.5, RC)
+    if system == "sheet":
+        return of(n, n * 32768 / 200000, n * 64770 / 200000, 0, 0.7, configs.RC_WCA)
+    if system == "disk":
+        return of(n, 367, 672, 0, 0.8, RC)
+    return of(n, 0, 0, 0, 0.8 if system == "liquid" else 0.69, RC if system == "liquid" else 2.1)
+
+
+def work(case):
+    n, tri, bonds, pairs = _sizes(case)
+    # per evaluation of the forces: a state read and written (32 bytes a
+    # particle), an element's nodes, reference shape and moduli (52), a bond's
+    # ends, stiffness and length (16); 22 operations a pair, 250 an element,
+    # 40 a bond, 20 a particle
+    step_b = 32 * n + 52 * tri + 16 * bonds
+    step_f = 22 * pairs + 250 * tri + 40 * bonds + 20 * n
+    kind, steps = case["kind"], case.get("steps", 1)
+    if kind == "forces":  # positions, direction in; forces, product, dE out
+        return dict(bytes=32 * n + 2 * 52 * tri + 8 * tri, flops=3 * step_f)
+    if kind == "adjoint":  # backward: cotangents read and written, dE
+        return dict(bytes=steps * (step_b + 40 * n + 68 * tri), flops=3 * steps * step_f)
+    out = dict(bytes=steps * step_b + 16 * n, flops=steps * step_f)
+    if kind == "sample":
+        out["flops"] += 22 * pairs
+    return out
+
+
+# ---------------------------------------------------------------------------
+# the same in float64
+# ---------------------------------------------------------------------------
+class _Exact:
+    """One system in float64 (positions, parameters and box as the float32
+    values the engine is given), half pair lists, index_add scatter."""
+
+    def __init__(self, w):
+        self.dev = "cuda" if torch.cuda.is_available() else "cpu"
+        ga = w.global_arrays()
+        f32 = lambda a: self.put(np.asarray(a, np.float32).astype(np.float64))  # noqa: E731
+        self.L = torch.tensor([float(np.float32(w.Lx)), float(np.float32(w.Ly))], dtype=torch.float64,
+                              device=self.dev)
+        self.dt = float(np.float32(w.dt))
+        self.x = torch.stack([f32(ga["x"]), f32(ga["y"])], 1)
+        self.ref = self.x.clone()
+        self.x = self.wrap(self.x)
+        vx, vy = configs.node_velocities(w)
+        self.v = torch.stack([f32(vx), f32(vy)], 1)
+        m = ga["mass"]
+        ok = np.isfinite(m) & (m > 0)
+        self.mass = f32(np.where(ok, m, 0.0))
+        self.im = f32(np.where(ok, 1.0 / np.where(ok, m, 1.0), 0.0))[:, None]
+        self.sig = f32(ga["sigma"])
+        self.excl = self.put(ga["excl"].astype(np.int64))
+        if hasattr(w, "tables"):
+            self.nt = int(round(math.sqrt(len(w.tables[0]))))
+            self.eps, self.rc, self.shift = (f32(t) for t in w.tables)
+            self.typ = self.put(w.types.astype(np.int64))
+        else:
+            self.nt, self.typ = 1, torch.zeros(len(m), dtype=torch.int64, device=self.dev)
+            self.eps, self.rc, self.shift = f32([w.eps]), f32([w.rc]), f32([w.ushift])
+        self.tri = self.put(ga["tri"].astype(np.int64))
+        self.E, self.nu = f32(ga["E"]), f32(ga["nu"])
+        self.bonds = None
+        if w.bonds is not None:
+            i, j, k, r0 = w.bonds
+            self.bonds = (self.put(np.asarray(i, np.int64)), self.put(np.asarray(j, np.int64)),
+                          f32(k), f32(r0))
+        if len(self.tri):
+            X = self.ref[self.tri]
+            D = torch.stack([X[:, 0] - X[:, 2], X[:, 1] - X[:, 2]], 2)
+            self.A0 = 0.5 * torch.linalg.det(D)
+            self.B = torch.linalg.inv(D)
+        self.scale = torch.ones((), dtype=torch.float64, device=self.dev)  # common sigma factor
+        self.built = None
+        self.reach = float(self.rc.max() * self.sig.max())
+        self.parts = {}
+
+    def put(self, a):
+        return torch.from_numpy(np.ascontiguousarray(a)).to(self.dev)
+
+    def wrap(self, x):
+        return x - torch.floor(x / self.L) * self.L
+
+    def image(self, d):
+        return d - torch.where(d >= 0.5 * self.L, self.L, torch.zeros_like(d)) + \
+            torch.where(d < -0.5 * self.L, self.L, torch.zeros_like(d))
+
+    def near(self, x, radius):
+        """Every unordered pair within radius, by cells (all pairs where the
+        box holds fewer than three cells)."""
+        n = len(x)
+        nc = torch.floor(self.L / radius).to(torch.int64)
+        got = []
+        if int(nc.min()) < 3:
+            i, j = torch.triu_indices(n, n, 1, device=self.dev)
+            got.append((i, j))
+        else:
+            c = torch.minimum((x / self.L * nc).to(torch.int64), nc - 1)
+            key = c[:, 0] + c[:, 1] * nc[0]
+            order = torch.argsort(key)
+            count = torch.bincount(key, minlength=int(nc.prod()))
+            start = torch.cumsum(count, 0) - count
+            most = int(count.max())
+            rank = torch.empty_like(order)
+            rank[order] = torch.arange(n, device=self.dev)
+            rank -= start[key]
+            for ox, oy in ((0, 0), (1, 0), (-1, 1), (0, 1), (1, 1)):
+                k2 = (c[:, 0] + ox) % nc[0] + ((c[:, 1] + oy) % nc[1]) * nc[0]
+                for k in range(most):
+                    i = torch.nonzero((k < count[k2]) & ((rank < k) if ox == oy == 0 else True))[:, 0]
+                    got.append((i, order[start[k2[i]] + k]))
+        keep_i, keep_j = [], []
+        for i, j in got:
+            d = self.image(x[i] - x[j])
+            e = self.excl[i]
+            m = ((d * d).sum(1) < radius * radius) & ~((e >= 0) & (e == self.excl[j]))
+            keep_i.append(i[m])
+            keep_j.append(j[m])
+        return torch.cat(keep_i), torch.cat(keep_j)
+
+    def pairs(self, x, margin=0.8):
+        with torch.no_grad():
+            x = x.detach()
+            if self.built is None or float(self.image(x - self.built).abs().max()) > 0.35 * margin:
+                self.i, self.j = self.near(x, self.reach + margin)
+                self.built = x.clone()
+            d = self.image(x[self.i] - x[self.j])
+            r2 = (d * d).sum(1)
+            s = 0.5 * (self.sig[self.i] + self.sig[self.j])
+            t = self.typ[self.i] * self.nt + self.typ[self.j]
+            hit = r2 < (self.rc[t] * s) ** 2
+            return self.i[hit], self.j[hit], s[hit], t[hit]
+
+    def forces(self, x, energies=False):
+        i, j, s, t = self.pairs(x)
+        s = s * self.scale
+        d = self.image(x[i] - x[j])
+        r2 = (d * d).sum(1)
+        s6 = (s * s / r2) ** 3
+        fij = (48 * self.eps[t] * (s6 * s6 - 0.5 * s6) / r2)[:, None] * d
+        f = torch.zeros_like(x).index_add(0, i, fij).index_add(0, j, -fij)
+        if energies:
+            self.parts["u_lj"] = (4 * self.eps[t] * (s6 * s6 - s6) + self.shift[t]).sum()
+            self.parts["w_lj"] = (fij * d).sum()
+        self.last = (i, j, fij)
+        if len(self.tri):
+            p0, p1, p2 = x[self.tri[:, 0]], x[self.tri[:, 1]], x[self.tri[:, 2]]
+            e1, e2 = self.image(p1 - p0), self.image(p2 - p0)
+            D = torch.stack([-e2, e1 - e2], 2)
+            F = torch.bmm(D, self.B)
+            J = F[:, 0, 0] * F[:, 1, 1] - F[:, 0, 1] * F[:, 1, 0]
+            C = torch.stack([torch.stack([F[:, 1, 1], -F[:, 1, 0]], 1),
+                             torch.stack([-F[:, 0, 1], F[:, 0, 0]], 1)], 1) / J[:, None, None]
+            lam = self.E * self.nu / ((1 - 2 * self.nu) * (1 + self.nu))
+            mu = self.E / (2 * (1 + self.nu))
+            lJ = torch.log(J)
+            P = mu[:, None, None] * (F - C) + (lam * lJ)[:, None, None] * C
+            H = -self.A0[:, None, None] * torch.bmm(P, self.B.transpose(1, 2).contiguous())
+            f = f.index_add(0, self.tri[:, 0], H[:, :, 0]).index_add(0, self.tri[:, 1], H[:, :, 1])
+            f = f.index_add(0, self.tri[:, 2], -H[:, :, 0] - H[:, :, 1])
+            if energies:
+                I1 = (F * F).sum((1, 2))
+                self.parts["u_fea"] = (self.A0 * (0.5 * mu * (I1 - 2) - mu * lJ +
+                                                  0.5 * lam * lJ * lJ)).sum()
+                self.parts["w_fea"] = (H * D).sum()
+        if self.bonds is not None:
+            i, j, k, r0 = self.bonds
+            d = self.image(x[i] - x[j])
+            r = torch.sqrt((d * d).sum(1))
+            fb = (-k * (r - r0) / r)[:, None] * d
+            f = f.index_add(0, i, fb).index_add(0, j, -fb)
+        return f
+
+    def steps(self, n, x, v):
+        h = 0.5 * self.dt
+        a = self.forces(x, n == 0) * self.im
+        for k in range(n):
+            v = v + h * a
+            x = self.wrap(x + self.dt * v)
+            a = self.forces(x, k == n - 1) * self.im
+            v = v + h * a
+        return x, v
+
+
+def _numpy(*tensors):
+    out = [t.detach().cpu().numpy() for t in tensors]
+    return out[0] if len(out) == 1 else out
+
+
+def _columns(x, v):
+    return _numpy(x[:, 0], x[:, 1], v[:, 0], v[:, 1])
+
+
+def _exact_sample(w, n):
+    """The elastomers' observables after n steps: clusters in the order of the
+    workload's elastomers."""
+    q = _Exact(w)
+    x, v = q.steps(n, q.x, q.v)
+    L, m = q.L, q.mass
+    first = w.n_solvent
+    ux = x.clone()
+    mass, cm, vcm, mid = [], [], [], []
+    cid = torch.full((len(x),), -1, dtype=torch.int64, device=q.dev)
+    for c, el in enumerate(w.elastomers):
+        at = slice(first, first + len(el.verts))
+        first = at.stop
+        cid[at] = c
+        p = x[at]
+        wide = (p.amax(0) - p.amin(0)) > 0.5 * L
+        u = torch.where(wide & (p > 0.5 * L), p - L, p)
+        u = u + torch.where(wide & (u.mean(0) < 0), L, torch.zeros_like(L))
+        ux[at] = u
+        M = m[at].sum()
+        mass.append(M)
+        cm.append((m[at][:, None] * u).sum(0) / M)
+        vcm.append((m[at][:, None] * v[at]).sum(0) / M)
+        th = 2 * math.pi * p / L
+        mid.append(L * (torch.atan2(-torch.sin(th).sum(0), -torch.cos(th).sum(0)) + math.pi)
+                   / (2 * math.pi))
+    cm = torch.stack(cm)
+    i, j, fij = q.last
+    both = (cid[i] >= 0) & (cid[j] >= 0)
+    d = q.image(cm[cid[i[both]]] - cm[cid[j[both]]])
+    return dict(mass=_numpy(torch.stack(mass)), cm=_numpy(cm), vcm=_numpy(torch.stack(vcm)),
+                centroid=_numpy(torch.stack(mid)), ux=_numpy(ux[:, 0]), uy=_numpy(ux[:, 1]),
+                virial=float((fij[both] * d).sum()))
+
+
+def exact(case, seed):
+    kind = case["kind"]
+    if kind == "batch":
+        if case["replicas"] * case["steps"] > 4000:
+            return None  # every replica by itself: minutes
+        got = []
+        for w in _replicas(case, seed):
+            q = _Exact(w)
+            got.append(_columns(*q.steps(case["steps"], q.x, q.v)))
+        return [np.concatenate(c) for c in zip(*got)]
+    w = _workload(case, seed)
+    if kind == "sample":
+        return _exact_sample(w, case["steps"])
+    q = _Exact(w)
+    if kind == "run":
+        x, v = q.steps(case["steps"], q.x, q.v)
+        out = dict(state=_columns(x, v))
+        if case.get("props"):
+            e = dict(q.parts, ke=0.5 * (q.mass * (v * v).sum(1)).sum())
+            out["props"] = [float(e.get(k, 0.0)) for k in _PROPS]
+        return out
+    par = [q.E, q.eps, q.scale]
+    for p in par:
+        p.requires_grad_(True)
+    if kind == "forces":
+        x, y, dx, dy = (q.put(a.astype(np.float64)) for a in _moved(case, seed, w))
+        at = torch.stack([x, y], 1).requires_grad_(True)
+        d = torch.stack([dx, dy], 1)
+        f = q.forces(at)
+        g = torch.autograd.grad((f * d).sum(), [at] + par, allow_unused=True)
+        z = lambda t, like: torch.zeros_like(like) if t is None else t  # noqa: E731
+        # sigma is 1 for every particle: d/dsigma is d/dscale
+        return dict(f=_numpy(f[:, 0], f[:, 1]), j=_numpy(g[0][:, 0], g[0][:, 1]),
+                    dE=_numpy(z(g[1], q.E)), deps=float(g[2].sum()), dsigma=float(g[3]))
+    if case["steps"] > 60:
+        return None  # the liquid's chaos: a gradient of float32 steps is no longer that of these
+    ids, target = _fit(w)
+    x, _ = q.steps(case["steps"], q.x, q.v)
+    d = q.image(x[q.put(ids.astype(np.int64))] - q.put(target.astype(np.float64)))
+    loss = (d * d).sum() / len(ids)
+    g = torch.autograd.grad(loss, par)
+    return dict(loss=float(loss.detach()), dE=_numpy(g[0]), deps=float(g[1].sum()),
+                dsigma=float(g[2]))
