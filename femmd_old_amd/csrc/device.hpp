@@ -22,10 +22,12 @@ constexpr int kKickThreads = 256;
 constexpr int kElemThreads = 256;
 constexpr int kMaxPairTypes = 16;  // particle types of a pair table
 constexpr int kMaxListCap = 512;  // neighbour-list capacity per particle
-// Largest per-cell capacity: a row of 3 cells holds < 256 candidates, so the
-// list build buffers an entry as its one-byte offset in that row.
-constexpr int kMaxCellCap = 60;
-static_assert(3 * kMaxCellCap < 256, "one-byte list-build offsets");
+constexpr int kMaxCellCap = 60;   // largest per-cell capacity
+// List build: mask words (32 candidates each) of a row of 3 cells, and the
+// staging slots past a tile's particles that its candidate loop may read
+// (a row's run rounded up to the loop's unrolling).
+__host__ __device__ constexpr int list_build_words(int cell_cap) { return (3 * cell_cap + 31) / 32; }
+__host__ __device__ constexpr int list_build_pad(int cell_cap) { return 3 * cell_cap + 8; }
 constexpr int kMaxListGroups = kMaxListCap / 4;
 // A list slot's word: length in the low bits, kListImg when the particle's
 // neighbours include a halo cell across the periodic boundary (its entries
@@ -271,8 +273,8 @@ struct ForceArgs {
                                // entries need the minimum image | (k << 16),
                                // k the tile index of the particle whose list
                                // it is
-    int32_t lbuf;              // list build: stage entries in LDS (coalesced
-                               // column writes) when set
+    int32_t lbuf;              // list build: hit masks in LDS, lists ranked by
+                               // length, when set (else stored as found)
     int32_t gated_grid;        // list build grid when gated (resident workgroups)
     int32_t cell_cap;          // slots per cell (cell counts are capped at it)
     const float2 *xys;         // list mode: positions in sorted order

@@ -964,9 +964,9 @@ ForceArgs Engine::force_args() {
     f.nbr_cap = nbr_cap_;
     f.nbr = nbr_.p;
     f.nnum = nnum_.p;
-    // stage list entries in LDS when the tile and the buffer fit in 64 KB
+    // hit masks and ranking in LDS when they fit in 64 KB beside the staging
     // (static LDS of the kernel: ~2 KB)
-    f.lbuf = list_build_lds_bytes(lds_cap_, cap_, nbr_cap_, block_, true) <= 62 * 1024;
+    f.lbuf = list_build_lds_bytes(lds_cap_, cap_, nbr_cap_, block_, sigma_, true) <= 62 * 1024;
     f.cell_cap = cap_;
     f.gated_grid = lb_grid_;
     f.sigs = sigs_.p;

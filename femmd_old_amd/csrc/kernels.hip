@@ -89,36 +89,79 @@ __device__ __forceinline__ float shifted_diff(float p, float q, int k, float L) 
     return p - q;
 }
 
+// Reductions and scans over the 64 lanes of a wavefront by DPP moves (row
+// shifts, then the broadcasts of lane 15 of each row and of lane 31), all
+// lanes active.  A DPP step is one or two vector instructions; a step through
+// the LDS crossbar (shuffle) waits ~100 cycles, and these chains sit at the
+// end of nearly every workgroup.  Order of the sums: fixed.
+template <int kCtrl, int kRows>
+__device__ __forceinline__ int dpp_int(int old, int v) {
+    return __builtin_amdgcn_update_dpp(old, v, kCtrl, kRows, 0xf, false);
+}
+constexpr int kDppShr1 = 0x111, kDppShr2 = 0x112, kDppShr4 = 0x114, kDppShr8 = 0x118;
+constexpr int kDppBcast15 = 0x142, kDppBcast31 = 0x143;
+
+template <int kCtrl, int kRows>
+__device__ __forceinline__ float dpp_float(float old, float v) {
+    return __int_as_float(dpp_int<kCtrl, kRows>(__float_as_int(old), __float_as_int(v)));
+}
+template <int kCtrl, int kRows>
+__device__ __forceinline__ double dpp_double(double old, double v) {
+    return __hiloint2double(dpp_int<kCtrl, kRows>(__double2hiint(old), __double2hiint(v)),
+                            dpp_int<kCtrl, kRows>(__double2loint(old), __double2loint(v)));
+}
+__device__ __forceinline__ int lane63(int v) { return __builtin_amdgcn_readlane(v, 63); }
+__device__ __forceinline__ float lane63(float v) { return __int_as_float(lane63(__float_as_int(v))); }
+__device__ __forceinline__ double lane63(double v) {
+    return __hiloint2double(lane63(__double2hiint(v)), lane63(__double2loint(v)));
+}
 __device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    return v;
+    v += dpp_double<kDppShr1, 0xf>(0.0, v);
+    v += dpp_double<kDppShr2, 0xf>(0.0, v);
+    v += dpp_double<kDppShr4, 0xf>(0.0, v);
+    v += dpp_double<kDppShr8, 0xf>(0.0, v);
+    v += dpp_double<kDppBcast15, 0xa>(0.0, v);
+    v += dpp_double<kDppBcast31, 0xc>(0.0, v);
+    return lane63(v);
 }
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));
-    return v;
+    v = fmaxf(v, dpp_float<kDppShr1, 0xf>(v, v));
+    v = fmaxf(v, dpp_float<kDppShr2, 0xf>(v, v));
+    v = fmaxf(v, dpp_float<kDppShr4, 0xf>(v, v));
+    v = fmaxf(v, dpp_float<kDppShr8, 0xf>(v, v));
+    v = fmaxf(v, dpp_float<kDppBcast15, 0xa>(v, v));
+    v = fmaxf(v, dpp_float<kDppBcast31, 0xc>(v, v));
+    return lane63(v);
 }
 __device__ __forceinline__ double wave_max_d(double v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o));
-    return v;
+    v = fmax(v, dpp_double<kDppShr1, 0xf>(v, v));
+    v = fmax(v, dpp_double<kDppShr2, 0xf>(v, v));
+    v = fmax(v, dpp_double<kDppShr4, 0xf>(v, v));
+    v = fmax(v, dpp_double<kDppShr8, 0xf>(v, v));
+    v = fmax(v, dpp_double<kDppBcast15, 0xa>(v, v));
+    v = fmax(v, dpp_double<kDppBcast31, 0xc>(v, v));
+    return lane63(v);
 }
-__device__ __forceinline__ int wave_sum_int(int v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    return v;
+__device__ __forceinline__ int wave_max_int(int v) {
+    v = max(v, dpp_int<kDppShr1, 0xf>(v, v));
+    v = max(v, dpp_int<kDppShr2, 0xf>(v, v));
+    v = max(v, dpp_int<kDppShr4, 0xf>(v, v));
+    v = max(v, dpp_int<kDppShr8, 0xf>(v, v));
+    v = max(v, dpp_int<kDppBcast15, 0xa>(v, v));
+    v = max(v, dpp_int<kDppBcast31, 0xc>(v, v));
+    return lane63(v);
 }
 // Inclusive prefix sum over the 64 lanes of a wavefront.
 __device__ __forceinline__ int wave_incl_scan(int v) {
-    int lane = threadIdx.x & 63;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        int t = __shfl_up(v, o);
-        if (lane >= o) v += t;
-    }
+    v += dpp_int<kDppShr1, 0xf>(0, v);
+    v += dpp_int<kDppShr2, 0xf>(0, v);
+    v += dpp_int<kDppShr4, 0xf>(0, v);
+    v += dpp_int<kDppShr8, 0xf>(0, v);
+    v += dpp_int<kDppBcast15, 0xa>(0, v);
+    v += dpp_int<kDppBcast31, 0xc>(0, v);
     return v;
 }
+__device__ __forceinline__ int wave_sum_int(int v) { return lane63(wave_incl_scan(v)); }
 
 // Deterministic block reduction of two doubles (fixed wave order); the
 // result is valid in thread 0.  red must hold 2 * (blockDim / 64) doubles.
@@ -1254,7 +1297,7 @@ __device__ int stage_layout(const ForceArgs &a, const Tile &T, const RepDesc &R,
     const int row = W + 2, S = 3 * row;
     const int tid = threadIdx.x;
     for (int s = tid; s < S; s += blockDim.x) {
-        const int r = s / row, col = s - r * row;
+        const int r = s >= 2 * row ? 2 : (s >= row ? 1 : 0), col = s - r * row;
         int cy = T.cy + r - 1;
         if (cy < 0) cy += R.ncy; else if (cy >= R.ncy) cy -= R.ncy;
         int cx = T.cx0 + col - 1;
@@ -1400,14 +1443,6 @@ __device__ void pair_tile(const ForceArgs &a, int tile, PairLds &L) {
 // from the current positions and gathers the neighbours from LDS.
 // ---------------------------------------------------------------------------
 
-// Stores group g (four LDS indices j[0..3]) of sorted position p.
-__device__ __forceinline__ void list_store_group(const ForceArgs &a, int g, int p,
-                                                 const int *j) {
-    const uint64_t v = (uint64_t)(uint16_t)j[0] | ((uint64_t)(uint16_t)j[1] << 16) |
-                       ((uint64_t)(uint16_t)j[2] << 32) | ((uint64_t)(uint16_t)j[3] << 48);
-    reinterpret_cast<uint64_t *>(a.nbr)[(size_t)g * a.n + p] = v;
-}
-
 // Stores slot k alone (list build without the LDS staging buffer).
 __device__ __forceinline__ void list_store_slot(const ForceArgs &a, int k, int p, int j) {
     reinterpret_cast<uint16_t *>(a.nbr)[((size_t)(k >> 2) * a.n + p) * 4 + (k & 3)] =
@@ -1440,15 +1475,44 @@ __device__ __forceinline__ ImgCols img_cols(const Tile &T, const RepDesc &R, int
     return c;
 }
 
+// Candidate pj within the list radius of pi (the margins of the radius cover
+// the rounding of the fused form).
+template <bool kWrap, bool kSigma>
+__device__ __forceinline__ bool list_near(const RepDesc &R, float2 pi, float2 pj, float si,
+                                          float sj) {
+    float dx = pi.x - pj.x;
+    float dy = pi.y - pj.y;
+    if (kWrap) {
+        // minimum image as two selects per axis
+        float ox = (dx >= R.hLx) ? R.Lx : 0.0f;
+        ox = (dx < -R.hLx) ? -R.Lx : ox;
+        float oy = (dy >= R.hLy) ? R.Ly : 0.0f;
+        oy = (dy < -R.hLy) ? -R.Ly : oy;
+        dx = dx - ox;
+        dy = dy - oy;
+    }
+    const float dr2 = __builtin_fmaf(dx, dx, dy * dy);
+    if (!kSigma) return dr2 < R.rl2_uniform;
+    const float rl = R.rc_list * ((si + sj) * 0.5f) + R.skin;
+    return dr2 < (rl * rl) * 1.00002f;
+}
+
+// Staging of the list build: positions (8 bytes: what the candidate loop
+// reads), exclusion groups and (mixed sigmas) sigma apart.
+struct BuildLds {
+    float2 *xy;
+    int *grp;
+    float *sig;
+};
+
 template <bool kWrap, bool kSigma>
 __device__ void list_tile_body_direct(const ForceArgs &a, const Tile &T, const RepDesc &R, int W,
-                                      PairLds &L) {
+                                      const PairLds &L, const BuildLds &B) {
     const ImgCols ic = img_cols(T, R, W);
     const int row = W + 2;
     const int c_lo = L.off[row + 1], c_hi = L.off[row + W + 1];
     const int nc = c_hi - c_lo;
     const int sbase = L.cstart[row + 1];
-    const float Lx = R.Lx, Ly = R.Ly, hLx = R.hLx, hLy = R.hLy;
     const int bd = blockDim.x;
     const int cap = a.nbr_cap;
     for (int k = threadIdx.x; k < nc; k += bd) {
@@ -1459,37 +1523,18 @@ __device__ void list_tile_body_direct(const ForceArgs &a, const Tile &T, const R
             if (L.off[mid] <= me) lo = mid; else hi = mid;
         }
         const int col = lo - row;
-        const float4 pi = L.ent[me];
-        const float xi = pi.x, yi = pi.y;
-        const int gi = __float_as_int(pi.z);
+        const float2 pi = B.xy[me];
+        const int gi = B.grp[me];
         const int gix = gi >= 0 ? gi : -2;
-        const float si = pi.w;
+        const float si = kSigma ? B.sig[me] : 0.0f;
         const int p = sbase + k;
         int cnt = 0;
 #pragma unroll
         for (int r = 0; r < 3; ++r) {
             const int j0 = L.off[r * row + col - 1], j1 = L.off[r * row + col + 2];
             for (int j = j0; j < j1; ++j) {
-                const float4 pj = L.ent[j];
-                float dx = xi - pj.x;
-                float dy = yi - pj.y;
-                if (kWrap) {
-                    float ox = (dx >= hLx) ? Lx : 0.0f;
-                    ox = (dx < -hLx) ? -Lx : ox;
-                    float oy = (dy >= hLy) ? Ly : 0.0f;
-                    oy = (dy < -hLy) ? -Ly : oy;
-                    dx = dx - ox;
-                    dy = dy - oy;
-                }
-                const float dr2 = dx * dx + dy * dy;
-                float rl2;
-                if (kSigma) {
-                    const float rl = R.rc_list * ((si + pj.w) * 0.5f) + R.skin;
-                    rl2 = (rl * rl) * 1.00002f;
-                } else {
-                    rl2 = R.rl2_uniform;
-                }
-                bool hit = (dr2 < rl2) & (__float_as_int(pj.z) != gix);
+                bool hit = list_near<kWrap, kSigma>(R, pi, B.xy[j], si, kSigma ? B.sig[j] : 0.0f) &
+                           (B.grp[j] != gix);
                 if (r == 1) hit &= (j != me);
                 if (hit) {
                     if (cnt < cap) list_store_slot(a, cnt, p, 8 * j);
@@ -1505,12 +1550,6 @@ __device__ void list_tile_body_direct(const ForceArgs &a, const Tile &T, const R
         a.nnum[p] = m | (kWrap && ic.needs(col, W) ? kListImg : 0) | (k << 16);
         if (cnt > cap) atomicOr(a.err, 16u);  // FM_DEV_LIST_OVERFLOW
     }
-}
-
-__device__ __forceinline__ int wave_max_int(int v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o));
-    return v;
 }
 
 // Rank of this lane's list among the active lanes of the workgroup: the
@@ -1553,29 +1592,56 @@ __device__ int list_rank(int n4, bool img, bool act, int capg, int *hist) {
     return act ? hist[key * nw + w] + __popcll(eq & before) : -1;
 }
 
-// List build of one staged tile through the LDS list buffer: slot k of lane
-// t at buf[k * (blockDim + 4) + t] holds the entry's offset in its row's run
-// of candidates (< 3 cell capacities <= 180: one byte; the lane's counts at
-// the two row ends tell the row): half the LDS of two-byte entries, so more
-// workgroups share a CU, which this latency-bound loop needs.  Each
-// row's candidate loop runs a wavefront-uniform trip count (the longest run
-// among the lanes; a lane past its own run is masked), and every candidate
-// is written to the lane's next buffer slot while only hits advance it, so
-// the loop has no branches.  Reads past a lane's run stay inside the
-// staging's headroom of 3 cells.
+// m with the lane's predicates h(0) .. h(7) shifted in at the low end, h(0)
+// first: one vector instruction each (m + m + carry-in).  The leading s_nop
+// keeps the two wait states gfx950 wants between the compare that wrote the
+// last predicate's scalar pair and its use as a carry.
+template <class H>
+__device__ __forceinline__ uint32_t shift_in8(uint32_t m, H &&h) {
+    unsigned long long c[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) c[u] = __ballot(h(u));
+    __asm__("s_nop 1\n\t"
+            "v_addc_co_u32 %0, vcc, %0, %0, %1\n\t"
+            "v_addc_co_u32 %0, vcc, %0, %0, %2\n\t"
+            "v_addc_co_u32 %0, vcc, %0, %0, %3\n\t"
+            "v_addc_co_u32 %0, vcc, %0, %0, %4\n\t"
+            "v_addc_co_u32 %0, vcc, %0, %0, %5\n\t"
+            "v_addc_co_u32 %0, vcc, %0, %0, %6\n\t"
+            "v_addc_co_u32 %0, vcc, %0, %0, %7\n\t"
+            "v_addc_co_u32 %0, vcc, %0, %0, %8"
+            : "+v"(m)
+            : "s"(c[0]), "s"(c[1]), "s"(c[2]), "s"(c[3]), "s"(c[4]), "s"(c[5]), "s"(c[6]), "s"(c[7])
+            : "vcc");
+    return m;
+}
+
+// List build of one staged tile; bound by vector issue.  Each row's
+// candidates (cells col-1 .. col+1, one contiguous run) are tested 32 at a
+// time into a bit mask per lane, with a wavefront-uniform trip count (the
+// longest run among the lanes; bits past a lane's own run and of the centre
+// itself are cleared afterwards): six vector instructions per candidate (8
+// with an exclusion group in the wavefront), where a compaction store per
+// candidate took 14 and conflicted in LDS.  The masks wait until the chunk's
+// lists are ranked -- in registers while every run of the wavefront is at
+// most 32 long, else in LDS (word w of lane t at mask[w * blockDim + t]) --
+// then each lane takes its set bits in order and stores its list in groups
+// of four.  The loop reads up to 7 slots past a lane's longest run: inside
+// the staging's headroom (list_build_pad).  A rebuild of 1.14 million
+// particles (lists of 21.7): 101 -> 82 us; 3.84 million in 512 replicas:
+// 543 -> 390 us.
 template <bool kWrap, bool kSigma>
-__device__ void list_tile_body_buf(const ForceArgs &a, const Tile &T, const RepDesc &R, int W,
-                                   PairLds &L, uint8_t *buf, int *hist) {
+__device__ void list_tile_body_mask(const ForceArgs &a, const Tile &T, const RepDesc &R, int W,
+                                    const PairLds &L, const BuildLds &B, uint32_t *mask, int *hist) {
     const ImgCols ic = img_cols(T, R, W);
     const int row = W + 2;
     const int c_lo = L.off[row + 1], c_hi = L.off[row + W + 1];
     const int nc = c_hi - c_lo;
     const int sbase = L.cstart[row + 1];
-    const float Lx = R.Lx, Ly = R.Ly, hLx = R.hLx, hLy = R.hLy;
     const int bd = blockDim.x;  // held in a register across the loops
-    const int bs = bd + 4;      // buffer row stride (bytes): a slot's rows rotate over the banks
     const int tid = threadIdx.x;
-    const int cap = a.nbr_cap, capm1 = a.nbr_cap - 1;
+    const int cap = a.nbr_cap;
+    const int wpr = list_build_words(a.cell_cap);  // mask words per row
     // every lane of a wavefront takes part in each pass (uniform loop)
     for (int k0 = 0; k0 < nc; k0 += bd) {
         const int k = k0 + tid;
@@ -1587,53 +1653,60 @@ __device__ void list_tile_body_buf(const ForceArgs &a, const Tile &T, const RepD
             if (L.off[mid] <= me) lo = mid; else hi = mid;
         }
         const int col = lo - row;
-        const float4 pi = L.ent[me];
-        const float xi = pi.x, yi = pi.y;
-        const int gi = __float_as_int(pi.z);
-        const int gix = gi >= 0 ? gi : -2;
-        const float si = pi.w;
-        int cnt = 0;
-        int jr[3], cr[2];  // each row's first candidate; the count after rows 0 and 1
-        // the three staged rows, each a contiguous run of candidates
-        // (cells col-1 .. col+1); the centre particle is in row 1 only
+        const float2 pi = B.xy[me];
+        const int gi = B.grp[me];
+        const int gix = gi >= 0 ? gi : -2;  // (-1 never matches -2)
+        const float si = kSigma ? B.sig[me] : 0.0f;
+        const bool excl = __ballot(act && gi >= 0) != 0ull;  // some lane has an exclusion group
+        int jr[3], len[3];  // each row's first candidate and run length
+        int most = 0;       // the wavefront's longest run
 #pragma unroll
         for (int r = 0; r < 3; ++r) {
-            const int j0 = L.off[r * row + col - 1];
-            jr[r] = j0;
-            const int len = act ? L.off[r * row + col + 2] - j0 : 0;
-            const int lmax = __builtin_amdgcn_readfirstlane(wave_max_int(len));
-#pragma unroll 2
-            for (int t = 0; t < lmax; ++t) {
-                const int j = j0 + t;
-                const float4 pj = L.ent[j];
-                float dx = xi - pj.x;
-                float dy = yi - pj.y;
-                if (kWrap) {
-                    // minimum image as two selects per axis
-                    float ox = (dx >= hLx) ? Lx : 0.0f;
-                    ox = (dx < -hLx) ? -Lx : ox;
-                    float oy = (dy >= hLy) ? Ly : 0.0f;
-                    oy = (dy < -hLy) ? -Ly : oy;
-                    dx = dx - ox;
-                    dy = dy - oy;
-                }
-                // the margins of the list radius cover the rounding of this
-                // fused form
-                const float dr2 = __builtin_fmaf(dx, dx, dy * dy);
-                float rl2;
-                if (kSigma) {
-                    const float rl = R.rc_list * ((si + pj.w) * 0.5f) + R.skin;
-                    rl2 = (rl * rl) * 1.00002f;
-                } else {
-                    rl2 = R.rl2_uniform;
-                }
-                bool hit = (t < len) & (dr2 < rl2) & (__float_as_int(pj.z) != gix);
-                if (r == 1) hit &= (j != me);
-                // (24-bit multiply: full rate; cnt <= cap <= 512, bs <= 260)
-                buf[__umul24(min(cnt, capm1), bs) + tid] = (uint8_t)t;
-                cnt += hit ? 1 : 0;
+            jr[r] = L.off[r * row + col - 1];
+            len[r] = act ? L.off[r * row + col + 2] - jr[r] : 0;
+            most = max(most, len[r]);
+        }
+        most = wave_max_int(most);
+        // hits among candidates b .. b + 31 of row r (n of them, uniform)
+        auto hits = [&](int r, int b, int n) -> uint32_t {
+            const int n8 = (n + 7) & ~7;
+            uint32_t m = 0;
+            for (int t = 0; t < n8; t += 8) {
+                const int j = jr[r] + b + t;
+                auto near = [&](int u) {
+                    return list_near<kWrap, kSigma>(R, pi, B.xy[j + u], si,
+                                                    kSigma ? B.sig[j + u] : 0.0f);
+                };
+                if (excl)
+                    m = shift_in8(m, [&](int u) { return near(u) & (B.grp[j + u] != gix); });
+                else
+                    m = shift_in8(m, near);
             }
-            if (r < 2) cr[r] = cnt;
+            m = __brev(m) >> (32 - n8);  // bit t: candidate jr[r] + b + t
+            const int left = len[r] - b;  // candidates of the lane's own run
+            m &= left >= 32 ? ~0u : (left > 0 ? (1u << left) - 1u : 0u);
+            if (r == 1) {
+                const int s = me - (jr[r] + b);
+                if (s >= 0 && s < 32) m &= ~(1u << s);
+            }
+            return m;
+        };
+        uint32_t m0 = 0, m1 = 0, m2 = 0;
+        int cnt;
+        if (most <= 32) {  // uniform per wavefront
+            m0 = hits(0, 0, most);
+            m1 = hits(1, 0, most);
+            m2 = hits(2, 0, most);
+            cnt = __popc(m0) + __popc(m1) + __popc(m2);
+        } else {
+            cnt = 0;
+#pragma unroll
+            for (int r = 0; r < 3; ++r)
+                for (int b = 0, w = 0; b < most; b += 32, ++w) {
+                    const uint32_t m = hits(r, b, min(most - b, 32));
+                    mask[(r * wpr + w) * bd + tid] = m;
+                    cnt += __popc(m);
+                }
         }
         const int m = min(cnt, cap);
         // the chunk's lists are stored longest first (list slot q = sbase +
@@ -1641,22 +1714,69 @@ __device__ void list_tile_body_buf(const ForceArgs &a, const Tile &T, const RepD
         // length; nnum[q] = length | (tile index k << 16)
         const bool img = kWrap && ic.needs(col, W);
         const int rank = list_rank((m + 3) >> 2, img, act, cap >> 2, hist);
-        if (act) {
-            const int p = sbase + k0 + rank;  // list slot
-            // groups of four, padded with the sentinel slot (staged far
-            // away: the pair pass's cutoff test rejects it); cap is a
-            // multiple of 8.
-            for (int g = 0; g < ((m + 3) >> 2); ++g) {
-                int jj[4];
+        // groups of four entries (offsets of staging slots, 8 bytes each),
+        // the last padded with the sentinel slot (staged far away: the pair
+        // pass's cutoff test rejects it); cap is a multiple of 8
+        const uint32_t pad = (uint32_t)(8 * a.lds_cap);
+        if (most <= 32) {
+            // a lane takes its rows' set bits in order: the row in hand is m0
+            // with first offset b0, an empty one is replaced by the next (the
+            // rows behind it move up), so every entry costs the same few
+            // instructions and the lanes store their groups together
+            uint32_t b0 = 8u * jr[0], b1 = 8u * jr[1], b2 = 8u * jr[2];
+            if (m1 == 0u) { m1 = m2; b1 = b2; m2 = 0u; }
+            if (m0 == 0u) { m0 = m1; b0 = b1; m1 = m2; b1 = b2; m2 = 0u; }
+            uint64_t *dst = reinterpret_cast<uint64_t *>(a.nbr) + (sbase + k0 + max(rank, 0));
+            const int g4 = wave_max_int((m + 3) >> 2);
+            for (int g = 0; g < g4; ++g) {
+                uint32_t off[4];
 #pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    const int kk = 4 * g + t;
-                    const int j0 = kk < cr[0] ? jr[0] : (kk < cr[1] ? jr[1] : jr[2]);
-                    jj[t] = kk < m ? 8 * (j0 + (int)buf[__umul24(kk, bs) + tid]) : 8 * a.lds_cap;
+                for (int u = 0; u < 4; ++u) {
+                    off[u] = (4 * g + u < m) ? b0 + 8u * (uint32_t)(__ffs(m0) - 1) : pad;
+                    m0 &= m0 - 1u;  // (0 stays 0)
+                    const bool z = m0 == 0u;
+                    m0 = z ? m1 : m0;
+                    b0 = z ? b1 : b0;
+                    m1 = z ? m2 : m1;
+                    b1 = z ? b2 : b1;
+                    m2 = z ? 0u : m2;
                 }
-                list_store_group(a, g, p, jj);
+                if (4 * g < m)
+                    dst[(size_t)g * a.n] = (uint64_t)(off[0] | (off[1] << 16)) |
+                                           ((uint64_t)(off[2] | (off[3] << 16)) << 32);
             }
-            a.nnum[p] = m | (img ? kListImg : 0) | (k << 16);
+        } else if (act) {
+            uint64_t *dst = reinterpret_cast<uint64_t *>(a.nbr) + (sbase + k0 + rank);
+            uint32_t g0 = 0, g1 = 0;  // the group being filled: entries enter at the top
+            int kk = 0;
+#pragma unroll
+            for (int r = 0; r < 3; ++r) {
+                for (int b = 0, w = 0; b < len[r]; b += 32, ++w) {
+                    uint32_t bits = mask[(r * wpr + w) * bd + tid];
+                    const int j8 = 8 * (jr[r] + b);
+                    while (bits != 0u && kk < m) {
+                        const uint32_t off = (uint32_t)(j8 + 8 * (__ffs(bits) - 1));
+                        bits &= bits - 1u;
+                        g0 = __builtin_amdgcn_alignbit(g1, g0, 16);
+                        g1 = __builtin_amdgcn_alignbit(off, g1, 16);
+                        ++kk;
+                        if ((kk & 3) == 0) {
+                            *dst = ((uint64_t)g1 << 32) | g0;
+                            dst += a.n;
+                        }
+                    }
+                }
+            }
+            if (kk & 3) {
+                for (; kk & 3; ++kk) {
+                    g0 = __builtin_amdgcn_alignbit(g1, g0, 16);
+                    g1 = __builtin_amdgcn_alignbit(pad, g1, 16);
+                }
+                *dst = ((uint64_t)g1 << 32) | g0;
+            }
+        }
+        if (act) {
+            a.nnum[sbase + k0 + rank] = m | (img ? kListImg : 0) | (k << 16);
             if (cnt > cap) atomicOr(a.err, 16u);  // FM_DEV_LIST_OVERFLOW
         }
     }
@@ -1668,17 +1788,22 @@ __global__ __launch_bounds__(256) void k_list_build(ForceArgs a) {
     __shared__ int s_cstart[kMaxSlots];
     __shared__ int s_off[kMaxSlots + 1];
     PairLds L;
-    L.ent = dyn;
+    L.ent = nullptr;
     L.typ = nullptr;
     L.sp = nullptr;
     L.cstart = s_cstart;
     L.off = s_off;
     L.pt = nullptr;  // the list radius comes from the replica (rc_list)
     L.red = nullptr;
-    // list buffer after the staging and its read headroom of 3 cells
-    uint8_t *buf = reinterpret_cast<uint8_t *>(dyn + a.lds_cap + 3 * a.cell_cap);
-    // the ranking histogram after the list buffer (list_build_lds_bytes)
-    int *hist = reinterpret_cast<int *>(buf + (size_t)a.nbr_cap * (blockDim.x + 4));
+    // staging with its read headroom, the masks, the ranking histogram
+    // (list_build_lds_bytes)
+    const int slots = a.lds_cap + list_build_pad(a.cell_cap);
+    BuildLds B;
+    B.xy = reinterpret_cast<float2 *>(dyn);
+    B.grp = reinterpret_cast<int *>(B.xy + slots);
+    B.sig = reinterpret_cast<float *>(B.grp + slots);
+    uint32_t *mask = reinterpret_cast<uint32_t *>(B.grp + (kSigma ? 2 : 1) * slots);
+    int *hist = reinterpret_cast<int *>(mask + 3 * list_build_words(a.cell_cap) * blockDim.x);
     if (a.ctl && a.any && !*a.any) return;  // gated, and no replica rebuilds
     // gated batches walk the listed tiles of the rebuilding replicas
     const int nt = a.ftile ? *a.nft : a.ntiles;
@@ -1687,18 +1812,26 @@ __global__ __launch_bounds__(256) void k_list_build(ForceArgs a) {
         if (a.ctl && !a.ftile && !a.ctl[T.rep].flag) continue;  // uniform per workgroup
         const RepDesc R = a.reps[T.rep];
         const int W = T.w_flags & 0xffff;
-        if (stage_tile<false, false>(a, T, R, W, L, nullptr, nullptr) < 0) {
+        if (stage_layout(a, T, R, W, L) < 0) {
             if (threadIdx.x == 0) atomicOr(a.err, 2u);  // FM_DEV_TILE_OVERFLOW
             __syncthreads();
             continue;
         }
+        stage_copy(
+            T, R, W, L, [&](int p) { return a.sorted[p]; },
+            [&](int e, const float4 &u) {
+                B.xy[e] = make_float2(u.x, u.y);
+                B.grp[e] = __float_as_int(u.z);
+                if (kSigma) B.sig[e] = u.w;
+            });
+        __syncthreads();
         const bool wrapT = (T.w_flags >> 16) & 1;
         if (a.lbuf) {
-            if (wrapT) list_tile_body_buf<true, kSigma>(a, T, R, W, L, buf, hist);
-            else list_tile_body_buf<false, kSigma>(a, T, R, W, L, buf, hist);
+            if (wrapT) list_tile_body_mask<true, kSigma>(a, T, R, W, L, B, mask, hist);
+            else list_tile_body_mask<false, kSigma>(a, T, R, W, L, B, mask, hist);
         } else {
-            if (wrapT) list_tile_body_direct<true, kSigma>(a, T, R, W, L);
-            else list_tile_body_direct<false, kSigma>(a, T, R, W, L);
+            if (wrapT) list_tile_body_direct<true, kSigma>(a, T, R, W, L, B);
+            else list_tile_body_direct<false, kSigma>(a, T, R, W, L, B);
         }
         __syncthreads();  // the next tile restages the LDS
     }
@@ -2785,11 +2918,7 @@ __device__ void block_sums_all(double (&v)[K], double *red) {
     __syncthreads();
 }
 
-__device__ __forceinline__ float wave_min(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fminf(v, __shfl_xor(v, o));
-    return v;
-}
+__device__ __forceinline__ float wave_min(float v) { return -wave_max(-v); }
 
 // Per cluster: the unfolded node positions (femmd2D/src/feaElements.cpp:
 // 86-133: a cluster wider than half the box has its nodes beyond L/2 moved
@@ -3180,10 +3309,12 @@ hipError_t launch_forces(bool sigma, bool types, bool debug, bool list, bool ene
     return hipGetLastError();
 }
 
-size_t list_build_lds_bytes(int lds_cap, int cell_cap, int nbr_cap, int block, bool buffered) {
-    // staging; list buffer and the ranking histogram (list_rank)
-    return (size_t)(lds_cap + 3 * cell_cap) * sizeof(float4) +
-           (buffered ? (size_t)nbr_cap * (block + 4) +
+size_t list_build_lds_bytes(int lds_cap, int cell_cap, int nbr_cap, int block, bool sigma,
+                            bool buffered) {
+    // staging with its read headroom; masks and the ranking histogram (list_rank)
+    return (size_t)(lds_cap + list_build_pad(cell_cap)) *
+               (sizeof(float2) + sizeof(int) + (sigma ? sizeof(float) : 0)) +
+           (buffered ? (size_t)3 * list_build_words(cell_cap) * block * sizeof(uint32_t) +
                            (size_t)2 * (nbr_cap / 4 + 1) * (block / 64) * sizeof(int)
                      : 0);
 }
@@ -3192,7 +3323,7 @@ size_t list_build_lds_bytes(int lds_cap, int cell_cap, int nbr_cap, int block, b
 // build is launched with this grid: skipped steps cost one resident wave of
 // workgroups, and a rebuild loses nothing since the rest would only queue).
 int list_build_resident(bool sigma, int block, const ForceArgs &a, int device) {
-    const size_t lds = list_build_lds_bytes(a.lds_cap, a.cell_cap, a.nbr_cap, block, a.lbuf != 0);
+    const size_t lds = list_build_lds_bytes(a.lds_cap, a.cell_cap, a.nbr_cap, block, sigma, a.lbuf != 0);
     int per_cu = 0, ncu = 0;
     hipError_t e = sigma
         ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_list_build<true>, block, lds)
@@ -3206,7 +3337,7 @@ int list_build_resident(bool sigma, int block, const ForceArgs &a, int device) {
 
 hipError_t launch_list_build(bool sigma, int block, const ForceArgs &a, hipStream_t s) {
     if (a.ntiles <= 0) return hipSuccess;
-    const size_t lds = list_build_lds_bytes(a.lds_cap, a.cell_cap, a.nbr_cap, block, a.lbuf != 0);
+    const size_t lds = list_build_lds_bytes(a.lds_cap, a.cell_cap, a.nbr_cap, block, sigma, a.lbuf != 0);
     const int gated = a.gated_grid > 0 ? a.gated_grid : kGatedGrid;
     const dim3 g(a.ctl ? std::min(a.ntiles, gated) : a.ntiles);
     if (sigma)
