@@ -60,7 +60,8 @@ struct alignas(16) RepDesc {
     float rc_list;     // list mode: the largest cutoff of the pair table (in
                        // sigma units); lists hold every pair within
                        // rc_list * sigma_ij + skin
-    int32_t pad_[3];
+    float m_uniform;   // 1 / im_uniform (0 when masses differ)
+    int32_t pad_[2];
 };
 
 // Per-step observables (femmd2D/src/properties.cpp:15-86, evaluated and
@@ -122,6 +123,20 @@ struct alignas(16) Tile {  // force pass, LJ role
     int32_t rep, cy, cx0;
     int32_t w_flags;  // W in bits 0..15, bit 16 = needs minimum image,
                       // bit 17 in x, bit 18 in y
+};
+// List mode: a tile's staging as its list build laid it out, for the force
+// passes that use the lists (the sorted order and the tiles stay fixed until
+// the next build).  The three staged rows are consecutive in LDS, row r the
+// slots [end[r - 1], end[r]); slot e holds sorted position e + d0[r], from
+// o1[r] on e + d1[r] and from o2[r] on e + d2[r] (where the row's columns wrap
+// around the box).
+struct alignas(32) TileRun {
+    int32_t sbase;  // sorted position (and list slot) of the first centre
+    int32_t c_lo;   // its LDS slot
+    int32_t nc;     // centres
+    int32_t m;      // staged particles, -1: more than the LDS holds
+    int32_t end[3], o1[3], o2[3], d0[3], d1[3], d2[3];
+    int32_t pad[2];
 };
 struct alignas(16) Span {  // kick / element / bond workgroups
     int32_t rep, begin, end, pad;
@@ -273,6 +288,8 @@ struct ForceArgs {
                                // entries need the minimum image | (k << 16),
                                // k the tile index of the particle whose list
                                // it is
+    int32_t *lid;              // per list slot: the internal id of its particle
+    TileRun *runs;             // per tile: the staging of the list build
     int32_t lbuf;              // list build: hit masks in LDS, lists ranked by
                                // length, when set (else stored as found)
     int32_t gated_grid;        // list build grid when gated (resident workgroups)
@@ -393,6 +410,8 @@ struct ReorderArgs {
     int32_t *spos;             // internal id -> sorted slot (list mode; rewritten)
     int32_t *bsum;             // per chunk: movable count, then its exclusive prefix
     int32_t *oldof;            // new internal id -> old internal id
+    int32_t *lid;              // list slot -> internal id (list mode; rewritten)
+    int32_t *newof;            // old internal id -> new internal id (list mode)
     int narr;                  // per-particle 4-byte arrays to permute
     uint32_t *arr[kReorderArrays];
     uint32_t *tmp;             // narr * n words

@@ -17,6 +17,10 @@ namespace fm {
 
 namespace {
 
+// Particles of a tile (its centres, on average) as a share of the workgroup:
+// above it some tiles exceed the workgroup and take a second, nearly empty
+// pass
+constexpr double kTileFill = 0.85;
 constexpr int kGraphSteps = 16;  // step bodies per captured graph of a run
 // node kicks of at least this many workgroups gather through LDS (measured:
 // 1950 workgroups, 500k nodes: faster; 364 workgroups: slower)
@@ -276,6 +280,7 @@ int Engine::build(const std::vector<const HostSystem *> &reps, std::unique_ptr<E
             bool uni = f > 0.0f;
             for (int k = 1; uni && k < n; ++k) uni = him[p0 + k] == f;
             D.im_uniform = uni ? f : 0.0f;
+            D.m_uniform = uni ? 1.0f / f : 0.0f;
         }
         D.ks0 = (int32_t)ks.size();
         for (int b = p0; b < p0 + n; b += kKickThreads)
@@ -339,8 +344,9 @@ int Engine::build(const std::vector<const HostSystem *> &reps, std::unique_ptr<E
     }
     E->N_ = p0;
     E->ncells_ = cell0;
-    // the list pass indexes list groups with 32-bit element indices: larger
-    // systems walk the cells every step (cells of side >= rc*sigma + skin)
+    // list groups are indexed with 32 bits (and, the capacity being at least
+    // 32, a list's slot has a 32-bit byte offset): larger systems walk the
+    // cells every step (cells of side >= rc*sigma + skin)
     if (E->list_ && (double)E->nbr_cap_ / 4 * p0 >= 4294967295.0) E->list_ = false;
 
     E->ntri_ = (int)ht0.size();
@@ -513,6 +519,7 @@ int Engine::build(const std::vector<const HostSystem *> &reps, std::unique_ptr<E
     if (E->list_) {
         FM_AL(nbr_, (size_t)E->nbr_cap_ * N / 2);  // uint16 entries
         FM_AL(nnum_, N);
+        FM_AL(lid_, N);
         FM_AL(ctl_, R);
         FM_AL(any_, 1);
         // two sets of displacement slots and two sorted-order position
@@ -536,6 +543,7 @@ int Engine::build(const std::vector<const HostSystem *> &reps, std::unique_ptr<E
         return E->check(he, "memset", err);
     if (E->list_) {
         if ((he = hipMemsetAsync(E->nnum_.p, 0, sizeof(int32_t) * N, st)) != hipSuccess ||
+            (he = hipMemsetAsync(E->lid_.p, 0, sizeof(int32_t) * N, st)) != hipSuccess ||
             (he = hipMemsetAsync(E->ctl_.p, 0, sizeof(Ctl) * R, st)) != hipSuccess ||
             (he = hipMemsetAsync(E->any_.p, 0, sizeof(int32_t), st)) != hipSuccess ||
             (he = hipMemsetAsync(E->spos_.p, 0, sizeof(int32_t) * N, st)) != hipSuccess ||
@@ -573,7 +581,7 @@ int Engine::build(const std::vector<const HostSystem *> &reps, std::unique_ptr<E
 
 // Tiles of one cell row each: (replica, row, first column, width).  Width 0
 // picks one from the mean cell occupancy so a tile's centre cells hold about
-// 0.9 x block particles.
+// kTileFill x block particles.
 int Engine::build_tiles(const std::vector<int> &tile_w, std::string &err) {
     drop_graph();
     tiles_h_.clear();
@@ -585,9 +593,13 @@ int Engine::build_tiles(const std::vector<int> &tile_w, std::string &err) {
         const RepDesc &D = reps_h_[r];
         const double ppc = (double)(D.p1 - D.p0) / (D.ncx * D.ncy);
         int W = (r < (int)tile_w.size()) ? tile_w[r] : 0;
-        if (W <= 0) W = (int)std::lround(0.9 * block_ / std::max(ppc, 0.5));
+        if (W <= 0) W = (int)std::lround(kTileFill * block_ / std::max(ppc, 0.5));
         W = std::max(1, std::min(W, std::min(kMaxTileW, (int)D.ncx)));
         tile_w_[r] = W;
+        // the row's columns shared evenly by its tiles (widths differ by at
+        // most one): a narrow last tile per row costs as much latency as a
+        // full one
+        const int ntx = (D.ncx + W - 1) / W;
         const int t_begin = (int)tiles_h_.size();
         // rows 0 and ncy - 1 first (their halo rows cross the periodic
         // boundary, so all their lists take the minimum image): the force
@@ -595,8 +607,9 @@ int Engine::build_tiles(const std::vector<int> &tile_w, std::string &err) {
         // costlier tiles then start early instead of closing the last band
         for (int iy = 0; iy < (lj_on_[r] ? D.ncy : 0); ++iy) {
             const int cy = iy == 0 ? 0 : (iy == 1 ? D.ncy - 1 : iy - 1);
-            for (int cx0 = 0; cx0 < D.ncx; cx0 += W) {
-                const int w = std::min(W, D.ncx - cx0);
+            for (int t = 0; t < ntx; ++t) {
+                const int cx0 = (int)((long long)D.ncx * t / ntx);
+                const int w = (int)((long long)D.ncx * (t + 1) / ntx) - cx0;
                 // interior tiles (no staged cell wraps, >= 5 cells per axis)
                 // never need the minimum image: |dx| < 2 cells <= 0.4 L
                 const bool big = D.ncx >= 5 && D.ncy >= 5;
@@ -641,6 +654,8 @@ int Engine::build_tiles(const std::vector<int> &tile_w, std::string &err) {
     if (list_ && R_ > kDecideMinReps &&
         (he = ftile_.alloc(std::max<size_t>(tiles_h_.size(), 1))) != hipSuccess)
         return check(he, "tile list", err);
+    if (list_ && (he = runs_.alloc(std::max<size_t>(tiles_h_.size(), 1))) != hipSuccess)
+        return check(he, "tile runs", err);
     if ((he = lj_part_.alloc(2 * std::max<size_t>(tiles_h_.size(), 1))) != hipSuccess ||
         (he = ke_tile_.alloc(2 * std::max<size_t>(tiles_h_.size(), 1))) != hipSuccess)
         return check(he, "tile partials", err);
@@ -964,6 +979,8 @@ ForceArgs Engine::force_args() {
     f.nbr_cap = nbr_cap_;
     f.nbr = nbr_.p;
     f.nnum = nnum_.p;
+    f.lid = lid_.p;
+    f.runs = runs_.p;
     // hit masks and ranking in LDS when they fit in 64 KB beside the staging
     // (static LDS of the kernel: ~2 KB)
     f.lbuf = list_build_lds_bytes(lds_cap_, cap_, nbr_cap_, block_, sigma_, true) <= 62 * 1024;
@@ -1126,6 +1143,15 @@ int Engine::launch_reorder_now() {
     a.bsum = ro_bsum_.p;
     a.oldof = ro_oldof_.p;
     a.tmp = ro_tmp_.p;
+    if (list_) {
+        if (ro_newof_.n < (size_t)N_) {
+            if ((he = ro_newof_.alloc(N_)) != hipSuccess) return -1;
+            if ((he = hipMemsetAsync(ro_newof_.p, 0, (size_t)N_ * sizeof(int32_t), stream_)) != hipSuccess)
+                return -1;
+        }
+        a.lid = lid_.p;
+        a.newof = ro_newof_.p;
+    }
     if (launch_reorder(a, stream_) != hipSuccess) return -1;
     order_stale_ = true;
     ++nreorder_;

@@ -297,7 +297,7 @@ private:
     DBuf<float> x_, y_, vx_, vy_, fx_, fy_, mass_, inv_m_, sig_;
     DBuf<int32_t> grp_, typ_, uid_;
     DBuf<uint8_t> mov_;                // per internal id: movable
-    DBuf<int32_t> movids_, ro_bsum_, ro_oldof_;
+    DBuf<int32_t> movids_, ro_bsum_, ro_oldof_, ro_newof_;
     DBuf<int32_t> fspan_, ftile_, fblock_, nf_;  // batches: compact rebuild work lists
     DBuf<int4> rinfo_;
     DBuf<uint8_t> mark_;
@@ -310,7 +310,8 @@ private:
     int lb_grid_ = 0;  // gated list-build grid (resident workgroups)
     DBuf<float4> sorted_;
     DBuf<Span> kspans_, espans_, bspans_;
-    DBuf<int32_t> nbr_, nnum_, any_;
+    DBuf<int32_t> nbr_, nnum_, lid_, any_;
+    DBuf<TileRun> runs_;
     DBuf<Ctl> ctl_;
     DBuf<float> sigs_;
     DBuf<uint32_t> dmax_;

@@ -262,30 +262,38 @@ __device__ void obs_level1(const ObsArgs &o, double *red) {
     for (int q = blockIdx.x; q < njob; q += gridDim.x) obs_chunk(o, q / o.nchunk, q % o.nchunk, red);
 }
 
-// Level 2 for replica r (one thread): the step's totals from its chunks in
-// chunk order, the averaged quantities of femmd2D/src/properties.cpp:15-36
-// and, when accumulate is set, Prop::accum of each (properties.h:10).
+// Level 2 for replica r, one wavefront (all lanes): the step's totals from
+// its chunks, the averaged quantities of femmd2D/src/properties.cpp:15-36
+// and, when accumulate is set, Prop::accum of each (properties.h:10).  Lane
+// 8 g + k takes value k of chunks g and g + 8, so the 128 loads are in flight
+// together (one thread reading them in turn took 5 us).
 __device__ void obs_finish(const ObsArgs &o, int r, bool accumulate) {
-    const double *ch = o.chunk + (size_t)r * kObsChunks * kObsRaw;
-    double t[kObsRaw] = {0, 0, 0, 0, 0, 0, 0, 0};
-    for (int c = 0; c < o.nchunk; ++c) {
-        const double *q = ch + c * kObsRaw;
-        for (int k = 0; k < kObsRaw; ++k) t[k] = (k == 1) ? fmax(t[1], q[1]) : t[k] + q[k];
+    static_assert(kObsRaw == 8 && kObsAvg == 8 && kObsChunks == 16, "lane layout of the totals");
+    const int lane = threadIdx.x & 63, k = lane & 7, g = lane >> 3;
+    const double *q = o.chunk + ((size_t)r * kObsChunks + g) * kObsRaw + k;
+    const double x = g < o.nchunk ? q[0] : 0.0;
+    const double y = g + 8 < o.nchunk ? q[8 * kObsRaw] : 0.0;
+    double t = k == 1 ? fmax(x, y) : x + y;
+#pragma unroll
+    for (int m = 8; m < 64; m <<= 1) {
+        const double z = __shfl_xor(t, m);
+        t = k == 1 ? fmax(t, z) : t + z;
     }
     double *ob = o.obs + (size_t)r * kObsStride;
-    for (int k = 0; k < kObsRaw; ++k) ob[k] = t[k];
+    if (lane < kObsRaw) ob[lane] = t;  // {KE2, max v^2, U, W of pairs, elements, bonds}
     if (!accumulate) return;
     const RepDesc &R = o.reps[r];
     const double n = (double)(R.p1 - R.p0), V = (double)R.Lx * (double)R.Ly;
-    const double uk = 0.5 * t[0] / n;
-    const double up = (t[2] + t[4] + t[6]) / n;
-    const double a[kObsAvg] = {uk, up, uk + up, 0.5 * t[0] / V + 0.5 * (t[3] + t[5]) / V,
-                               t[3], t[5], t[6] / n, t[4] / n};
-    ob[kObsRaw] += 1.0;
-    for (int k = 0; k < kObsAvg; ++k) {
-        ob[kObsRaw + 1 + k] += a[k];
-        ob[kObsRaw + 1 + kObsAvg + k] += a[k] * a[k];
-    }
+    const double ke2 = __shfl(t, 0), ulj = __shfl(t, 2), wlj = __shfl(t, 3), ufea = __shfl(t, 4),
+                 wfea = __shfl(t, 5), ub = __shfl(t, 6);
+    const double uk = 0.5 * ke2 / n, up = (ulj + ufea + ub) / n;
+    if (lane >= kObsAvg) return;
+    const double a = lane == 0 ? uk : lane == 1 ? up : lane == 2 ? uk + up
+                   : lane == 3 ? 0.5 * ke2 / V + 0.5 * (wlj + wfea) / V
+                   : lane == 4 ? wlj : lane == 5 ? wfea : lane == 6 ? ub / n : ufea / n;
+    if (lane == 0) ob[kObsRaw] += 1.0;
+    ob[kObsRaw + 1 + lane] += a;
+    ob[kObsRaw + 1 + kObsAvg + lane] += a * a;
 }
 
 // Bin one particle per lane into its cell's slot list (the reference's
@@ -337,7 +345,9 @@ __device__ __forceinline__ void kick_particle(const RepDesc &R, float ax, float 
         vy = vy + R.hdt * ay;
         if (kEnergy) {
             vv = vx * vx + vy * vy;
-            const float m = im > 0.0f ? 1.0f / im : 0.0f;
+            float m;  // (uniform branch: no division when the masses are equal)
+            if (R.im_uniform > 0.0f) m = R.m_uniform;
+            else m = im > 0.0f ? 1.0f / im : 0.0f;
             ke = (double)(m * vv);
         }
     }
@@ -1003,8 +1013,7 @@ struct PairLds {
     int *cstart;   // per slot: first sorted position
     int *off;      // per slot: first LDS entry (S + 1)
     PairEntry *pt; // pair table of the replica
-    double *red;   // 3 per wavefront
-    float *redf;   // 2 per wavefront
+    double *red;   // reductions (2 per wavefront)
 };
 
 // The kick a tile gives its centre particles (the kick modes of k_forces):
@@ -1016,7 +1025,8 @@ struct TileKick {
 };
 
 // Kick of the tile's centre particle id (sorted position p) at its staged
-// position (x, y) (the same bits as x[id]) with pair force (fxs, fys).
+// position (x, y) (the same bits as x[id]) and velocity (vx, vy) with pair
+// force (fxs, fys).
 // kKick 1: second half-kick only (the closing kick of a run); 2: second and
 // first half-kick, drift and wrap.  A particle with element or bond corners
 // is left to the node kick, which adds its gathered corner forces: its pair
@@ -1025,7 +1035,8 @@ struct TileKick {
 // walk, mode 2), -1 when there is none to bin.
 template <int kKick, bool kList, bool kEnergy>
 __device__ __forceinline__ int tile_kick(const ForceArgs &a, const RepDesc &R, int id, int p,
-                                         float x, float y, float fxs, float fys, TileKick &tk) {
+                                         float x, float y, float vx, float vy, float fxs,
+                                         float fys, TileKick &tk) {
     const bool node = id >= R.pg;  // (internal order: these come last)
     if (kKick != 2 || node) {
         a.fx[id] = fxs;
@@ -1034,7 +1045,7 @@ __device__ __forceinline__ int tile_kick(const ForceArgs &a, const RepDesc &R, i
     if (kKick == 0 || node) return -1;
     const float im = R.im_uniform > 0.0f ? R.im_uniform : a.inv_m[id];
     const float ax = fxs * im, ay = fys * im;
-    float vx = a.vx[id], vy = a.vy[id], dxp = 0.0f, dyp = 0.0f, vv = 0.0f;
+    float dxp = 0.0f, dyp = 0.0f, vv = 0.0f;
     double ke = 0.0;
     kick_particle<true, kKick == 2, kEnergy>(R, ax, ay, im, vx, vy, x, y, ke, vv, dxp, dyp, a.err);
     a.vx[id] = vx;
@@ -1058,60 +1069,59 @@ __device__ __forceinline__ int tile_kick(const ForceArgs &a, const RepDesc &R, i
     return R.cell0 + cell_key(x, y, R);
 }
 
-// End of a tile: fixed-order sums of U, W and the kinetic energy, maxima of
-// v^2 and of the squared displacement (valid in thread 0).
-__device__ void tile_reduce(double &u, double &w, TileKick &tk, const PairLds &L) {
-    u = wave_sum(u);
-    w = wave_sum(w);
-    double ke = wave_sum(tk.ke);
-    float vv = wave_max(tk.vv), d2 = wave_max(tk.d2);
-    const int wv = threadIdx.x >> 6, nw = blockDim.x >> 6;
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) {
-        L.red[3 * wv] = u;
-        L.red[3 * wv + 1] = w;
-        L.red[3 * wv + 2] = ke;
-        L.redf[2 * wv] = vv;
-        L.redf[2 * wv + 1] = d2;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double su = 0.0, sw = 0.0, sk = 0.0;
-        float mv = 0.0f, md = 0.0f;
-        for (int k = 0; k < nw; ++k) {
-            su += L.red[3 * k];
-            sw += L.red[3 * k + 1];
-            sk += L.red[3 * k + 2];
-            mv = fmaxf(mv, L.redf[2 * k]);
-            md = fmaxf(md, L.redf[2 * k + 1]);
-        }
-        u = su;
-        w = sw;
-        tk.ke = sk;
-        tk.vv = mv;
-        tk.d2 = md;
-    }
-}
+// End of a tile: the workgroup's sums of u, w (scaled by cu, cw) and of the
+// kicked particles' kinetic energy, and the maxima of v^2 and of the squared
+// displacement, written as the tile's partials (the displacement into one of
+// the replica's slots for the next rebuild decision).  The lanes' values go
+// through LDS (the staging, free by now: tile_scratch_bytes), each quantity
+// is then reduced by one wavefront: 40 vector instructions a wavefront, where
+// every wavefront reducing all five took 150.  Fixed order.
+__host__ __device__ constexpr size_t tile_scratch_bytes(int block) { return (size_t)block * 32; }
 
-// Writes a tile's partials: U, W (kEnergy), the kicked particles' kinetic
-// energy and max v^2 (kEnergy with a kick) and its largest displacement
-// into one of the replica's slots for the next rebuild decision (list mode,
-// step kick).  Thread 0.
 template <int kKick, bool kList, bool kEnergy>
-__device__ __forceinline__ void tile_partials(const ForceArgs &a, int tile, int rep, double u,
-                                              double w, const TileKick &tk) {
-    if (threadIdx.x != 0) return;
+__device__ void tile_finish(const ForceArgs &a, int tile, int rep, double u, double w, double cu,
+                            double cw, const TileKick &tk, void *scratch) {
+    constexpr bool kKe = kEnergy && kKick != 0, kDisp = kList && kKick == 2;
+    if (!kEnergy && !kDisp) return;
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int bd = blockDim.x, nw = bd >> 6;
+    double *sd = reinterpret_cast<double *>(scratch);
+    float *sf = reinterpret_cast<float *>(sd + 3 * bd);
+    __syncthreads();  // the staging's readers are done
     if (kEnergy) {
-        a.lj_part[2 * tile] = u;
-        a.lj_part[2 * tile + 1] = w;
+        sd[tid] = u;
+        sd[bd + tid] = w;
     }
-    if (kEnergy && kKick != 0) {
-        a.ke_tile[2 * tile] = tk.ke;
-        a.ke_tile[2 * tile + 1] = (double)tk.vv;
+    if (kKe) {
+        sd[2 * bd + tid] = tk.ke;
+        sf[tid] = tk.vv;
     }
-    if (kList && kKick == 2)
-        atomicMax(a.dmax_out + ((size_t)rep * kDispSlots + tile % kDispSlots) * kDispStride,
-                  __float_as_uint(tk.d2));
+    if (kDisp) sf[bd + tid] = tk.d2;
+    __syncthreads();
+    for (int q = wv; q < 5; q += nw) {  // (uniform per wavefront)
+        if (q < 3) {
+            if (q < 2 ? !kEnergy : !kKe) continue;
+            double t = 0.0;
+            for (int k = 0; k < nw; ++k) t += sd[q * bd + 64 * k + lane];
+            t = wave_sum(t);
+            if (lane == 0) {
+                if (q == 0) a.lj_part[2 * tile] = cu * t;
+                else if (q == 1) a.lj_part[2 * tile + 1] = cw * t;
+                else a.ke_tile[2 * tile] = t;
+            }
+        } else {
+            if (q == 3 ? !kKe : !kDisp) continue;
+            float t = 0.0f;
+            for (int k = 0; k < nw; ++k) t = fmaxf(t, sf[(q - 3) * bd + 64 * k + lane]);
+            t = wave_max(t);
+            if (lane == 0) {
+                if (q == 3) a.ke_tile[2 * tile + 1] = (double)t;
+                else
+                    atomicMax(a.dmax_out + ((size_t)rep * kDispSlots + tile % kDispSlots) * kDispStride,
+                              __float_as_uint(t));
+            }
+        }
+    }
 }
 
 // LJ over one tile (femmd2D/src/interactionsCuda.cu:43-100 pair maths,
@@ -1262,10 +1272,11 @@ __device__ void pair_tile_body(const ForceArgs &a, const RepDesc &R, int rep, in
             Wi = (double)accB;
         }
         id = a.perm[sbase + k];
-        cell = tile_kick<kKick, false, kEnergy>(a, R, id, sbase + k, xi, yi, fx, fy, tk);
+        cell = tile_kick<kKick, false, kEnergy>(a, R, id, sbase + k, xi, yi, kKick ? a.vx[id] : 0.0f,
+                                                kKick ? a.vy[id] : 0.0f, fx, fy, tk);
         if (kEnergy) {
-            Ublk += 0.5 * Ui;
-            Wblk += 0.5 * Wi;
+            Ublk += Ui;
+            Wblk += Wi;
         }
         if (kDebug) {
             const int u = a.uid[id];
@@ -1276,10 +1287,7 @@ __device__ void pair_tile_body(const ForceArgs &a, const RepDesc &R, int rep, in
         }
         if (kKick == 2) bin_wave_to(a.count, a.tmp, a.cell_cap, a.err, cell >= 0, id, cell);
     }
-    if (kEnergy || kKick == 2) {
-        tile_reduce(Ublk, Wblk, tk, L);
-        tile_partials<kKick, false, kEnergy>(a, tile, rep, Ublk, Wblk, tk);
-    }
+    tile_finish<kKick, false, kEnergy>(a, tile, rep, Ublk, Wblk, 0.5, 0.5, tk, L.ent);
 }
 
 // Stages the 3 x (W+2) cells of a tile into LDS: rows cy-1, cy, cy+1 and
@@ -1336,6 +1344,12 @@ __device__ int stage_layout(const ForceArgs &a, const Tile &T, const RepDesc &R,
     return M > a.lds_cap ? -1 : M;
 }
 
+// Slots (within a staged row) where its columns wrap to 0; W + 2: none.
+__device__ __forceinline__ void row_wraps(const Tile &T, const RepDesc &R, int W, int &b1, int &b2) {
+    b1 = min(T.cx0 == 0 ? 1 : R.ncx - T.cx0 + 1, W + 2);
+    b2 = min(b1 + R.ncx, W + 2);
+}
+
 // Copies every staged entry e (LDS index) from its sorted position p:
 // st(e, ld(p)).  The cells of one staged row are consecutive in sorted order
 // except where the column index wraps to 0 (at most twice), so each row is
@@ -1351,11 +1365,8 @@ __device__ void stage_copy(const Tile &T, const RepDesc &R, int W, const PairLds
                            St &&st) {
     using V = decltype(ld(0));
     const int row = W + 2;
-    // slots (within a row) where the column wraps to 0
-    int b1 = (T.cx0 == 0) ? 1 : (R.ncx - T.cx0 + 1);
-    int b2 = b1 + R.ncx;
-    if (b1 >= row) b1 = row;
-    if (b2 >= row) b2 = row;
+    int b1, b2;
+    row_wraps(T, R, W, b1, b2);
     const int r1 = L.off[row], r2 = L.off[2 * row], M = L.off[3 * row];
     const int bd = blockDim.x;
     for (int e0 = (int)threadIdx.x; e0 < M; e0 += kStageBatch * bd) {
@@ -1420,7 +1431,7 @@ __device__ void pair_tile(const ForceArgs &a, int tile, PairLds &L) {
     const bool wrapT = (T.w_flags >> 16) & 1;
     if (stage_tile<kTypes, kDebug>(a, T, R, W, L, nullptr, nullptr) < 0) {
         atomicOr(a.err, 2u);  // FM_DEV_TILE_OVERFLOW (its particles are not moved)
-        tile_partials<kKick, false, kEnergy>(a, tile, T.rep, 0.0, 0.0, TileKick{});
+        tile_finish<kKick, false, kEnergy>(a, tile, T.rep, 0.0, 0.0, 0.0, 0.0, TileKick{}, L.ent);
         return;
     }
     if (wrapT)
@@ -1548,6 +1559,7 @@ __device__ void list_tile_body_direct(const ForceArgs &a, const Tile &T, const R
         for (int kk = m; kk < ((m + 3) & ~3); ++kk) list_store_slot(a, kk, p, 8 * a.lds_cap);
         // list slot p holds particle k of the tile
         a.nnum[p] = m | (kWrap && ic.needs(col, W) ? kListImg : 0) | (k << 16);
+        a.lid[p] = a.perm[p];
         if (cnt > cap) atomicOr(a.err, 16u);  // FM_DEV_LIST_OVERFLOW
     }
 }
@@ -1653,6 +1665,7 @@ __device__ void list_tile_body_mask(const ForceArgs &a, const Tile &T, const Rep
             if (L.off[mid] <= me) lo = mid; else hi = mid;
         }
         const int col = lo - row;
+        const int id = a.perm[sbase + min(k, nc - 1)];
         const float2 pi = B.xy[me];
         const int gi = B.grp[me];
         const int gix = gi >= 0 ? gi : -2;  // (-1 never matches -2)
@@ -1777,9 +1790,31 @@ __device__ void list_tile_body_mask(const ForceArgs &a, const Tile &T, const Rep
         }
         if (act) {
             a.nnum[sbase + k0 + rank] = m | (img ? kListImg : 0) | (k << 16);
+            a.lid[sbase + k0 + rank] = id;
             if (cnt > cap) atomicOr(a.err, 16u);  // FM_DEV_LIST_OVERFLOW
         }
     }
+}
+
+// The record of a tile's staging, row r of it (and the tile's own words with
+// row 0).
+__device__ void store_run(TileRun *o, const Tile &T, const RepDesc &R, int W, const PairLds &L, int M,
+                          int r) {
+    const int row = W + 2, s0 = r * row;
+    if (r == 0) {
+        o->m = M;
+        o->sbase = L.cstart[row + 1];
+        o->c_lo = L.off[row + 1];
+        o->nc = M < 0 ? 0 : L.off[row + W + 1] - L.off[row + 1];
+    }
+    int b1, b2;
+    row_wraps(T, R, W, b1, b2);
+    o->end[r] = L.off[s0 + row];
+    o->o1[r] = L.off[s0 + b1];
+    o->o2[r] = L.off[s0 + b2];
+    o->d0[r] = L.cstart[s0] - L.off[s0];
+    o->d1[r] = b1 < row ? L.cstart[s0 + b1] - L.off[s0 + b1] : 0;
+    o->d2[r] = b2 < row ? L.cstart[s0 + b2] - L.off[s0 + b2] : 0;
 }
 
 template <bool kSigma>
@@ -1808,11 +1843,14 @@ __global__ __launch_bounds__(256) void k_list_build(ForceArgs a) {
     // gated batches walk the listed tiles of the rebuilding replicas
     const int nt = a.ftile ? *a.nft : a.ntiles;
     for (int b = blockIdx.x; b < nt; b += gridDim.x) {
-        const Tile T = a.tiles[a.ftile ? a.ftile[xcd_remap(b, nt)] : xcd_remap(b, nt)];
+        const int tile = a.ftile ? a.ftile[xcd_remap(b, nt)] : xcd_remap(b, nt);
+        const Tile T = a.tiles[tile];
         if (a.ctl && !a.ftile && !a.ctl[T.rep].flag) continue;  // uniform per workgroup
         const RepDesc R = a.reps[T.rep];
         const int W = T.w_flags & 0xffff;
-        if (stage_layout(a, T, R, W, L) < 0) {
+        const int M = stage_layout(a, T, R, W, L);
+        if (threadIdx.x < 3) store_run(a.runs + tile, T, R, W, L, M, threadIdx.x);
+        if (M < 0) {
             if (threadIdx.x == 0) atomicOr(a.err, 2u);  // FM_DEV_TILE_OVERFLOW
             __syncthreads();
             continue;
@@ -1837,71 +1875,101 @@ __global__ __launch_bounds__(256) void k_list_build(ForceArgs a) {
     }
 }
 
-// LJ over the neighbour lists: one lane per particle of a kick span, the
-// pair maths and accumulation of pair_tile_body (FP32 cutoff predicate on
-// the current positions, so the interacting set is the same as the cell
-// walk's whenever the list is complete).
+typedef uint32_t v2u __attribute__((ext_vector_type(2)));
+
 // LJ over the neighbour lists, one workgroup per tile of the list build: the
 // tile's current positions (and sigmas) are staged in LDS in the build's
 // layout, each lane takes a centre particle and gathers its listed
 // neighbours from LDS (the pair maths and accumulation of pair_tile_body;
 // the FP32 cutoff predicate on the current positions, so the interacting
-// set is the cell walk's whenever the list is complete).
-// Energies and virials (kEnergy) from two FP32 sums per particle, three
-// vector instructions per list entry: T = sum_hit tv with tv = s12 - s6 / 2
-// (the force's own factor) and Q = sum over all evaluated entries of
-// (hit ? s6 : kq), kq = shift / (2 eps).  With A = sum s12, B = sum s6 and
-// n interacting pairs, T = A - B / 2 and Q = B + kq (L - n) for L evaluated
-// entries, so U_i = 4 eps (A - B) + n shift = 4 eps T - 2 eps (Q - kq L)
-// and W_i = 48 eps (A - B / 2) = 48 eps T (femmd2D/src/interactionsCuda.cu:
-// 91-96).  kCount (eps = 0, or the dump): n is counted instead.
-template <int kWrap, bool kSigma, bool kTypes, bool kEnergy, bool kUnit, bool kDebug, bool kCount,
-          int kKick>
-__device__ void list_tile_pass_body(const ForceArgs &a, const RepDesc &R, int rep, int W, int tile,
-                                    const PairLds &L, const float2 *lp, const float *ls,
-                                    const int *lid, const int *lt) {
-    const int row = W + 2;
-    const int c_lo = L.off[row + 1], c_hi = L.off[row + W + 1];
-    const int nc = c_hi - c_lo;
-    const int sbase = L.cstart[row + 1];
+// set is the cell walk's whenever the list is complete).  Bound by vector
+// issue and by its chain of loads: 18 instructions per list entry (37 where
+// the minimum image applies in both axes).  1.14 million particles (lists of
+// 21.7): 41.2 -> 37.1 us; 512 replicas, 3.84 million: 182 -> 168 us; 4,367
+// particles: 10.6 -> 8.4 us; 30,011 of six types: 16.7 -> 8.8 us.
+// A non-interacting entry has its 1 / r^2 replaced by 0, which makes every
+// term of it 0 (force, T, Q); the interacting entries are counted on the
+// scalar unit.  Energies and virials (kEnergy) from two FP32 sums per
+// particle, T = sum (s12 - s6 / 2) (the force's own factor) and Q = sum s6:
+// U = 4 eps (T - Q / 2) + n shift and W = 48 eps T
+// (femmd2D/src/interactionsCuda.cu:91-96), scaled per tile.
+// The loop over the list's groups runs to the longest list of the wavefront
+// (lists are ranked by length; a lane past its own list takes the padding
+// slot four times), so its control and the group addresses are scalar.
+// What a lane needs of its list slot, loaded before the staging is waited
+// for: length word, internal id, the first two groups of entries.
+struct ListSlot {
+    int nq, id;
+    v2u g0, g1;
+};
+// A list's group g (clamped inside the array; a group past the list is
+// loaded and not used): a scalar base and the lane's 32-bit offset.
+__device__ __forceinline__ v2u list_group(const ForceArgs &a, int g, uint32_t q8) {
+    typedef const __attribute__((address_space(1))) char *gptr;
+    uint64_t base = reinterpret_cast<uint64_t>(a.nbr) +
+                    (uint64_t)(uint32_t)min(g, (a.nbr_cap >> 2) - 1) * ((uint64_t)(uint32_t)a.n * 8u);
+    __asm__("" : "+s"(base));
+    return *(const __attribute__((address_space(1))) v2u *)((gptr)base + q8);
+}
+__device__ __forceinline__ ListSlot list_slot(const ForceArgs &a, int q) {
+    ListSlot s;
+    s.nq = a.nnum[q];
+    s.id = a.lid[q];
+    s.g0 = list_group(a, 0, 8u * (uint32_t)q);
+    s.g1 = list_group(a, 1, 8u * (uint32_t)q);
+    return s;
+}
+
+template <int kWrap, bool kSigma, bool kTypes, bool kEnergy, bool kUnit, bool kDebug, int kKick>
+__device__ void list_tile_pass_body(const ForceArgs &a, const RepDesc &R, const TileRun &V, int rep,
+                                    int tile, const PairEntry &pe, const PairEntry *pt,
+                                    ListSlot slot, float2 *lp, const float *ls, const int *lid,
+                                    const int *lt) {
+    const int c_lo = V.c_lo, nc = V.nc, sbase = V.sbase;
     const float Lx = R.Lx, Ly = R.Ly, hLx = R.hLx, hLy = R.hLy;
-    const PairEntry pe = L.pt[0];
     const float rc2_u = R.rc2_uniform;
-    // (not used when kCount: eps may be 0 there; nor with a type table,
-    // whose pairs accumulate their own eps-weighted terms)
-    const float kq = (kCount || kTypes) ? 0.0f : 2.0f * pe.shift / pe.e4;
     const int nt = R.ntypes;
-    const uint32_t Nu = (uint32_t)a.n;
-    const int capg = a.nbr_cap >> 2;
-    const uint64_t *nb = reinterpret_cast<const uint64_t *>(a.nbr);
+    // the padding slot twice: what a lane past its list evaluates
+    uint32_t pad2 = (uint32_t)(8 * a.lds_cap) * 0x10001u;
+    __asm__("" : "+v"(pad2));  // (held in a register: one select per half group)
     double Ublk = 0.0, Wblk = 0.0;
+    int nhit = 0;  // interacting entries of the wavefront (scalar)
     TileKick tk;
-    for (int l = threadIdx.x; l < nc; l += blockDim.x) {
+    // every lane of a wavefront takes part in each pass
+    const int w0 = __builtin_amdgcn_readfirstlane((int)(threadIdx.x & ~63u));
+    const int lane = (int)(threadIdx.x & 63u);
+    for (int l0 = w0; l0 < nc; l0 += (int)blockDim.x) {
         // list slot q holds the list of the tile's particle k (slots of a
-        // chunk of blockDim particles are ordered longest list first)
-        const int q = sbase + l;
-        const int nq = a.nnum[q];
+        // chunk of blockDim particles are ordered longest list first); a
+        // lane past the tile's slots takes the last one with no entries
+        const bool act = l0 + lane < nc;
+        const int q = sbase + min(l0 + lane, nc - 1);
+        if (l0 != w0) slot = list_slot(a, q);
+        const int nq = slot.nq, id = slot.id;
         const int k = nq >> 16;
         const int me = c_lo + k, p = sbase + k;
+        float vx = 0.0f, vy = 0.0f;  // (in flight while the list is walked)
+        if (kKick != 0) {
+            vx = a.vx[id];
+            vy = a.vy[id];
+        }
         const float2 pi = lp[me];
         const float xi = pi.x, yi = pi.y;
         const float xim = xi - Lx, yim = yi - Ly;
         const float si = kSigma ? ls[me] : 0.0f;
         const int ti = kTypes ? lt[me] : 0;
-        const int n4 = ((nq & kListLen) + 3) >> 2;  // padded with the sentinel slot
+        const int n4 = act ? ((nq & kListLen) + 3) >> 2 : 0;  // padded with the sentinel slot
+        const int n4w = wave_max_int(n4);
         // in a tile that needs the minimum image, only the wavefronts
         // holding a list flagged for it take the image path (the build
         // ranks those lists after the others); elsewhere the shift is 0
         const bool wimg = kWrap != 0 && __ballot((nq & kListImg) != 0) != 0ull;
-        // single type: T = sum_hit tv, Q as described above; with a type
-        // table: T = sum_hit e4 (s12 - s6), Q = sum_hit e48 tv, ush = sum_hit
-        // shift (femmd2D/src/interactions.cpp:347-389 per type pair)
+        // single type: T = sum_hit tv, Q = sum_hit s6; with a type table:
+        // T = sum_hit e4 (s12 - s6), Q = sum_hit e48 tv, ush = sum_hit shift
+        // (femmd2D/src/interactions.cpp:347-389 per type pair)
         float fx = 0.f, fy = 0.f, accT = 0.f, accQ = 0.f, ush = 0.f;
         int nint = 0;
         long long d1 = 0, d2 = 0;  // diagnostic dump: sums of (id + 1), (id + 1)^2
-        // one list entry, without branches: the force of a non-interacting
-        // entry (or of the padding entry) is computed and discarded by a
-        // select
         // wrapc: the axes that may need the minimum image (bit 0 x, bit 1
         // y); an axis left out has no shift in this tile, and its plain
         // difference has the bits the image path would give
@@ -1910,21 +1978,15 @@ __device__ void list_tile_pass_body(const ForceArgs &a, const RepDesc &R, int re
             constexpr bool kWX = (kW & 1) != 0, kWY = (kW & 2) != 0;
             const float xj = pj.x, yj = pj.y;
             const float ex = xi - xj, ey = yi - yj;
-            float ox = 0.0f, oy = 0.0f;
-            if (kWX) {  // minimum image as two selects per axis
-                ox = (ex >= hLx) ? Lx : 0.0f;
-                ox = (ex < -hLx) ? -Lx : ox;
-            }
-            if (kWY) {
-                oy = (ey >= hLy) ? Ly : 0.0f;
-                oy = (ey < -hLy) ? -Ly : oy;
-            }
-            const float dx = ex - ox;
-            const float dy = ey - oy;
+            // minimum image: whether the difference is shifted by -L or +L
+            const bool px = kWX && ex >= hLx, mx = kWX && ex < -hLx;
+            const bool py = kWY && ey >= hLy, my = kWY && ey < -hLy;
+            const float dx = kWX ? ex - (mx ? -Lx : (px ? Lx : 0.0f)) : ex;
+            const float dy = kWY ? ey - (my ? -Ly : (py ? Ly : 0.0f)) : ey;
             const float dr2 = dx * dx + dy * dy;
             float s2ij, rc2, e48 = 0.0f, e4 = 0.0f, shift = 0.0f;
             if (kTypes) {
-                const PairEntry q = L.pt[ti * nt + tj];
+                const PairEntry q = pt[ti * nt + tj];
                 e48 = q.e48;
                 e4 = q.e4;
                 shift = q.shift;
@@ -1946,30 +2008,28 @@ __device__ void list_tile_pass_body(const ForceArgs &a, const RepDesc &R, int re
             if (kW) {
                 // image-exact difference: the far coordinate is shifted by L
                 // before subtracting (same bits as dx where no shift applies)
-                if (kWX) dxa = (ox > 0.0f) ? (xim - xj) : ((ox < 0.0f) ? (xi - (xj - Lx)) : dx);
-                if (kWY) dya = (oy > 0.0f) ? (yim - yj) : ((oy < 0.0f) ? (yi - (yj - Ly)) : dy);
+                if (kWX) dxa = (px ? xim : xi) - (mx ? xj - Lx : xj);
+                if (kWY) dya = (py ? yim : yi) - (my ? yj - Ly : yj);
                 r2a = dxa * dxa + dya * dya;
             }
-            const float inv = __builtin_amdgcn_rcpf(r2a);
+            const float inv = hit ? __builtin_amdgcn_rcpf(r2a) : 0.0f;
             const float sr2 = kUnit ? inv : s2ij * inv;  // sigma^2 = 1: the same bits
             const float sr4 = sr2 * sr2;
             const float sr6 = sr4 * sr2;
             const float s12 = sr6 * sr6;
             const float tv = __builtin_fmaf(-0.5f, sr6, s12);
-            // (a non-interacting entry has r2a > 0, so its rcp is finite)
-            const float tvh = hit ? tv : 0.0f;
-            const float fc = kTypes ? e48 * tvh * inv : tvh * inv;
+            const float fc = kTypes ? e48 * tv * inv : tv * inv;
             fx = __builtin_fmaf(fc, dxa, fx);
             fy = __builtin_fmaf(fc, dya, fy);
-            if (kCount) nint += hit ? 1 : 0;
+            if (kDebug) nint += hit ? 1 : 0;
             if (kEnergy && kTypes) {
-                accT = __builtin_fmaf(e4, hit ? s12 - sr6 : 0.0f, accT);
-                accQ = __builtin_fmaf(e48, tvh, accQ);
+                accT = __builtin_fmaf(e4, s12 - sr6, accT);
+                accQ = __builtin_fmaf(e48, tv, accQ);
                 ush += hit ? shift : 0.0f;
             } else if (kEnergy) {
-                accT += tvh;
-                if (!kCount) accQ += hit ? sr6 : kq;
-                else accQ += hit ? sr6 : 0.0f;
+                accT += tv;
+                accQ += sr6;
+                nhit += (int)__popcll(__ballot(hit));
             }
             if (kDebug && hit) {
                 const long long v = (long long)lid[jo >> 3] + 1;
@@ -1977,9 +2037,9 @@ __device__ void list_tile_pass_body(const ForceArgs &a, const RepDesc &R, int re
                 d2 += v * v;
             }
         };
-        auto group = [&](auto wrapc, uint64_t cur) {
-            const int j0 = (int)(cur & 0xffffu), j1 = (int)((cur >> 16) & 0xffffu);
-            const int j2 = (int)((cur >> 32) & 0xffffu), j3 = (int)(cur >> 48);
+        auto group = [&](auto wrapc, v2u cur) {
+            const int j0 = (int)(cur.x & 0xffffu), j1 = (int)(cur.x >> 16);
+            const int j2 = (int)(cur.y & 0xffffu), j3 = (int)(cur.y >> 16);
             // entries are byte offsets of float2 staging slots
             const char *lpb = reinterpret_cast<const char *>(lp);
             const float2 q0 = *reinterpret_cast<const float2 *>(lpb + j0);
@@ -2005,36 +2065,40 @@ __device__ void list_tile_pass_body(const ForceArgs &a, const RepDesc &R, int re
             term(wrapc, q2, s2, t2, j2);
             term(wrapc, q3, s3, t3, j3);
         };
-        // the next group is loaded while this one is evaluated (the group
-        // index is clamped inside the array; a group past the list is loaded
-        // and not used); the empty asm keeps the compiler from moving the
-        // load down to its use in the next iteration
+        // two groups in flight while one is evaluated, in two registers taken
+        // in turn; the empty asm keeps the compiler from moving a load down
+        // to its use
+        const uint32_t q8 = 8u * (uint32_t)q;  // (list mode: 8 n < 2^32)
         auto groups = [&](auto wrapc) {
-            uint64_t gv = nb[(uint32_t)q];
-            for (int g = 0; g < n4; ++g) {
-                const uint64_t cur = gv;
-                gv = nb[(uint32_t)min(g + 1, capg - 1) * Nu + (uint32_t)q];
+            v2u g0 = slot.g0, g1 = slot.g1;
+            auto one = [&](int g, v2u &gr) {
+                v2u cur;
+                cur.x = g < n4 ? gr.x : pad2;
+                cur.y = g < n4 ? gr.y : pad2;
+                gr = list_group(a, g + 2, q8);
                 __asm__ volatile("" ::: "memory");
                 group(wrapc, cur);
+            };
+            for (int g = 0; g < n4w; g += 2) {
+                one(g, g0);
+                if (g + 1 >= n4w) break;
+                one(g + 1, g1);
             }
         };
         if (wimg) groups(std::integral_constant<int, kWrap>{});
         else groups(std::integral_constant<int, 0>{});
-        const int id = a.perm[p];
+        if (!act) continue;
         if (kTypes)
-            tile_kick<kKick, true, kEnergy>(a, R, id, p, xi, yi, fx, fy, tk);
+            tile_kick<kKick, true, kEnergy>(a, R, id, p, xi, yi, vx, vy, fx, fy, tk);
         else
-            tile_kick<kKick, true, kEnergy>(a, R, id, p, xi, yi, fx * pe.e48, fy * pe.e48, tk);
+            tile_kick<kKick, true, kEnergy>(a, R, id, p, xi, yi, vx, vy, fx * pe.e48, fy * pe.e48, tk);
         if (kEnergy && kTypes) {
-            Ublk += 0.5 * ((double)accT + (double)ush);
-            Wblk += 0.5 * (double)accQ;
+            Ublk += (double)accT + (double)ush;
+            Wblk += (double)accQ;
         } else if (kEnergy) {
-            const double T = accT, Q = accQ, e4 = pe.e4;
-            // kCount: Q = B exactly; otherwise Q - kq L = B - kq n
-            const double Ui = kCount ? e4 * (T - 0.5 * Q) + (double)nint * pe.shift
-                                     : e4 * T - 0.5 * e4 * (Q - (double)kq * (4.0 * n4));
-            Ublk += 0.5 * Ui;
-            Wblk += 0.5 * ((double)pe.e48 * T);
+            const double T = accT;
+            Ublk += T - 0.5 * (double)accQ;
+            Wblk += T;
         }
         if (kDebug) {
             const int u = a.uid[id];
@@ -2043,39 +2107,65 @@ __device__ void list_tile_pass_body(const ForceArgs &a, const RepDesc &R, int re
             a.dbg_s2[u] = d2;
         }
     }
-    if (kEnergy || kKick == 2) {
-        tile_reduce(Ublk, Wblk, tk, L);
-        tile_partials<kKick, true, kEnergy>(a, tile, rep, Ublk, Wblk, tk);
+    if (kEnergy && !kTypes) {
+        Ublk *= (double)pe.e4;
+        if (lane == 0) Ublk += (double)nhit * (double)pe.shift;
     }
+    tile_finish<kKick, true, kEnergy>(a, tile, rep, Ublk, Wblk, 0.5,
+                                      kTypes ? 0.5 : 0.5 * (double)pe.e48, tk, lp);
 }
 
+// One tile of the list pass.  A workgroup's time is its chain of dependent
+// loads, so everything is asked for as soon as its address is known: the
+// tile's record (the layout is not formed again), then the lanes' list slots
+// and the staged positions together, then the velocities, which arrive while
+// the lists are walked.
 template <bool kSigma, bool kTypes, bool kEnergy, bool kDebug, int kKick>
-__device__ void list_tile_pass(const ForceArgs &a, int tile, PairLds &L, float2 *lp,
-                               float *ls, int *lid, int *lt) {
+__device__ void list_tile_pass(const ForceArgs &a, int tile, PairEntry *pt, float2 *lp, float *ls,
+                               int *lid, int *lt) {
     const Tile T = a.tiles[tile];
-    const RepDesc R = a.reps[T.rep];
-    const int W = T.w_flags & 0xffff;
-    if (stage_layout(a, T, R, W, L) < 0) {
+    const TileRun V = a.runs[tile];
+    const int rep = a.nrep == 1 ? 0 : T.rep;  // (one replica: no load waits for the tile)
+    const RepDesc R = a.reps[rep];
+    if (V.m < 0) {
         atomicOr(a.err, 2u);  // FM_DEV_TILE_OVERFLOW (its particles are not moved)
-        tile_partials<kKick, true, kEnergy>(a, tile, T.rep, 0.0, 0.0, TileKick{});
+        tile_finish<kKick, true, kEnergy>(a, tile, rep, 0.0, 0.0, 0.0, 0.0, TileKick{}, lp);
         return;
     }
-    stage_copy(
-        T, R, W, L,
-        [&](int p) {
-            const float2 q = a.xys[p];
-            return make_float4(q.x, q.y, kSigma ? a.sigs[p] : 0.0f,
-                               kDebug ? __int_as_float(a.uid[a.perm[p]]) : 0.0f);
-        },
-        [&](int e, const float4 &u) {
-            lp[e] = make_float2(u.x, u.y);
-            if (kSigma) ls[e] = u.z;
-            if (kDebug) lid[e] = __float_as_int(u.w);  // caller id (diagnostic dump)
-        });
-    if (kTypes)  // the types in the same staging order (sorted positions)
-        stage_copy(
-            T, R, W, L, [&](int p) { return make_float4(__int_as_float(a.sorted_typ[p]), 0.f, 0.f, 0.f); },
-            [&](int e, const float4 &u) { lt[e] = __float_as_int(u.x); });
+    const int tid = threadIdx.x, bd = blockDim.x;
+    const ListSlot slot = list_slot(a, V.sbase + max(min(tid, V.nc - 1), 0));
+    const PairEntry pe = a.ptab[R.pt];
+    if (kTypes)
+        for (int k = tid; k < R.ntypes * R.ntypes; k += bd) pt[k] = a.ptab[R.pt + k];
+    // the three staged rows together, one particle of each per lane and pass
+    const int beg[3] = {0, V.end[0], V.end[1]};
+    const int most = max(V.end[0], max(V.end[1] - V.end[0], V.end[2] - V.end[1]));
+    for (int i = 0; i < most; i += bd) {
+        float2 x[3];
+        float sg[3];
+        int ty[3], u[3];
+#pragma unroll
+        for (int r = 0; r < 3; ++r) {
+            const int e = beg[r] + i + tid;
+            if (e < V.end[r]) {
+                const int p = e + (e >= V.o2[r] ? V.d2[r] : (e >= V.o1[r] ? V.d1[r] : V.d0[r]));
+                x[r] = a.xys[p];
+                if (kSigma) sg[r] = a.sigs[p];
+                if (kTypes) ty[r] = a.sorted_typ[p];
+                if (kDebug) u[r] = a.uid[a.perm[p]];
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < 3; ++r) {
+            const int e = beg[r] + i + tid;
+            if (e < V.end[r]) {
+                lp[e] = x[r];
+                if (kSigma) ls[e] = sg[r];
+                if (kTypes) lt[e] = ty[r];
+                if (kDebug) lid[e] = u[r];  // caller id (diagnostic dump)
+            }
+        }
+    }
     if (threadIdx.x == 0) {  // the padding entries' slot, far from any particle
         lp[a.lds_cap] = make_float2(kSentinel, kSentinel);
         if (kSigma) ls[a.lds_cap] = 1.0f;
@@ -2087,23 +2177,20 @@ __device__ void list_tile_pass(const ForceArgs &a, int tile, PairLds &L, float2 
     // a tile at the left or right edge away from the top and bottom rows
     // (it needs no y image), else both (bit 0 x, bit 1 y)
     const int wm = ((T.w_flags >> 17) & 3) == 1 ? 1 : (((T.w_flags >> 16) & 1) ? 3 : 0);
-#define FM_LPB(WR, U, C) \
-    list_tile_pass_body<WR, kSigma, kTypes, kEnergy, U, kDebug, C, kKick>(a, R, T.rep, W, tile, L, lp, ls, lid, lt)
-    // hits are counted for the dump, and for the energy when eps = 0
-    if (kDebug || (!kTypes && kEnergy && L.pt[0].e4 == 0.0f)) {
-        if (wm) FM_LPB(3, false, true);
-        else FM_LPB(0, false, true);
-    } else if (!kSigma && R.s2_uniform == 1.0f) {  // (sigma^2 = 1: the same bits)
+#define FM_LPB(WR, U) \
+    list_tile_pass_body<WR, kSigma, kTypes, kEnergy, U, kDebug, kKick>(a, R, V, rep, tile, pe, pt, slot, lp, ls, \
+                                                                       lid, lt)
+    if (!kSigma && R.s2_uniform == 1.0f && !kDebug) {  // (sigma^2 = 1: the same bits)
         switch (wm) {
-            case 1: FM_LPB(1, true, false); break;
-            case 3: FM_LPB(3, true, false); break;
-            default: FM_LPB(0, true, false);
+            case 1: FM_LPB(1, true); break;
+            case 3: FM_LPB(3, true); break;
+            default: FM_LPB(0, true);
         }
     } else {
         switch (wm) {
-            case 1: FM_LPB(1, false, false); break;
-            case 3: FM_LPB(3, false, false); break;
-            default: FM_LPB(0, false, false);
+            case 1: FM_LPB(1, false); break;
+            case 3: FM_LPB(3, false); break;
+            default: FM_LPB(0, false);
         }
     }
 #undef FM_LPB
@@ -2241,70 +2328,77 @@ __device__ void bond_block(const ForceArgs &a, int b, double *red) {
     }
 }
 
+// Bookkeeping workgroups of a force pass (per replica two jobs, a wavefront
+// each): apart from the tiles, whose path they would lengthen.
+__host__ __device__ inline int forces_book(const ForceArgs &a) {
+    return a.nrep < 128 ? (a.nrep + 1) / 2 : 64;
+}
+
+// Per replica: the previous step's observables, level 2; and (the rebuild of
+// this step, if any, is complete) its summary cleared, this step folded into
+// the replica's displacement bound (zero after a rebuild) and the
+// displacement slots cleared for the next kick.  The diagnostic dump pass
+// leaves the rebuild state alone.
+template <bool kList, bool kDebug>
+__device__ void step_book(const ForceArgs &a, int b, int nb) {
+    const int wv = threadIdx.x >> 6, nw = blockDim.x >> 6, lane = threadIdx.x & 63;
+    if (kList && !kDebug && b == 0 && threadIdx.x == 0 && a.any) *a.any = 0;
+    for (int j = b * nw + wv; j < 2 * a.nrep; j += nb * nw) {  // (uniform per wavefront)
+        const int r = j >> 1;
+        if (j & 1) {
+            if (a.obs_l2) obs_finish(a.obs, r, true);
+        } else if (kList && !kDebug) {
+            const float d = list_disp(a.dmax, a.ctl_w, r, a.reps[r]);
+            if (lane == 0) a.ctl_w[r].disp = a.ctl_w[r].flag ? 0.0f : d;
+            if (lane < kDispSlots) a.dmax[((size_t)r * kDispSlots + lane) * kDispStride] = 0u;
+        }
+    }
+}
+
 // The force pass (femmd2D/src/interactions.cpp:83-109).  kKick: 0 forces
 // only; 1 forces and the closing second half-kick of a run; 2 forces, the
 // second half-kick of this step and the first half-kick, drift and wrap of
 // the next (femmd2D/src/integrator.cpp:8-29), for every particle without
 // element or bond corners (tile_kick).
-// (8 wavefronts per SIMD: measured faster than the 6 its registers would
-// otherwise allow, at the cost of one spilled register)
+// Wavefronts per SIMD: the list pass 6 (5 with a type table), where what it
+// keeps in flight needs no spilled register (1.14 million particles: 38 us;
+// 39 at 7, 45 at 8 with 14 spilled, 42 at 5; 30,011 particles of six types:
+// 10.8 us at 5, 12.1 at 6); the cell walk 8.
+template <bool kList, bool kTypes>
+constexpr int kForceWaves = kList ? (kTypes ? 5 : 6) : 8;
 template <bool kSigma, bool kTypes, bool kDebug, bool kList, bool kEnergy, int kKick>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_forces(ForceArgs a) {
+__global__ __launch_bounds__(256) __attribute__((
+    amdgpu_waves_per_eu(kForceWaves<kList, kTypes>, kForceWaves<kList, kTypes>))) void
+k_forces(ForceArgs a) {
     extern __shared__ float4 dyn[];
     __shared__ int s_cstart[kMaxSlots];
     __shared__ int s_off[kMaxSlots + 1];
     __shared__ PairEntry s_pt[kMaxPairTypes * kMaxPairTypes];
-    __shared__ double s_red[3 * 4];
-    __shared__ float s_redf[2 * 4];
+    __shared__ double s_red[2 * 4];
     int b = blockIdx.x;
-    // the previous step's observables, level 2 (one thread per replica)
-    if (a.obs_l2 && threadIdx.x == 0)
-        for (int r = blockIdx.x; r < a.obs.nrep; r += gridDim.x) obs_finish(a.obs, r, true);
-    // the rebuild of this step (if any) is complete: clear its summary,
-    // fold this step into each replica's displacement bound (zero after a
-    // rebuild) and clear the displacement slots for the next kick
-    // (the diagnostic dump pass leaves the rebuild state alone)
-    if (kList && !kDebug) {
-        if (b == 0 && a.any && threadIdx.x == 0) *a.any = 0;
-        // replica r by workgroup r (the first wavefront): bound, then slots
-        if (threadIdx.x < 64) {
-            for (int r = blockIdx.x; r < a.nrep; r += gridDim.x) {
-                const float d = list_disp(a.dmax, a.ctl_w, r, a.reps[r]);
-                if (threadIdx.x == 0) a.ctl_w[r].disp = a.ctl_w[r].flag ? 0.0f : d;
-                if (threadIdx.x < kDispSlots)
-                    a.dmax[((size_t)r * kDispSlots + threadIdx.x) * kDispStride] = 0u;
-            }
-        }
-    }
-    // element and bond workgroups first (a whole number of rounds over the
-    // 8 XCDs, so each XCD's tiles still form one contiguous band), then the
-    // tiles: the kernel's tail is made of the uniform tile work
+    // element and bond workgroups first, then the bookkeeping of the step (a
+    // whole number of rounds over the 8 XCDs together, so each XCD's tiles
+    // still form one contiguous band), then the tiles: the kernel's tail is
+    // made of the uniform tile work
     {
         const int ne = a.nespans + a.nbspans;
-        const int nfirst = (ne + 7) & ~7;
+        const int nb = forces_book(a);
+        const int nfirst = (ne + nb + 7) & ~7;
         if (b < nfirst) {
             if (b < a.nespans) elem_block(a, b, s_red);
             else if (b < ne) bond_block(a, b - a.nespans, s_red);
+            else if (b < ne + nb) step_book<kList, kDebug>(a, b - ne, nb);
             return;
         }
         b -= nfirst;
     }
     if (kList) {
         if (b < a.ntiles) {
-            PairLds L;
-            L.ent = nullptr;
-            L.typ = nullptr;
-            L.sp = nullptr;
-            L.cstart = s_cstart;
-            L.off = s_off;
-            L.pt = s_pt;
-            L.red = s_red;
-            L.redf = s_redf;
             float2 *lp = reinterpret_cast<float2 *>(dyn);
             float *ls = reinterpret_cast<float *>(lp + a.lds_cap + 1);
             int *lid = reinterpret_cast<int *>(ls + (kSigma ? a.lds_cap + 1 : 0));
             int *lt = lid + (kDebug ? a.lds_cap + 1 : 0);
-            list_tile_pass<kSigma, kTypes, kEnergy, kDebug, kKick>(a, xcd_remap(b, a.ntiles), L, lp,
+            list_tile_pass<kSigma, kTypes, kEnergy, kDebug, kKick>(a, xcd_remap(b, a.ntiles), s_pt, lp,
                                                                    ls, lid, lt);
         }
     } else if (b < a.ntiles) {
@@ -2317,15 +2411,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
         L.off = s_off;
         L.pt = s_pt;
         L.red = s_red;
-        L.redf = s_redf;
         pair_tile<kSigma, kTypes, kDebug, kEnergy, kKick>(a, xcd_remap(b, a.ntiles), L);
     }
 }
 
-// Workgroups of one force pass: element and bond spans (rounded up to a
-// multiple of 8), then the tiles.
+// Workgroups of one force pass: element and bond spans and the bookkeeping
+// (rounded up to a multiple of 8), then the tiles.
 __host__ __device__ inline int forces_grid(const ForceArgs &a) {
-    return ((a.nespans + a.nbspans + 7) & ~7) + a.ntiles;
+    return ((a.nespans + a.nbspans + forces_book(a) + 7) & ~7) + a.ntiles;
 }
 
 // Total force per particle (pair + gathered corners), internal order.
@@ -2357,8 +2450,8 @@ __global__ __launch_bounds__(256) void k_observe_l1(ObsArgs o) {
     __shared__ double red[kObsRed];
     obs_level1(o, red);
 }
-__global__ __launch_bounds__(64) void k_observe_l2(ObsArgs o, int accumulate) {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(256) void k_observe_l2(ObsArgs o, int accumulate) {
+    const int r = blockIdx.x * 4 + (int)(threadIdx.x >> 6);  // one wavefront per replica
     if (r < o.nrep) obs_finish(o, r, accumulate != 0);
 }
 
@@ -2366,8 +2459,7 @@ hipError_t launch_observe(const ObsArgs &o, bool accumulate, hipStream_t s) {
     if (o.nrep <= 0) return hipSuccess;
     hipLaunchKernelGGL(k_observe_l1, dim3(std::min(o.nrep * o.nchunk, 4096)), dim3(256), 0, s,
                        o);
-    hipLaunchKernelGGL(k_observe_l2, dim3((o.nrep + 63) / 64), dim3(64), 0, s, o,
-                       accumulate ? 1 : 0);
+    hipLaunchKernelGGL(k_observe_l2, dim3((o.nrep + 3) / 4), dim3(256), 0, s, o, accumulate ? 1 : 0);
     return hipGetLastError();
 }
 
@@ -3261,9 +3353,10 @@ hipError_t launch_forces(bool sigma, bool types, bool debug, bool list, bool ene
     if (list) {
         // neighbour lists (types: the pair table per pair); debug: the
         // interacting-set dump over the lists (with energies)
-        const size_t lds = (size_t)(a.lds_cap + 1) *
-                           (sizeof(float2) + (sigma ? sizeof(float) : 0) + (debug ? sizeof(int) : 0) +
-                            (types ? sizeof(int) : 0));
+        const size_t lds = std::max(tile_scratch_bytes(block),
+                                    (size_t)(a.lds_cap + 1) *
+                                        (sizeof(float2) + (sigma ? sizeof(float) : 0) +
+                                         (debug ? sizeof(int) : 0) + (types ? sizeof(int) : 0)));
 #define FM_LIST(S, T, D, E, K) FM_GO((k_forces<S, T, D, true, E, K>), g, b, lds, s, a)
 #define FM_LIST_K(S, T, E)                    \
     do {                                      \
@@ -3286,7 +3379,7 @@ hipError_t launch_forces(bool sigma, bool types, bool debug, bool list, bool ene
 #undef FM_LIST
         return hipGetLastError();
     }
-    const size_t lds = forces_lds_bytes(a.lds_cap, types, debug);
+    const size_t lds = std::max(tile_scratch_bytes(block), forces_lds_bytes(a.lds_cap, types, debug));
 #define FM_LAUNCH(S, T, D, E, K) FM_GO((k_forces<S, T, D, false, E, K>), g, b, lds, s, a)
 #define FM_LAUNCH_K(S, T, E)                    \
     do {                                        \
@@ -3422,13 +3515,14 @@ hipError_t launch_vel_scale(const int32_t *ids, int n, float *vx, float *vy, flo
 // cluster refers to them) new internal ids in the order of the last
 // counting sort, on the same set of internal slots, so no topology changes:
 // the k-th movable particle in sorted order takes the k-th movable slot.
-// perm and spos are rewritten for the new ids (the sorted order itself, and
-// so the neighbour lists, stay valid); the per-particle arrays are gathered
-// through oldof.
+// perm, spos and lid are rewritten for the new ids (the sorted order itself,
+// and so the neighbour lists, stay valid); the per-particle arrays are
+// gathered through oldof.
 //   k_ro_count   movable count per chunk of sorted slots
 //   k_ro_scan    exclusive prefix of the chunk counts (one workgroup)
-//   k_ro_map     rank of each movable particle -> new id; oldof, perm, spos
-//   k_ro_gather  tmp[k][q] = arr[k][oldof[q]]
+//   k_ro_map     rank of each movable particle -> new id; oldof, newof, perm,
+//                spos
+//   k_ro_gather  tmp[k][q] = arr[k][oldof[q]], lid[q] = newof[lid[q]]
 //   k_ro_copy    arr[k][q] = tmp[k][q]
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ int ro_flags(const ReorderArgs &a, int b, int4 &ids) {
@@ -3500,6 +3594,7 @@ __global__ __launch_bounds__(256) void k_ro_map(ReorderArgs a) {
         const bool mv = ((m >> u) & 1) && rank < a.nmov;
         const int nid = mv ? a.movids[rank++] : id;
         a.oldof[nid] = id;
+        if (a.newof) a.newof[id] = nid;
         a.perm[s0 + u] = nid;
         if (a.spos) a.spos[nid] = s0 + u;
     }
@@ -3510,6 +3605,7 @@ __global__ __launch_bounds__(256) void k_ro_gather(ReorderArgs a) {
     if (q >= a.n) return;
     int o = a.oldof[q];
     if ((unsigned)o >= (unsigned)a.n) o = q;  // only after a dropped particle
+    if (a.lid) a.lid[q] = a.newof[a.lid[q]];
     for (int k = 0; k < a.narr; ++k) a.tmp[(size_t)k * a.n + q] = a.arr[k][o];
 }
 
