@@ -340,8 +340,8 @@ int Engine::adj_record_segment(int len, bool close) {
     }
     if (hipGraphLaunch(ex, stream_) != hipSuccess) return -1;
     // the host state the segment leaves: one drift per step of it (each
-    // flips the list-mode parity), bins pending after a drift (cell walk)
-    par_ = par0 ^ ((len & 1) && list_ ? 1 : 0);
+    // flips the parity), bins pending after a drift (cell walk)
+    par_ = par0 ^ (len & 1);
     bins_pending_ = !list_ && !close;
     ene_valid_ = false;
     return 0;

@@ -55,8 +55,8 @@ struct alignas(16) RepDesc {
     float im_uniform;  // 1/m shared by every particle of the replica (the
                        // kick then loads no inv_m); 0: masses differ
     int32_t pg;        // particles [pg, p1) have element or bond corners (or
-                       // the replica has no pair forces): the node kick
-                       // integrates them, the force pass the others
+                       // the replica has no pair forces: no tile integrates
+                       // them, the node kick does)
     float rc_list;     // list mode: the largest cutoff of the pair table (in
                        // sigma units); lists hold every pair within
                        // rc_list * sigma_ij + skin
@@ -246,6 +246,32 @@ struct ScanArgs {
     int32_t obs_l1;            // (cell walk) form the previous step's level-1 chunks
 };
 
+// Elements and bonds: corner forces of the current positions, by workgroups
+// of their own beside the binning (list mode) or the sort (cell walk), before
+// the force pass, whose kick gathers them.
+struct ElemArgs {
+    const RepDesc *reps;
+    int32_t nrep;
+    const Span *espans;        // kElemThreads elements each
+    int32_t nespans, ntri;
+    const int32_t *t0, *t1, *t2;
+    const float4 *dmbm;        // per element: Dm {00,01,10,11}, Bm {00,01,10,11}
+    const float2 *alm;         // A0 * lambda, A0 * mu
+    int32_t model;             // 0 NH, 1 SVK (legacy is SVK with doubled moduli)
+    const float *x, *y;        // current positions, internal order
+    float2 *cf;                // corner forces out, in gather order
+    const int32_t *gpos;       // corner slot (3e + k, then bonds 2l + k) ->
+                               // its entry in the per-particle gather order
+    double *fea_part;          // 2 per element workgroup: U, W
+    const Span *bspans;        // kElemThreads bonds each
+    int32_t nbspans, nbond;
+    const int32_t *bi, *bj;
+    const float *bk, *br0;
+    int32_t cf_bond0;          // first corner slot of the bonds
+    double *bond_part;         // 2 per bond workgroup: U, W
+    uint32_t *err;
+};
+
 struct ForceArgs {
     const RepDesc *reps;
     const PairEntry *ptab;
@@ -259,25 +285,9 @@ struct ForceArgs {
     const int32_t *sorted_typ;
     float *fx, *fy;            // pair forces out, internal order
     double *lj_part;           // 2 per tile: U, W
-    // element role
-    const Span *espans;
-    int32_t nespans;
-    const int32_t *t0, *t1, *t2;
-    const float4 *dmbm;        // per element: Dm {00,01,10,11}, Bm {00,01,10,11}
-    const float2 *alm;         // A0 * lambda, A0 * mu
-    int32_t model;             // 0 NH, 1 SVK (legacy is SVK with doubled moduli)
+    ElemArgs el;               // elements and bonds (the adjoint pass; their
+                               // corner forces, gathered by the kick)
     const float *x, *y;        // current positions, internal order
-    float2 *cf;                // corner forces out, in gather order
-    const int32_t *gpos;       // corner slot (3e + k, then bonds 2l + k) ->
-                               // its entry in the per-particle gather order
-    double *fea_part;          // 2 per element workgroup: U, W
-    // bond role
-    const Span *bspans;
-    int32_t nbspans;
-    const int32_t *bi, *bj;
-    const float *bk, *br0;
-    int32_t cf_bond0;          // first corner slot of the bonds
-    double *bond_part;         // 2 per bond workgroup: U, W
     // neighbour-list mode (pair role over the tiles of the list build)
     int32_t nbr_cap;           // list capacity per particle (multiple of 8)
     void *nbr;                 // neighbours of the particle at sorted position
@@ -312,10 +322,9 @@ struct ForceArgs {
     ObsArgs obs;               // per-step observables
     int32_t obs_l2;            // combine the previous step's chunks and accumulate
     // The kick of the pass (kick modes of k_forces): each tile integrates its
-    // centre particles that have no element or bond corners (the others are
-    // left to the node kick, which needs their gathered corner forces):
-    // second half-kick of the previous step with the kinetic energy and, in
-    // the step mode, first half-kick, drift and wrap.
+    // centre particles (their element and bond corner forces gathered from
+    // el.cf): second half-kick of the previous step with the kinetic energy
+    // and, in the step mode, first half-kick, drift and wrap.
     float *xw, *yw;            // internal positions written (the same arrays as x, y)
     float *vx, *vy;
     const float *inv_m, *mass;

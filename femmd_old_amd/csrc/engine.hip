@@ -238,9 +238,8 @@ int Engine::build(const std::vector<const HostSystem *> &reps, std::unique_ptr<E
         }
         // wrap, key, internal order of this replica: the particles without
         // element or bond corners in cell order, then those with corners (and
-        // every particle of a replica without pair forces) in cell order.
-        // The force pass kicks the first group itself; the node kick takes
-        // the second, [pg, p1), as one contiguous range.
+        // every particle of a replica without pair forces) in cell order,
+        // [pg, p1), as one contiguous range.
         std::vector<float> xw(n), yw(n);
         std::vector<int> key(n), order(n);
         std::vector<char> gat(n, S.lj_on ? 0 : 1);
@@ -493,17 +492,18 @@ int Engine::build(const std::vector<const HostSystem *> &reps, std::unique_ptr<E
     FM_AL(cf_, std::max(1, 3 * E->ntri_ + 2 * E->nbond_));
     FM_AL(ke_part_, 2 * std::max<size_t>(ks.size(), 1));
     {
-        // the node kick: per replica its particles [pg, p1) (those with
-        // element or bond corners, and every particle of a replica without
-        // pair forces: no tile kicks them), spans of kKickThreads
+        // the node kick: the particles of the replicas without pair forces
+        // (no tile kicks them), spans of kKickThreads
         hnr.assign(2 * R, 0);
         E->nnode_ = 0;
         for (int r = 0; r < R; ++r) {
             hnr[2 * r] = (int)hns.size();
-            for (int b = rd[r].pg; b < rd[r].p1; b += kKickThreads)
-                hns.push_back(Span{r, b, std::min(b + kKickThreads, rd[r].p1), 0});
+            if (!reps[r]->lj_on) {
+                for (int b = rd[r].p0; b < rd[r].p1; b += kKickThreads)
+                    hns.push_back(Span{r, b, std::min(b + kKickThreads, rd[r].p1), 0});
+                E->nnode_ += rd[r].p1 - rd[r].p0;
+            }
             hnr[2 * r + 1] = (int)hns.size();
-            E->nnode_ += rd[r].p1 - rd[r].pg;
         }
         E->nspans_h_ = hns;
         if ((he = upload(E->nspans_, hns, st)) != hipSuccess ||
@@ -511,8 +511,8 @@ int Engine::build(const std::vector<const HostSystem *> &reps, std::unique_ptr<E
             return E->check(he, "upload node kick", err);
         FM_AL(ke_node_, 2 * std::max<size_t>(hns.size(), 1));
     }
-    FM_AL(fea_part_, 2 * std::max<size_t>(es.size(), 1));
-    FM_AL(bond_part_, 2 * std::max<size_t>(bs.size(), 1));
+    FM_AL(fea_part_, 2 * 2 * std::max<size_t>(es.size(), 1));  // two sets (par_)
+    FM_AL(bond_part_, 2 * 2 * std::max<size_t>(bs.size(), 1));
     FM_AL(obs_chunk_, (size_t)R * kObsChunks * kObsRaw);
     FM_AL(obs_, (size_t)R * kObsStride);
     FM_AL(err_, 1);
@@ -726,8 +726,10 @@ int Engine::launch_bin(bool gated) {
     a.cap = cap_;
     a.err = err_.p;
     a.nspans = (int)kspans_h_.size();
-    a.obs = obs_args();
+    a.obs = obs_args(true);
     a.obs_l1 = (gated && l1_) ? 1 : 0;
+    ElemArgs el{};  // a step's element and bond forces beside its gated binning
+    if (gated) el = elem_args();
     if (gated) {  // list mode: decide and bin only the replicas that rebuild
         a.ctl = ctl_.p;
         a.any = any_.p;
@@ -754,7 +756,7 @@ int Engine::launch_bin(bool gated) {
             a.nfs = nf_.p;
         }
     }
-    return launch_kick(0, false, false, (int)kspans_h_.size(), a, stream_) == hipSuccess ? 0 : -1;
+    return ::fm::launch_bin(a, el, stream_) == hipSuccess ? 0 : -1;
 }
 
 // The kick arguments shared by the first half-kick of a run (every
@@ -794,15 +796,15 @@ KickArgs Engine::kick_args(bool drift) {
 //         from the stored forces (k_kick);
 //   body  (drift, kick2):  the neighbour update of the current positions
 //         (list mode: binning, counting sort and list build gated on the
-//         rebuild decision; cell walk: the sort of the last binning), then
-//         the force pass, which also gives every particle without element or
-//         bond corners its second half-kick of this step and the first
-//         half-kick, drift and wrap of the next, then the node kick of the
-//         others (their gathered corner forces added);
+//         rebuild decision; cell walk: the sort of the last binning) with
+//         the element and bond forces beside its first kernel, then the
+//         force pass, which also gives every particle its second half-kick of
+//         this step and the first half-kick, drift and wrap of the next (the
+//         node kick does so for replicas without pair forces);
 //   close (!drift, kick2): as a body with the second half-kick only; the
 //         forces are stored for the next run's first half-kick.
-// In list mode the drift writes the other buffer of the sorted-order
-// positions and displacement slots (par_ flips).
+// Every drift flips par_; in list mode it writes the other buffer of the
+// sorted-order positions and displacement slots.
 int Engine::launch_step_body(bool kick2, bool drift, bool energy, bool l1, bool l2) {
     struct Restore {  // the flags of this body, restored on every return
         Engine *e;
@@ -815,10 +817,12 @@ int Engine::launch_step_body(bool kick2, bool drift, bool energy, bool l1, bool 
     if (!kick2) {
         if (!drift) return 0;
         const KickArgs k = kick_args(true);
+        time_next(0);
         const hipError_t e = launch_kick(1, gather_, false, (int)kspans_h_.size(), k, stream_);
+        arm_kernel_timer(nullptr, nullptr);
         if (e != hipSuccess) return -1;
-        if (list_) par_ ^= 1;
-        else bins_pending_ = true;
+        par_ ^= 1;
+        if (!list_) bins_pending_ = true;
         return 0;
     }
     if (list_) {
@@ -831,7 +835,7 @@ int Engine::launch_step_body(bool kick2, bool drift, bool energy, bool l1, bool 
         if (launch_sort(true)) return -1;
         if (launch_list_build(true)) return -1;
     } else {
-        if (launch_sort()) return -1;  // the binning of the last drift
+        if (launch_sort(false, true)) return -1;  // the binning of the last drift
     }
     {
         const ForceArgs f = force_args();
@@ -854,13 +858,13 @@ int Engine::launch_step_body(bool kick2, bool drift, bool energy, bool l1, bool 
         arm_kernel_timer(nullptr, nullptr);
         if (e != hipSuccess) return -1;
     }
-    if (drift && list_) par_ ^= 1;
+    if (drift) par_ ^= 1;
     if (drift && !list_) bins_pending_ = true;  // the next body's sort consumes it
     return 0;
 }
 
 // Counting sort of the last binning (single pass: scan and scatter).
-int Engine::launch_sort(bool gated) {
+int Engine::launch_sort(bool gated, bool elems) {
     ScanArgs s{};
     s.reps = reps_.p;
     s.nrep = R_;
@@ -883,7 +887,7 @@ int Engine::launch_sort(bool gated) {
     s.sorted = sorted_.p;
     s.sorted_typ = types_ ? sorted_typ_.p : nullptr;
     s.err = err_.p;
-    s.obs = obs_args();
+    s.obs = obs_args(true);
     s.obs_l1 = (!list_ && l1_) ? 1 : 0;  // the cell walk's sort forms level 1
     if (list_) {
         s.spos = spos_.p;
@@ -900,7 +904,7 @@ int Engine::launch_sort(bool gated) {
         }
     }
     time_next(2);
-    const hipError_t e = ::fm::launch_sort(s, stream_);
+    const hipError_t e = ::fm::launch_sort(s, elems ? elem_args() : ElemArgs{}, stream_);
     arm_kernel_timer(nullptr, nullptr);
     if (!gated) bins_pending_ = false;
     return e == hipSuccess ? 0 : -1;
@@ -921,6 +925,7 @@ int Engine::launch_list_build(bool gated) {
 }
 
 int Engine::launch_pair_pass() {
+    if (launch_elems(elem_args(), stream_) != hipSuccess) return -1;
     const ForceArgs f = force_args();
     time_next(4);
     const hipError_t e = launch_forces(sigma_, types_, false, true, energy_, 0, block_, f, stream_);
@@ -931,7 +936,7 @@ int Engine::launch_pair_pass() {
 
 // Cell-walk force pass over the current binning (sort first).
 int Engine::launch_forces_only(bool debug) {
-    if (launch_sort()) return -1;  // (the binning is in the kick)
+    if (launch_sort(false, true)) return -1;  // (the binning is in the kick)
     const ForceArgs f = force_args();
     time_next(4);
     const hipError_t e =
@@ -955,27 +960,9 @@ ForceArgs Engine::force_args() {
     f.fx = fx_.p;
     f.fy = fy_.p;
     f.lj_part = lj_part_.p;
-    f.espans = espans_.p;
-    f.nespans = (int)espans_h_.size();
-    f.t0 = t0_.p;
-    f.t1 = t1_.p;
-    f.t2 = t2_.p;
-    f.dmbm = dmbm_.p;
-    f.alm = alm_.p;
-    f.model = (model_ == FM_NEO_HOOKEAN) ? 0 : 1;
+    f.el = elem_args();
     f.x = xcur();
     f.y = ycur();
-    f.cf = cf_.p;
-    f.gpos = gpos_.p;
-    f.fea_part = fea_part_.p;
-    f.bspans = bspans_.p;
-    f.nbspans = (int)bspans_h_.size();
-    f.bi = bi_.p;
-    f.bj = bj_.p;
-    f.bk = bk_.p;
-    f.br0 = br0_.p;
-    f.cf_bond0 = 3 * ntri_;
-    f.bond_part = bond_part_.p;
     f.nbr_cap = nbr_cap_;
     f.nbr = nbr_.p;
     f.nnum = nnum_.p;
@@ -1017,7 +1004,39 @@ ForceArgs Engine::force_args() {
     return f;
 }
 
-ObsArgs Engine::obs_args() {
+ElemArgs Engine::elem_args() {
+    ElemArgs e{};
+    e.reps = reps_.p;
+    e.nrep = R_;
+    e.espans = espans_.p;
+    e.nespans = (int)espans_h_.size();
+    e.ntri = ntri_;
+    e.t0 = t0_.p;
+    e.t1 = t1_.p;
+    e.t2 = t2_.p;
+    e.dmbm = dmbm_.p;
+    e.alm = alm_.p;
+    e.model = (model_ == FM_NEO_HOOKEAN) ? 0 : 1;
+    e.x = xcur();
+    e.y = ycur();
+    e.cf = cf_.p;
+    e.gpos = gpos_.p;
+    e.fea_part = fea_part_.p + (size_t)par_ * (fea_part_.n / 2);
+    e.bspans = bspans_.p;
+    e.nbspans = (int)bspans_h_.size();
+    e.nbond = nbond_;
+    e.bi = bi_.p;
+    e.bj = bj_.p;
+    e.bk = bk_.p;
+    e.br0 = br0_.p;
+    e.cf_bond0 = 3 * ntri_;
+    e.bond_part = bond_part_.p + (size_t)par_ * (bond_part_.n / 2);
+    e.err = err_.p;
+    return e;
+}
+
+ObsArgs Engine::obs_args(bool prev) {
+    const size_t set = (size_t)(prev ? par_ ^ 1 : par_);
     ObsArgs o{};
     o.reps = reps_.p;
     o.rng = rng_.p;
@@ -1027,8 +1046,8 @@ ObsArgs Engine::obs_args() {
     o.ke_tile = ke_tile_.p;
     o.ke_node = ke_node_.p;
     o.lj_part = lj_part_.p;
-    o.fea_part = fea_part_.p;
-    o.bond_part = bond_part_.p;
+    o.fea_part = fea_part_.p + set * (fea_part_.n / 2);
+    o.bond_part = bond_part_.p + set * (bond_part_.n / 2);
     o.chunk = obs_chunk_.p;
     o.obs = obs_.p;
     o.nrep = R_;
@@ -1039,17 +1058,18 @@ ObsArgs Engine::obs_args() {
     return o;
 }
 
-// Per-kernel device time of nsteps step bodies (no graph): HIP events on
-// the engine's stream around each launch.  out[0..5] = kick (+ bin in cell
-// mode), bin, sort, list build, forces, whole body, in ms per step (list
-// mode: the rebuild kernels are gated, so their time is the average over
-// rebuild and skip steps).
+// Per-kernel device time of nsteps steps (no graph): each dispatch's start and
+// end.  out[0..5] = kick (the run's first half-kick; and the node kick, where
+// a step has one), bin, sort, list build, forces, whole step, in ms per step
+// (list mode: the rebuild kernels are gated, so their time is the average
+// over rebuild and skip steps; the binning, or the cell walk's sort, carries
+// the element and bond forces).
 int Engine::profile(int nsteps, double *out, std::string &err) {
     if (nsteps <= 0) { err = "nsteps must be > 0"; return FM_ERR_ARG; }
     int rc = ensure_primed(err);
     if (rc) return rc;
     const int K = 2 * kProfKernels;
-    std::vector<hipEvent_t> ev(K * nsteps);
+    std::vector<hipEvent_t> ev(K * nsteps + 2);  // and the first half-kick's
     for (auto &e : ev) {
         rc = check(hipEventCreate(&e), "event", err);
         if (rc) return rc;
@@ -1060,7 +1080,10 @@ int Engine::profile(int nsteps, double *out, std::string &err) {
     const bool every = obs_every_ > 0;
     obs_valid_ = false;
     (void)every;
-    if (launch_bodies_eager(kind_open())) return check(hipGetLastError(), "step", err);
+    prof_ev_ = &ev[K * nsteps];
+    const int bad_open = launch_bodies_eager(kind_open());
+    prof_ev_ = nullptr;
+    if (bad_open) return check(hipGetLastError(), "step", err);
     for (int s = 0; s < nsteps; ++s) {
         prof_ev_ = &ev[K * s];
         const BodyKind k = s == 0 ? kind_first() : kind_body(1);
@@ -1074,9 +1097,10 @@ int Engine::profile(int nsteps, double *out, std::string &err) {
     rc = sync(err);
     if (!rc) obs_valid_ = true;
     // out[k] = dispatch duration of kernel k (0 where the mode launches no
-    // such kernel: its events were never recorded), out[5] = whole body,
-    // from its first kernel's start (binning in list mode, else the sort) to
-    // its last kernel's end (the node kick, else the force pass)
+    // such kernel: its events were never recorded), out[5] = whole step: the
+    // bodies, from the first kernel's start (binning in list mode, else the
+    // sort) to the last kernel's end (the node kick, else the force pass), and
+    // the first half-kick
     double acc[kProfKernels + 1] = {0};
     const int k_first = list_ ? 1 : 2, k_last = nnode_ > 0 ? 0 : 4;
     for (int s = 0; s < nsteps && !rc; ++s) {
@@ -1086,6 +1110,11 @@ int Engine::profile(int nsteps, double *out, std::string &err) {
             if (hipEventElapsedTime(&t, e[2 * k], e[2 * k + 1]) == hipSuccess) acc[k] += t;
         if (hipEventElapsedTime(&t, e[2 * k_first], e[2 * k_last + 1]) == hipSuccess)
             acc[kProfKernels] += t;
+    }
+    float t_open = 0.0f;
+    if (!rc && hipEventElapsedTime(&t_open, ev[K * nsteps], ev[K * nsteps + 1]) == hipSuccess) {
+        acc[0] += t_open;
+        acc[kProfKernels] += t_open;
     }
     (void)hipGetLastError();  // the elapsed times of unrecorded events failed
     for (auto &e : ev) (void)hipEventDestroy(e);
@@ -1236,7 +1265,7 @@ int Engine::launch_bodies(const BodyKind &k) {
     hipGraphExec_t ex = graph_of(k);
     if (!ex) return -1;
     if (hipGraphLaunch(ex, stream_) != hipSuccess) return -1;
-    if (list_ && k.drift) par_ ^= (k.count & 1);  // each drift flips the parity
+    if (k.drift) par_ ^= (k.count & 1);           // each drift flips the parity
     if (!list_) bins_pending_ = k.drift;          // a body or the opening kick bins
     return 0;
 }
@@ -1264,7 +1293,7 @@ int Engine::prepare_graphs() {
     const int par0 = par_;
     const BodyKind kinds[] = {kind_open(), kind_first(), kind_body(kGraphSteps), kind_body(1),
                               kind_close(true), kind_close(false)};
-    for (int p = 0; p < (list_ ? 2 : 1); ++p) {
+    for (int p = 0; p < 2; ++p) {
         par_ = p;
         for (const BodyKind &k : kinds)
             if (!graph_of(k)) {

@@ -198,16 +198,21 @@ private:
     // that the first run of any length already replays graphs only
     int prepare_graphs();
     int launch_forces_only(bool debug);
-    int launch_sort(bool gated = false);
+    // elems: with the element and bond forces of the current positions
+    int launch_sort(bool gated = false, bool elems = false);
     int launch_list_build(bool gated);
     int launch_pair_pass();  // list mode: list pair pass + elements + bonds
     ForceArgs force_args();
+    ElemArgs elem_args();
     KickArgs kick_args(bool drift);
-    ObsArgs obs_args();
-    // list mode: the sorted-order positions and displacement slots come in
-    // pairs; par_ names the buffer that holds the current positions (and the
-    // slots of the drift that produced them), the other one receives the
-    // next drift's
+    // the observables of the current positions, or (prev) of the step before:
+    // what level 1 forms while the current ones' element forces are computed
+    ObsArgs obs_args(bool prev = false);
+    // every drift flips par_.  The element and bond partials come in pairs,
+    // par_ naming those of the current positions; list mode: the sorted-order
+    // positions and displacement slots too (par_: the current positions and
+    // the slots of the drift that produced them; the other receives the next
+    // drift's)
     int par_ = 0;
     // cell walk: a drift's binning not yet consumed by a sort (a body ends
     // with the next step's binning pending); a fresh binning clears it first
@@ -323,10 +328,10 @@ private:
     DBuf<float2> alm_, cf_;
     DBuf<float> bk_, br0_;
     DBuf<double> ke_part_, lj_part_, fea_part_, bond_part_;
-    // node kick: the number of particles it integrates (per replica
-    // [pg, p1)), its spans (per replica [nrng[2r], nrng[2r+1])) and their
-    // kinetic-energy partials; the force pass's partials of the particles it
-    // integrates, per tile
+    // node kick: the number of particles it integrates (those of the replicas
+    // without pair forces: no tile), its spans (per replica [nrng[2r],
+    // nrng[2r+1])) and their kinetic-energy partials; the force pass's
+    // partials of the particles it integrates, per tile
     int nnode_ = 0;
     DBuf<int32_t> nrng_;
     DBuf<Span> nspans_;
@@ -374,7 +379,11 @@ private:
 // launchers (kernels.hip)
 hipError_t launch_kick(int mode, bool gather, bool energy, int nblk, const KickArgs &a,
                        hipStream_t s);
-hipError_t launch_sort(const ScanArgs &a, hipStream_t s);
+// binning and sort, with the element and bond forces beside them (el may
+// hold none)
+hipError_t launch_bin(const KickArgs &a, const ElemArgs &el, hipStream_t s);
+hipError_t launch_sort(const ScanArgs &a, const ElemArgs &el, hipStream_t s);
+hipError_t launch_elems(const ElemArgs &el, hipStream_t s);
 hipError_t launch_forces(bool sigma, bool types, bool debug, bool list, bool energy, int kick,
                          int block, const ForceArgs &a, hipStream_t s);
 hipError_t launch_list_build(bool sigma, int block, const ForceArgs &a, hipStream_t s);

@@ -4,21 +4,22 @@
 //   k_kick       first half-kick, drift and wrap of every particle from the
 //                stored forces (the start of a run; cell walk: binning)
 // then per step (femmd2D/src/integrator.cpp:8-29):
-//   k_bin        list mode: rebuild decision (displacement bound > skin/2)
+//   k_bin        list mode: CST elements and harmonic bonds (corner forces
+//                into a buffer in gather order, no atomics) by workgroups of
+//                their own; rebuild decision (displacement bound > skin/2)
 //                and binning of the replicas that rebuild (gated)
 //   k_sort       single-pass counting sort of the binning (decoupled
-//                look-back): cell starts, sorted order, sorted copies
+//                look-back): cell starts, sorted order, sorted copies (cell
+//                walk: the elements and bonds beside it)
 //   k_list_build list mode: Verlet lists of the rebuilding replicas' tiles
-//   k_forces     one launch with three workgroup roles: LJ cell tiles
-//                (LDS-staged neighbours, lists or the 3x3 cell walk), CST
-//                elements and harmonic bonds (corner forces into a buffer in
-//                gather order, no atomics); each tile then gives its centre
-//                particles that have no element or bond corners their second
-//                half-kick, and the first half-kick, drift and wrap of the
-//                next step (cell walk: binning of the new positions)
-//   k_kick       the node kick: the same for the particles with corners,
-//                their corner forces gathered through a per-particle CSR in
-//                a fixed order
+//   k_forces     LJ cell tiles (LDS-staged neighbours, lists or the 3x3 cell
+//                walk); each tile then gives its centre particles, with their
+//                corner forces gathered through a per-particle CSR in a fixed
+//                order, their second half-kick, and the first half-kick,
+//                drift and wrap of the next step (cell walk: binning of the
+//                new positions)
+//   k_kick       the node kick: the same for replicas without pair forces
+//                (no tiles)
 // and at the end of a run the second half-kick only, then the observables.
 // Energies, virials and the kinetic energy are per-workgroup FP64 partials
 // summed in a fixed order (k_bin / k_sort level 1, k_forces level 2).
@@ -199,39 +200,40 @@ __device__ __forceinline__ void obs_slice(int b, int e, int c, int nc, int &lo, 
 __device__ void obs_chunk(const ObsArgs &o, int r, int c, double *red) {
     const int32_t *g = o.rng + 8 * r;
     const int tid = threadIdx.x;
+    // the slices of the partials: kinetic energy of a query (k_ke, over the
+    // kick spans) or of the particles the node kick integrated, tiles (U and
+    // W; kinetic energy of the particles the pair pass integrated), elements,
+    // bonds
+    const int kb = o.ke_kick ? g[0] : o.nrng[2 * r], ke = o.ke_kick ? g[1] : o.nrng[2 * r + 1];
+    int l0, h0, l1, h1, l2, h2, l3, h3;
+    obs_slice(kb, ke, c, o.nchunk, l0, h0);
+    obs_slice(g[2], g[3], c, o.nchunk, l1, h1);
+    obs_slice(g[4], g[5], c, o.nchunk, l2, h2);
+    obs_slice(g[6], g[7], c, o.nchunk, l3, h3);
+    const double2 *kin = reinterpret_cast<const double2 *>(o.ke_kick ? o.ke_part : o.ke_node);
+    const double2 *lj = reinterpret_cast<const double2 *>(o.lj_part);
+    const double2 *kt = reinterpret_cast<const double2 *>(o.ke_tile);
+    const double2 *fea = reinterpret_cast<const double2 *>(o.fea_part);
+    const double2 *bond = reinterpret_cast<const double2 *>(o.bond_part);
+    const double2 zero = make_double2(0.0, 0.0);
     double v[kObsRaw] = {0, 0, 0, 0, 0, 0, 0, 0};
-    int lo, hi;
-    if (o.ke_kick) {  // a query: the partials of k_ke over the kick spans
-        obs_slice(g[0], g[1], c, o.nchunk, lo, hi);
-        for (int k = lo + tid; k < hi; k += 256) {
-            v[0] += o.ke_part[2 * k];
-            v[1] = fmax(v[1], o.ke_part[2 * k + 1]);
-        }
-    } else {  // a step: the particles the node kick integrated
-        obs_slice(o.nrng[2 * r], o.nrng[2 * r + 1], c, o.nchunk, lo, hi);
-        for (int k = lo + tid; k < hi; k += 256) {
-            v[0] += o.ke_node[2 * k];
-            v[1] = fmax(v[1], o.ke_node[2 * k + 1]);
-        }
-    }
-    obs_slice(g[2], g[3], c, o.nchunk, lo, hi);
-    for (int k = lo + tid; k < hi; k += 256) {
-        v[2] += o.lj_part[2 * k];
-        v[3] += o.lj_part[2 * k + 1];
-        if (!o.ke_kick) {  // and those the pair pass integrated, per tile
-            v[0] += o.ke_tile[2 * k];
-            v[1] = fmax(v[1], o.ke_tile[2 * k + 1]);
-        }
-    }
-    obs_slice(g[4], g[5], c, o.nchunk, lo, hi);
-    for (int k = lo + tid; k < hi; k += 256) {
-        v[4] += o.fea_part[2 * k];
-        v[5] += o.fea_part[2 * k + 1];
-    }
-    obs_slice(g[6], g[7], c, o.nchunk, lo, hi);
-    for (int k = lo + tid; k < hi; k += 256) {
-        v[6] += o.bond_part[2 * k];
-        v[7] += o.bond_part[2 * k + 1];
+    // one entry of each per lane and pass, all loads in flight together (a
+    // loop per kind waits out its own; most slices are shorter than 256)
+    const int most = max(max(h0 - l0, h1 - l1), max(h2 - l2, h3 - l3));
+    for (int i = tid; i < ((most + 255) & ~255); i += 256) {
+        const double2 k0 = l0 + i < h0 ? kin[l0 + i] : zero;
+        const double2 u1 = l1 + i < h1 ? lj[l1 + i] : zero;
+        const double2 k1 = l1 + i < h1 && !o.ke_kick ? kt[l1 + i] : zero;
+        const double2 u2 = l2 + i < h2 ? fea[l2 + i] : zero;
+        const double2 u3 = l3 + i < h3 ? bond[l3 + i] : zero;
+        v[0] += k0.x + k1.x;
+        v[1] = fmax(v[1], fmax(k0.y, k1.y));
+        v[2] += u1.x;
+        v[3] += u1.y;
+        v[4] += u2.x;
+        v[5] += u2.y;
+        v[6] += u3.x;
+        v[7] += u3.y;
     }
     // the chunk's seven sums and its max v^2: each wavefront's in a fixed
     // butterfly, then the four wavefronts in order (one exchange through
@@ -255,11 +257,12 @@ __device__ void obs_chunk(const ObsArgs &o, int r, int c, double *red) {
     __syncthreads();  // red is free again
 }
 
-// The level-1 jobs (replica, chunk) of one step, spread over a kernel's
-// workgroups (256 threads each; uniform per workgroup).
-__device__ void obs_level1(const ObsArgs &o, double *red) {
+// The level-1 jobs (replica, chunk) of one step, spread over nb workgroups of
+// a kernel, of which this is number b (256 threads each; uniform per
+// workgroup).
+__device__ void obs_level1(const ObsArgs &o, int b, int nb, double *red) {
     const int njob = o.nrep * o.nchunk;
-    for (int q = blockIdx.x; q < njob; q += gridDim.x) obs_chunk(o, q / o.nchunk, q % o.nchunk, red);
+    for (int q = b; q < njob; q += nb) obs_chunk(o, q / o.nchunk, q % o.nchunk, red);
 }
 
 // Level 2 for replica r, one wavefront (all lanes): the step's totals from
@@ -371,10 +374,8 @@ __device__ __forceinline__ void kick_particle(const RepDesc &R, float ax, float 
 // ---------------------------------------------------------------------------
 // k_kick: integrator + binning (femmd2D/src/integrator.cpp:100-135,
 // femmd2D/src/nnCuda.cu:69-82 re-designed).  One workgroup covers one span
-// of one replica: particles [begin, end) (all particles: the first
-// half-kick of a run; the replica's [pg, p1): the node kick, of the
-// particles with element or bond corners, which the force pass does not
-// kick).
+// of one replica: particles [begin, end) (the first half-kick of a run, and
+// the node kick of the replicas without pair forces, which have no tiles).
 //   kKick2: second half-kick of the previous step (kinetic-energy and max
 //           v^2 partials of the workgroup with kEnergy)
 //   kDrift: first half-kick, drift, wrap; bin (cell walk every step) or
@@ -672,10 +673,176 @@ __global__ __launch_bounds__(1024) void k_decide(DecideArgs d) {
     }
 }
 
-__global__ __launch_bounds__(kKickThreads) void k_bin(KickArgs a) {
+// Span b of the elements or bonds (n of them; one replica: no load).
+__device__ __forceinline__ Span elem_span(const ElemArgs &a, const Span *spans, int b, int n) {
+    if (a.nrep != 1) return spans[b];
+    return Span{0, b * kElemThreads, min((b + 1) * kElemThreads, n), 0};
+}
+
+// CST element forces (femmd2D/src/interactions.cpp:532-689), re-derived in
+// displacement form: with U = Ds - Dm and G = U Bm = F - I, every term of P
+// is O(|G|), so FP32 keeps relative accuracy at small strain.  Corner forces
+// go to their entries of the per-particle gather order, cf[gpos[3e + k]]; no
+// atomics.
+__device__ void elem_block(const ElemArgs &a, int b, double *red) {
+    const Span sp = elem_span(a, a.espans, b, a.ntri);
+    const RepDesc R = a.reps[sp.rep];
+    double U = 0.0, Wv = 0.0;
+    for (int e = sp.begin + (int)threadIdx.x; e < sp.end; e += blockDim.x) {
+        const int n0 = a.t0[e], n1 = a.t1[e], n2 = a.t2[e];
+        const int g0 = a.gpos[3 * e], g1 = a.gpos[3 * e + 1], g2 = a.gpos[3 * e + 2];
+        const float x0 = a.x[n0], y0 = a.y[n0];
+        const float x1 = a.x[n1], y1 = a.y[n1];
+        const float x2 = a.x[n2], y2 = a.y[n2];
+        // half-box unwrap of nodes 1, 2 against node 0
+        // (femmd2D/src/interactions.cpp:554-568): shifts s1, s2 in {-1,0,1}
+        const float Lx = R.Lx, Ly = R.Ly, hLx = R.hLx, hLy = R.hLy;
+        const float dx01 = x0 - x1, dx02 = x0 - x2, dy01 = y0 - y1, dy02 = y0 - y2;
+        const int s1x = (dx01 > hLx) - (dx01 < -hLx);
+        const int s2x = (dx02 > hLx) - (dx02 < -hLx);
+        const int s1y = (dy01 > hLy) - (dy01 < -hLy);
+        const int s2y = (dy02 > hLy) - (dy02 < -hLy);
+        const float Ds00 = shifted_diff(x0, x2, -s2x, Lx);
+        const float Ds10 = shifted_diff(y0, y2, -s2y, Ly);
+        const float Ds01 = shifted_diff(x1, x2, s1x - s2x, Lx);
+        const float Ds11 = shifted_diff(y1, y2, s1y - s2y, Ly);
+        const float4 Dm = a.dmbm[2 * e];
+        const float4 B = a.dmbm[2 * e + 1];
+        const float2 alm = a.alm[e];
+        const float al = alm.x, am = alm.y;
+        // Dm = {Dm00, Dm01, Dm10, Dm11}; B = {B00, B01, B10, B11}
+        const float U00 = Ds00 - Dm.x, U01 = Ds01 - Dm.y;
+        const float U10 = Ds10 - Dm.z, U11 = Ds11 - Dm.w;
+        const float G00 = U00 * B.x + U01 * B.z;
+        const float G10 = U10 * B.x + U11 * B.z;
+        const float G01 = U00 * B.y + U01 * B.w;
+        const float G11 = U10 * B.y + U11 * B.w;
+        const float F00 = 1.0f + G00, F11 = 1.0f + G11;
+        float P00, P01, P10, P11, ue;
+        const float trG = G00 + G11;
+        const float detG = G00 * G11 - G01 * G10;
+        const float tJ = trG + detG;  // J - 1
+        if (!(tJ > -1.0f)) atomicOr(a.err, 4u);  // FM_DEV_INVERTED
+        if (a.model == 0) {
+            // Neo-Hookean: P = [mu (J F - cof F) + lambda lnJ cof F] / J
+            const float lJ = log1pf(tJ);
+            const float iJ = 1.0f / (1.0f + tJ);
+            const float A00 = (G00 - G11) + tJ * F00;
+            const float A01 = G01 + tJ * G01 + G10;
+            const float A10 = G10 + tJ * G10 + G01;
+            const float A11 = (G11 - G00) + tJ * F11;
+            const float ll = al * lJ;
+            P00 = (am * A00 + ll * F11) * iJ;
+            P01 = (am * A01 - ll * G10) * iJ;
+            P10 = (am * A10 - ll * G01) * iJ;
+            P11 = (am * A11 + ll * F00) * iJ;
+            const float g2 = G00 * G00 + G01 * G01 + G10 * G10 + G11 * G11;
+            ue = am * (trG - lJ) + 0.5f * am * g2 + 0.5f * al * lJ * lJ;
+        } else {
+            // SVK: E = (G + G^T + G^T G)/2, S = 2 mu E + lambda tr(E) I, P = F S
+            const float E00 = G00 + 0.5f * (G00 * G00 + G10 * G10);
+            const float E11 = G11 + 0.5f * (G01 * G01 + G11 * G11);
+            const float E01 = 0.5f * (G01 + G10) + 0.5f * (G00 * G01 + G10 * G11);
+            const float tr = E00 + E11;
+            const float S00 = 2.0f * am * E00 + al * tr;
+            const float S11 = 2.0f * am * E11 + al * tr;
+            const float S01 = 2.0f * am * E01;
+            P00 = F00 * S00 + G01 * S01;
+            P01 = F00 * S01 + G01 * S11;
+            P10 = G10 * S00 + F11 * S01;
+            P11 = G10 * S01 + F11 * S11;
+            ue = am * (E00 * E00 + E11 * E11 + 2.0f * E01 * E01) + 0.5f * al * tr * tr;
+        }
+        // H = -P' Bm^T (P' = A0 P, A0 folded into al, am)
+        const float f0x = -(P00 * B.x + P01 * B.y);
+        const float f0y = -(P10 * B.x + P11 * B.y);
+        const float f1x = -(P00 * B.z + P01 * B.w);
+        const float f1y = -(P10 * B.z + P11 * B.w);
+        a.cf[g0] = make_float2(f0x, f0y);
+        a.cf[g1] = make_float2(f1x, f1y);
+        a.cf[g2] = make_float2(-f0x - f1x, -f0y - f1y);
+        U += (double)ue;
+        Wv += (double)(f0x * Ds00 + f0y * Ds10) + (double)(f1x * Ds01 + f1y * Ds11);
+    }
+    block_sum2(U, Wv, red);
+    if (threadIdx.x == 0) {
+        a.fea_part[2 * b] = U;
+        a.fea_part[2 * b + 1] = Wv;
+    }
+}
+
+// Harmonic bonds (femmd2D/src/interactions.cpp:143-173, per-bond k, r0).
+__device__ void bond_block(const ElemArgs &a, int b, double *red) {
+    const Span sp = elem_span(a, a.bspans, b, a.nbond);
+    const RepDesc R = a.reps[sp.rep];
+    double U = 0.0, Wv = 0.0;
+    for (int l = sp.begin + (int)threadIdx.x; l < sp.end; l += blockDim.x) {
+        const int i = a.bi[l], j = a.bj[l];
+        const float xi = a.x[i], yi = a.y[i], xj = a.x[j], yj = a.y[j];
+        float dx = xi - xj, dy = yi - yj;
+        const int sx = (dx >= R.hLx) - (dx < -R.hLx);
+        const int sy = (dy >= R.hLy) - (dy < -R.hLy);
+        dx = shifted_diff(xi, xj, -sx, R.Lx);
+        dy = shifted_diff(yi, yj, -sy, R.Ly);
+        // r - r0 = (r^2 - r0^2) / (r + r0) with r^2 - r0^2 formed from
+        // error-free products and sums, so a bond near rest keeps its
+        // relative accuracy (r - r0 in FP32 would cancel to nothing)
+        const float p1 = dx * dx, e1 = __builtin_fmaf(dx, dx, -p1);
+        const float p2 = dy * dy, e2 = __builtin_fmaf(dy, dy, -p2);
+        const float r2 = p1 + p2;
+        const float bb = r2 - p1;
+        const float t2 = (p1 - (r2 - bb)) + (p2 - bb);
+        const float r0 = a.br0[l];
+        const float h0 = r0 * r0, l0 = __builtin_fmaf(r0, r0, -h0);
+        const float q = (r2 - h0) + ((t2 + e1 + e2) - l0);
+        const float r = sqrtf(r2);
+        const float k = a.bk[l];
+        const float d = q / (r + r0);
+        const float kdr = -k * d / r;
+        const float fx = kdr * dx, fy = kdr * dy;
+        a.cf[a.gpos[a.cf_bond0 + 2 * l]] = make_float2(fx, fy);
+        a.cf[a.gpos[a.cf_bond0 + 2 * l + 1]] = make_float2(-fx, -fy);
+        U += 0.5 * (double)(k * d * d);
+        Wv += (double)(kdr * r2);
+    }
+    block_sum2(U, Wv, red);
+    if (threadIdx.x == 0) {
+        a.bond_part[2 * b] = U;
+        a.bond_part[2 * b + 1] = Wv;
+    }
+}
+
+// Workgroup b of the elements and bonds (256 threads; red: 2 per wavefront).
+// Run beside the step's first kernel, which most steps leave idle, so that
+// the force pass finds every corner force complete and kicks the particles
+// with corners itself: before, they shared the force pass's launch and a
+// second kernel integrated those particles (866,616 elements, 1.11 million
+// particles, us per step: 52.5 force pass + 14.5 node kick + 6 binning ->
+// 38.2 + 21.4; 4,367 particles: 10.9 + 4.4 + 5.5 -> 8.5 + 4.5).  Bound by
+// HBM at that size: 100 bytes an element, 4.1 TB/s.
+__device__ void elem_role(const ElemArgs &a, int b, double *red) {
+    if (b < a.nespans) elem_block(a, b, red);
+    else if (b < a.nespans + a.nbspans) bond_block(a, b - a.nespans, red);
+}
+
+// The same alone (force passes outside a step).
+__global__ __launch_bounds__(kElemThreads) void k_elems(ElemArgs a) {
+    __shared__ double red[2 * (kElemThreads / 64)];
+    elem_role(a, blockIdx.x, red);
+}
+
+__global__ __launch_bounds__(kKickThreads) void k_bin(KickArgs a, ElemArgs el) {
   __shared__ double ored[kObsRed];
+  // the step's element and bond forces, by workgroups of their own: they
+  // need the positions only, and most steps bin nothing
+  const int ne = el.nespans + el.nbspans;
+  if ((int)blockIdx.x < ne) {
+      elem_role(el, blockIdx.x, ored);
+      return;
+  }
+  const int wb = (int)blockIdx.x - ne, nwb = (int)gridDim.x - ne;
   // the previous step's observables, level 1 (before any early exit)
-  if (a.obs_l1) obs_level1(a.obs, ored);
+  if (a.obs_l1) obs_level1(a.obs, wb, nwb, ored);
   int last_rep = -1, flag = 1;
   if (a.ctl && !a.fspan && a.one_rep) {
       // a single replica: the decision comes first, from the replica's
@@ -683,7 +850,7 @@ __global__ __launch_bounds__(kKickThreads) void k_bin(KickArgs a) {
       // before them), so that a step without a rebuild leaves at once
       const RepDesc &R0 = a.reps[0];
       flag = list_disp(a.dmax, a.ctl, 0, R0) > 0.5f * R0.skin;
-      if (blockIdx.x == 0 && threadIdx.x == 0) {  // as list_decide records it
+      if (wb == 0 && threadIdx.x == 0) {  // as list_decide records it
           a.ctl->flag = flag;
           if (flag) {
               a.ctl->nbuild += 1u;
@@ -696,7 +863,7 @@ __global__ __launch_bounds__(kKickThreads) void k_bin(KickArgs a) {
   }
   // decided (batches): only the rebuilding replicas' spans, listed
   const int nsp = a.fspan ? *a.nfs : a.nspans;
-  for (int b = blockIdx.x; b < nsp; b += gridDim.x) {
+  for (int b = wb; b < nsp; b += nwb) {
     const Span sp = a.spans[a.fspan ? a.fspan[b] : b];
     const RepDesc R = a.reps[sp.rep];
     if (a.ctl && !a.fspan) {  // list mode: bin only the replicas that rebuild this step
@@ -706,7 +873,7 @@ __global__ __launch_bounds__(kKickThreads) void k_bin(KickArgs a) {
         }
         if (!flag) {
             // on to this workgroup's first span of the next replica
-            const int e = R.ks0 + R.nks, g = (int)gridDim.x;
+            const int e = R.ks0 + R.nks, g = nwb;
             if (e > b + g) b += ((e - b - 1) / g) * g;
             continue;
         }
@@ -770,7 +937,7 @@ __device__ __forceinline__ int rep_of_cell(const ScanArgs &a, int b, int c) {
     return lo;
 }
 
-__global__ __launch_bounds__(kSortCells) void k_sort(ScanArgs a) {
+__global__ __launch_bounds__(kSortCells) void k_sort(ScanArgs a, ElemArgs el) {
     __shared__ int s_ex[kSortCells + 1];  // local exclusive prefix of the counts
     __shared__ int s_st[kSortCells];      // cell starts
     __shared__ int s_lim[kSortCells];     // end of each cell's replica range
@@ -780,9 +947,14 @@ __global__ __launch_bounds__(kSortCells) void k_sort(ScanArgs a) {
     __shared__ int s_ids[kSortIds];       // the block's slot entries' caller indices, cell order
     __shared__ uint8_t s_cl[kSortIds];    // their cell (local index)
     __shared__ double s_ored[kObsRed];
-    // (cell walk) the previous step's observables, level 1, before the
+    // (cell walk) the step's element and bond forces, by the workgroups past
+    // the sort's, and the previous step's observables, level 1, before the
     // ticket: no workgroup waits on one that has not taken its ticket
-    if (a.obs_l1) obs_level1(a.obs, s_ored);
+    if ((int)blockIdx.x >= a.nsort) {
+        elem_role(el, (int)blockIdx.x - a.nsort, s_ored);
+        return;
+    }
+    if (a.obs_l1) obs_level1(a.obs, blockIdx.x, a.nsort, s_ored);
     if (a.any && !*a.any) return;  // list mode, no replica rebuilds (uniform)
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
     // listed (gated batches): workgroups beyond the listed blocks leave at
@@ -1028,21 +1200,34 @@ struct TileKick {
 // position (x, y) (the same bits as x[id]) and velocity (vx, vy) with pair
 // force (fxs, fys).
 // kKick 1: second half-kick only (the closing kick of a run); 2: second and
-// first half-kick, drift and wrap.  A particle with element or bond corners
-// is left to the node kick, which adds its gathered corner forces: its pair
-// force is stored for it (and every particle's in mode 0 and 1, for the next
-// run's first half-kick).  Returns the cell of the drifted position (cell
-// walk, mode 2), -1 when there is none to bin.
+// first half-kick, drift and wrap.  The corner forces of a particle with
+// element or bond corners are gathered and added in their order; the pair
+// force is stored in modes 0 and 1 (for queries and the next run's first
+// half-kick, which adds the corners itself).  Returns the cell of the drifted
+// position (cell walk, mode 2), -1 when there is none to bin.
 template <int kKick, bool kList, bool kEnergy>
 __device__ __forceinline__ int tile_kick(const ForceArgs &a, const RepDesc &R, int id, int p,
                                          float x, float y, float vx, float vy, float fxs,
                                          float fys, TileKick &tk) {
-    const bool node = id >= R.pg;  // (internal order: these come last)
-    if (kKick != 2 || node) {
+    if (kKick != 2) {
         a.fx[id] = fxs;
         a.fy[id] = fys;
     }
-    if (kKick == 0 || node) return -1;
+    if (kKick == 0) return -1;
+    if (id >= R.pg) {  // (internal order: the particles with corners come last)
+        const int e0 = a.goff[id], e1 = a.goff[id + 1];
+        for (int e = e0; e < e1; e += 4) {  // four in flight, added in order
+            float2 c[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) c[u] = a.el.cf[min(e + u, e1 - 1)];
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (e + u < e1) {
+                    fxs += c[u].x;
+                    fys += c[u].y;
+                }
+        }
+    }
     const float im = R.im_uniform > 0.0f ? R.im_uniform : a.inv_m[id];
     const float ax = fxs * im, ay = fys * im;
     float dxp = 0.0f, dyp = 0.0f, vv = 0.0f;
@@ -2196,138 +2381,6 @@ __device__ void list_tile_pass(const ForceArgs &a, int tile, PairEntry *pt, floa
 #undef FM_LPB
 }
 
-// CST element forces (femmd2D/src/interactions.cpp:532-689), re-derived in
-// displacement form: with U = Ds - Dm and G = U Bm = F - I, every term of P
-// is O(|G|), so FP32 keeps relative accuracy at small strain.  Corner forces
-// go to their entries of the per-particle gather order, cf[gpos[3e + k]]; no
-// atomics.
-__device__ void elem_block(const ForceArgs &a, int b, double *red) {
-    const Span sp = a.espans[b];
-    const RepDesc R = a.reps[sp.rep];
-    double U = 0.0, Wv = 0.0;
-    for (int e = sp.begin + (int)threadIdx.x; e < sp.end; e += blockDim.x) {
-        const int n0 = a.t0[e], n1 = a.t1[e], n2 = a.t2[e];
-        const float x0 = a.x[n0], y0 = a.y[n0];
-        const float x1 = a.x[n1], y1 = a.y[n1];
-        const float x2 = a.x[n2], y2 = a.y[n2];
-        // half-box unwrap of nodes 1, 2 against node 0
-        // (femmd2D/src/interactions.cpp:554-568): shifts s1, s2 in {-1,0,1}
-        const float Lx = R.Lx, Ly = R.Ly, hLx = R.hLx, hLy = R.hLy;
-        const float dx01 = x0 - x1, dx02 = x0 - x2, dy01 = y0 - y1, dy02 = y0 - y2;
-        const int s1x = (dx01 > hLx) - (dx01 < -hLx);
-        const int s2x = (dx02 > hLx) - (dx02 < -hLx);
-        const int s1y = (dy01 > hLy) - (dy01 < -hLy);
-        const int s2y = (dy02 > hLy) - (dy02 < -hLy);
-        const float Ds00 = shifted_diff(x0, x2, -s2x, Lx);
-        const float Ds10 = shifted_diff(y0, y2, -s2y, Ly);
-        const float Ds01 = shifted_diff(x1, x2, s1x - s2x, Lx);
-        const float Ds11 = shifted_diff(y1, y2, s1y - s2y, Ly);
-        const float4 Dm = a.dmbm[2 * e];
-        const float4 B = a.dmbm[2 * e + 1];
-        const float2 alm = a.alm[e];
-        const float al = alm.x, am = alm.y;
-        // Dm = {Dm00, Dm01, Dm10, Dm11}; B = {B00, B01, B10, B11}
-        const float U00 = Ds00 - Dm.x, U01 = Ds01 - Dm.y;
-        const float U10 = Ds10 - Dm.z, U11 = Ds11 - Dm.w;
-        const float G00 = U00 * B.x + U01 * B.z;
-        const float G10 = U10 * B.x + U11 * B.z;
-        const float G01 = U00 * B.y + U01 * B.w;
-        const float G11 = U10 * B.y + U11 * B.w;
-        const float F00 = 1.0f + G00, F11 = 1.0f + G11;
-        float P00, P01, P10, P11, ue;
-        const float trG = G00 + G11;
-        const float detG = G00 * G11 - G01 * G10;
-        const float tJ = trG + detG;  // J - 1
-        if (!(tJ > -1.0f)) atomicOr(a.err, 4u);  // FM_DEV_INVERTED
-        if (a.model == 0) {
-            // Neo-Hookean: P = [mu (J F - cof F) + lambda lnJ cof F] / J
-            const float lJ = log1pf(tJ);
-            const float iJ = 1.0f / (1.0f + tJ);
-            const float A00 = (G00 - G11) + tJ * F00;
-            const float A01 = G01 + tJ * G01 + G10;
-            const float A10 = G10 + tJ * G10 + G01;
-            const float A11 = (G11 - G00) + tJ * F11;
-            const float ll = al * lJ;
-            P00 = (am * A00 + ll * F11) * iJ;
-            P01 = (am * A01 - ll * G10) * iJ;
-            P10 = (am * A10 - ll * G01) * iJ;
-            P11 = (am * A11 + ll * F00) * iJ;
-            const float g2 = G00 * G00 + G01 * G01 + G10 * G10 + G11 * G11;
-            ue = am * (trG - lJ) + 0.5f * am * g2 + 0.5f * al * lJ * lJ;
-        } else {
-            // SVK: E = (G + G^T + G^T G)/2, S = 2 mu E + lambda tr(E) I, P = F S
-            const float E00 = G00 + 0.5f * (G00 * G00 + G10 * G10);
-            const float E11 = G11 + 0.5f * (G01 * G01 + G11 * G11);
-            const float E01 = 0.5f * (G01 + G10) + 0.5f * (G00 * G01 + G10 * G11);
-            const float tr = E00 + E11;
-            const float S00 = 2.0f * am * E00 + al * tr;
-            const float S11 = 2.0f * am * E11 + al * tr;
-            const float S01 = 2.0f * am * E01;
-            P00 = F00 * S00 + G01 * S01;
-            P01 = F00 * S01 + G01 * S11;
-            P10 = G10 * S00 + F11 * S01;
-            P11 = G10 * S01 + F11 * S11;
-            ue = am * (E00 * E00 + E11 * E11 + 2.0f * E01 * E01) + 0.5f * al * tr * tr;
-        }
-        // H = -P' Bm^T (P' = A0 P, A0 folded into al, am)
-        const float f0x = -(P00 * B.x + P01 * B.y);
-        const float f0y = -(P10 * B.x + P11 * B.y);
-        const float f1x = -(P00 * B.z + P01 * B.w);
-        const float f1y = -(P10 * B.z + P11 * B.w);
-        a.cf[a.gpos[3 * e]] = make_float2(f0x, f0y);
-        a.cf[a.gpos[3 * e + 1]] = make_float2(f1x, f1y);
-        a.cf[a.gpos[3 * e + 2]] = make_float2(-f0x - f1x, -f0y - f1y);
-        U += (double)ue;
-        Wv += (double)(f0x * Ds00 + f0y * Ds10) + (double)(f1x * Ds01 + f1y * Ds11);
-    }
-    block_sum2(U, Wv, red);
-    if (threadIdx.x == 0) {
-        a.fea_part[2 * b] = U;
-        a.fea_part[2 * b + 1] = Wv;
-    }
-}
-
-// Harmonic bonds (femmd2D/src/interactions.cpp:143-173, per-bond k, r0).
-__device__ void bond_block(const ForceArgs &a, int b, double *red) {
-    const Span sp = a.bspans[b];
-    const RepDesc R = a.reps[sp.rep];
-    double U = 0.0, Wv = 0.0;
-    for (int l = sp.begin + (int)threadIdx.x; l < sp.end; l += blockDim.x) {
-        const int i = a.bi[l], j = a.bj[l];
-        const float xi = a.x[i], yi = a.y[i], xj = a.x[j], yj = a.y[j];
-        float dx = xi - xj, dy = yi - yj;
-        const int sx = (dx >= R.hLx) - (dx < -R.hLx);
-        const int sy = (dy >= R.hLy) - (dy < -R.hLy);
-        dx = shifted_diff(xi, xj, -sx, R.Lx);
-        dy = shifted_diff(yi, yj, -sy, R.Ly);
-        // r - r0 = (r^2 - r0^2) / (r + r0) with r^2 - r0^2 formed from
-        // error-free products and sums, so a bond near rest keeps its
-        // relative accuracy (r - r0 in FP32 would cancel to nothing)
-        const float p1 = dx * dx, e1 = __builtin_fmaf(dx, dx, -p1);
-        const float p2 = dy * dy, e2 = __builtin_fmaf(dy, dy, -p2);
-        const float r2 = p1 + p2;
-        const float bb = r2 - p1;
-        const float t2 = (p1 - (r2 - bb)) + (p2 - bb);
-        const float r0 = a.br0[l];
-        const float h0 = r0 * r0, l0 = __builtin_fmaf(r0, r0, -h0);
-        const float q = (r2 - h0) + ((t2 + e1 + e2) - l0);
-        const float r = sqrtf(r2);
-        const float k = a.bk[l];
-        const float d = q / (r + r0);
-        const float kdr = -k * d / r;
-        const float fx = kdr * dx, fy = kdr * dy;
-        a.cf[a.gpos[a.cf_bond0 + 2 * l]] = make_float2(fx, fy);
-        a.cf[a.gpos[a.cf_bond0 + 2 * l + 1]] = make_float2(-fx, -fy);
-        U += 0.5 * (double)(k * d * d);
-        Wv += (double)(kdr * r2);
-    }
-    block_sum2(U, Wv, red);
-    if (threadIdx.x == 0) {
-        a.bond_part[2 * b] = U;
-        a.bond_part[2 * b + 1] = Wv;
-    }
-}
-
 // Bookkeeping workgroups of a force pass (per replica two jobs, a wavefront
 // each): apart from the tiles, whose path they would lengthen.
 __host__ __device__ inline int forces_book(const ForceArgs &a) {
@@ -2355,11 +2408,11 @@ __device__ void step_book(const ForceArgs &a, int b, int nb) {
     }
 }
 
-// The force pass (femmd2D/src/interactions.cpp:83-109).  kKick: 0 forces
-// only; 1 forces and the closing second half-kick of a run; 2 forces, the
-// second half-kick of this step and the first half-kick, drift and wrap of
-// the next (femmd2D/src/integrator.cpp:8-29), for every particle without
-// element or bond corners (tile_kick).
+// The force pass (femmd2D/src/interactions.cpp:83-109; the element and bond
+// forces came before it, elem_role).  kKick: 0 forces only; 1 forces and the
+// closing second half-kick of a run; 2 forces, the second half-kick of this
+// step and the first half-kick, drift and wrap of the next
+// (femmd2D/src/integrator.cpp:8-29), for every particle (tile_kick).
 // Wavefronts per SIMD: the list pass 6 (5 with a type table), where what it
 // keeps in flight needs no spilled register (1.14 million particles: 38 us;
 // 39 at 7, 45 at 8 with 14 spilled, 42 at 5; 30,011 particles of six types:
@@ -2374,20 +2427,14 @@ k_forces(ForceArgs a) {
     __shared__ int s_cstart[kMaxSlots];
     __shared__ int s_off[kMaxSlots + 1];
     __shared__ PairEntry s_pt[kMaxPairTypes * kMaxPairTypes];
-    __shared__ double s_red[2 * 4];
     int b = blockIdx.x;
-    // element and bond workgroups first, then the bookkeeping of the step (a
-    // whole number of rounds over the 8 XCDs together, so each XCD's tiles
-    // still form one contiguous band), then the tiles: the kernel's tail is
-    // made of the uniform tile work
+    // the bookkeeping of the step first (a whole number of rounds over the 8
+    // XCDs, so each XCD's tiles form one contiguous band), then the tiles
     {
-        const int ne = a.nespans + a.nbspans;
         const int nb = forces_book(a);
-        const int nfirst = (ne + nb + 7) & ~7;
+        const int nfirst = (nb + 7) & ~7;
         if (b < nfirst) {
-            if (b < a.nespans) elem_block(a, b, s_red);
-            else if (b < ne) bond_block(a, b - a.nespans, s_red);
-            else if (b < ne + nb) step_book<kList, kDebug>(a, b - ne, nb);
+            if (b < nb) step_book<kList, kDebug>(a, b, nb);
             return;
         }
         b -= nfirst;
@@ -2410,15 +2457,15 @@ k_forces(ForceArgs a) {
         L.cstart = s_cstart;
         L.off = s_off;
         L.pt = s_pt;
-        L.red = s_red;
+        L.red = nullptr;
         pair_tile<kSigma, kTypes, kDebug, kEnergy, kKick>(a, xcd_remap(b, a.ntiles), L);
     }
 }
 
-// Workgroups of one force pass: element and bond spans and the bookkeeping
-// (rounded up to a multiple of 8), then the tiles.
+// Workgroups of one force pass: the bookkeeping (rounded up to a multiple of
+// 8), then the tiles.
 __host__ __device__ inline int forces_grid(const ForceArgs &a) {
-    return ((a.nespans + a.nbspans + forces_book(a) + 7) & ~7) + a.ntiles;
+    return ((forces_book(a) + 7) & ~7) + a.ntiles;
 }
 
 // Total force per particle (pair + gathered corners), internal order.
@@ -2448,7 +2495,7 @@ __global__ __launch_bounds__(256) void k_total_force(int n, const float *fx,
 // level 2 (one thread per replica); accumulate: add them to the running sums.
 __global__ __launch_bounds__(256) void k_observe_l1(ObsArgs o) {
     __shared__ double red[kObsRed];
-    obs_level1(o, red);
+    obs_level1(o, blockIdx.x, gridDim.x, red);
 }
 __global__ __launch_bounds__(256) void k_observe_l2(ObsArgs o, int accumulate) {
     const int r = blockIdx.x * 4 + (int)(threadIdx.x >> 6);  // one wavefront per replica
@@ -2769,10 +2816,10 @@ __device__ void adj_list_tile(const AdjArgs &A, int tile, PairLds &L, float2 *lp
 // proportional to E at fixed nu).
 __device__ void adj_elem_block(const AdjArgs &A, int b, double *red) {
     const ForceArgs &a = A.f;
-    const Span sp = a.espans[b];
+    const Span sp = a.el.espans[b];
     const RepDesc R = a.reps[sp.rep];
     for (int e = sp.begin + (int)threadIdx.x; e < sp.end; e += blockDim.x) {
-        const int n0 = a.t0[e], n1 = a.t1[e], n2 = a.t2[e];
+        const int n0 = a.el.t0[e], n1 = a.el.t1[e], n2 = a.el.t2[e];
         const float x0 = a.x[n0], y0 = a.y[n0];
         const float x1 = a.x[n1], y1 = a.y[n1];
         const float x2 = a.x[n2], y2 = a.y[n2];
@@ -2786,9 +2833,9 @@ __device__ void adj_elem_block(const AdjArgs &A, int b, double *red) {
         const float Ds10 = shifted_diff(y0, y2, -s2y, Ly);
         const float Ds01 = shifted_diff(x1, x2, s1x - s2x, Lx);
         const float Ds11 = shifted_diff(y1, y2, s1y - s2y, Ly);
-        const float4 Dm = a.dmbm[2 * e];
-        const float4 B = a.dmbm[2 * e + 1];
-        const float2 alm = a.alm[e];
+        const float4 Dm = a.el.dmbm[2 * e];
+        const float4 B = a.el.dmbm[2 * e + 1];
+        const float2 alm = a.el.alm[e];
         const float al = alm.x, am = alm.y;
         const float G00 = (Ds00 - Dm.x) * B.x + (Ds01 - Dm.y) * B.z;
         const float G10 = (Ds10 - Dm.z) * B.x + (Ds11 - Dm.w) * B.z;
@@ -2802,7 +2849,7 @@ __device__ void adj_elem_block(const AdjArgs &A, int b, double *red) {
         const float dF01 = d00 * B.y + d01 * B.w;
         const float dF11 = d10 * B.y + d11 * B.w;
         float P00, P01, P10, P11, Q00, Q01, Q10, Q11;
-        if (a.model == 0) {
+        if (a.el.model == 0) {
             const float tJ = (G00 + G11) + (G00 * G11 - G01 * G10);
             const float lJ = log1pf(tJ);
             const float iJ = 1.0f / (1.0f + tJ);
@@ -2870,10 +2917,10 @@ __device__ void adj_elem_block(const AdjArgs &A, int b, double *red) {
 // Bond part of J w: g = -k (r - r0) / r, g' = dg/ds = -k r0 / (2 r^3).
 __device__ void adj_bond_block(const AdjArgs &A, int b) {
     const ForceArgs &a = A.f;
-    const Span sp = a.bspans[b];
+    const Span sp = a.el.bspans[b];
     const RepDesc R = a.reps[sp.rep];
     for (int l = sp.begin + (int)threadIdx.x; l < sp.end; l += blockDim.x) {
-        const int i = a.bi[l], j = a.bj[l];
+        const int i = a.el.bi[l], j = a.el.bj[l];
         const float xi = a.x[i], yi = a.y[i], xj = a.x[j], yj = a.y[j];
         float dx = xi - xj, dy = yi - yj;
         const int sx = (dx >= R.hLx) - (dx < -R.hLx);
@@ -2882,15 +2929,15 @@ __device__ void adj_bond_block(const AdjArgs &A, int b) {
         dy = shifted_diff(yi, yj, -sy, R.Ly);
         const float r2 = dx * dx + dy * dy;
         const float r = sqrtf(r2);
-        const float k = a.bk[l], r0 = a.br0[l];
+        const float k = a.el.bk[l], r0 = a.el.br0[l];
         const float g = -k * (r - r0) / r;
         const float gp = -k * r0 / (2.0f * r2 * r);
         const float2 wi = A.w[i], wj = A.w[j];
         const float dwx = wi.x - wj.x, dwy = wi.y - wj.y;
         const float g2 = 2.0f * gp * (dx * dwx + dy * dwy);
         const float jx = g * dwx + g2 * dx, jy = g * dwy + g2 * dy;
-        A.cfa[a.cf_bond0 + 2 * l] = make_float2(jx, jy);
-        A.cfa[a.cf_bond0 + 2 * l + 1] = make_float2(-jx, -jy);
+        A.cfa[a.el.cf_bond0 + 2 * l] = make_float2(jx, jy);
+        A.cfa[a.el.cf_bond0 + 2 * l + 1] = make_float2(-jx, -jy);
     }
 }
 
@@ -2924,12 +2971,12 @@ __global__ __launch_bounds__(256) void k_adj_forces(AdjArgs A) {
         return;
     }
     b -= a.ntiles;
-    if (b < a.nespans) {
+    if (b < a.el.nespans) {
         adj_elem_block(A, b, s_red);
         return;
     }
-    b -= a.nespans;
-    if (b < a.nbspans) adj_bond_block(A, b);
+    b -= a.el.nespans;
+    if (b < a.el.nbspans) adj_bond_block(A, b);
 }
 
 __global__ __launch_bounds__(kKickThreads) void k_adj_kick(AdjKickArgs a) {
@@ -3235,7 +3282,7 @@ __global__ __launch_bounds__(256) void k_vel_scale(const int32_t *ids, int n, fl
 // ---------------------------------------------------------------------------
 hipError_t launch_adj_forces(bool sigma, bool list, int block, const AdjArgs &A, hipStream_t s) {
     const ForceArgs &a = A.f;
-    const int nblk = a.ntiles + a.nespans + a.nbspans;
+    const int nblk = a.ntiles + a.el.nespans + a.el.nbspans;
     if (nblk <= 0) return hipSuccess;
     if (list) {
         const size_t lds = (size_t)(a.lds_cap + 1) * (2 * sizeof(float2) + (sigma ? sizeof(float) : 0));
@@ -3290,8 +3337,8 @@ void arm_kernel_timer(hipEvent_t start, hipEvent_t stop) {
 
 hipError_t launch_kick(int mode, bool gather, bool energy, int nblk, const KickArgs &a,
                        hipStream_t s) {
-    // mode: 0 = bin only, 1 = kick + drift, 2 = final kick, 3 = both,
-    // 4 = kinetic-energy partials only; a.dmax set = list mode (the drift
+    // mode: 1 = kick + drift, 2 = final kick, 3 = both, 4 = kinetic-energy
+    // partials only; a.dmax set = list mode (the drift
     // measures the displacement since the list build instead of binning);
     // energy: the final-kick part writes the kinetic-energy partials
     if (nblk <= 0) return hipSuccess;
@@ -3307,12 +3354,6 @@ hipError_t launch_kick(int mode, bool gather, bool energy, int nblk, const KickA
         if (K2 && energy) FM_KICK1(K2, D, G, true); else FM_KICK1(K2, D, G, false); \
     } while (0)
     switch (mode) {
-        case 0:
-            // gated list-mode binning: a smaller grid-stride grid keeps the
-            // skipped steps cheap
-            if (a.ctl) g = dim3(std::min(nblk, kGatedBinGrid));
-            FM_GO(k_bin, g, b, 0, s, a);
-            break;
         case 4: FM_GO(k_ke, g, b, 0, s, a); break;
         case 1:
             if (gather) FM_KICK1(false, true, true, false); else FM_KICK1(false, true, false, false);
@@ -3329,9 +3370,24 @@ hipError_t launch_kick(int mode, bool gather, bool energy, int nblk, const KickA
     return hipGetLastError();
 }
 
-hipError_t launch_sort(const ScanArgs &a, hipStream_t s) {
+hipError_t launch_bin(const KickArgs &a, const ElemArgs &el, hipStream_t s) {
+    // gated list-mode binning: a smaller grid-stride grid keeps the skipped
+    // steps cheap
+    const int nbin = a.ctl ? std::min(a.nspans, kGatedBinGrid) : a.nspans;
+    FM_GO(k_bin, dim3(el.nespans + el.nbspans + nbin), dim3(kKickThreads), 0, s, a, el);
+    return hipGetLastError();
+}
+
+hipError_t launch_sort(const ScanArgs &a, const ElemArgs &el, hipStream_t s) {
     if (a.nsort <= 0) return hipSuccess;
-    FM_GO(k_sort, dim3(a.nsort), dim3(kSortCells), 0, s, a);
+    FM_GO(k_sort, dim3(a.nsort + el.nespans + el.nbspans), dim3(kSortCells), 0, s, a, el);
+    return hipGetLastError();
+}
+
+hipError_t launch_elems(const ElemArgs &el, hipStream_t s) {
+    const int n = el.nespans + el.nbspans;
+    if (n <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_elems, dim3(n), dim3(kElemThreads), 0, s, el);
     return hipGetLastError();
 }
 
@@ -3345,8 +3401,7 @@ hipError_t launch_forces(bool sigma, bool types, bool debug, bool list, bool ene
     // kick: 0 forces only, 1 with the closing half-kick, 2 with the step's
     // kick and drift (the closing and step kicks always form the kinetic
     // energy when energy is set; the dump pass has no kick)
-    const int nblk = a.ntiles + a.nespans + a.nbspans > 0 ? forces_grid(a) : 0;
-    if (nblk <= 0) return hipSuccess;
+    const int nblk = forces_grid(a);
     dim3 g(nblk), b(block);
     if (debug) kick = 0;
     if (kick == 1) energy = true;

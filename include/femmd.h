@@ -242,9 +242,11 @@ int fm_time_forces(fm_system *h, int32_t reps, double *ms);
 /* Advance nsteps + 1 steps, timing nsteps of them kernel by kernel (no
  * graph): each kernel's dispatch start and end timestamps, taken by HIP
  * events armed on its launch (hipExtLaunchKernel).  ms[6] = per step: kick
- * (with the binning when cells are walked every step), binning (list mode),
- * counting sort, list build, force pass (0 for a kernel the mode does not
- * launch), whole step from the kick's start to the force pass's end. */
+ * (the opening half-kick of the steps; the steps' own kicks are part of the
+ * force pass, except for replicas without pair forces), binning (list mode;
+ * with the element and bond forces), counting sort (cell walk: with the
+ * element and bond forces), list build, force pass (0 for a kernel the mode
+ * does not launch), whole step with its share of the opening half-kick. */
 int fm_profile_step(fm_system *h, int32_t nsteps, double *ms);
 /* Elastomer clusters (one per fm_add_elastomer call, in call order). */
 int fm_cluster_count(fm_system *h, int32_t *nc);
