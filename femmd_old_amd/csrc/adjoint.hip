@@ -158,18 +158,13 @@ int Engine::adjoint_op(const float *wx, const float *wy, float *jx, float *jy, d
                        double *deps, double *dsig, std::string &err) {
     int rc = check(hipSetDevice(device_), "hipSetDevice", err);
     if (rc) return rc;
-    rc = ensure_order(err);
-    if (rc) return rc;
     rc = adj_alloc(err);
     if (rc) return rc;
-    const int N = N_;
-    const std::vector<int32_t> &iid = iid_h_[0];
-    std::vector<float2> wh(N);
-    for (int u = 0; u < N; ++u) wh[iid[u]] = make_float2(wx[u], wy[u]);
+    const float *const win[2] = {wx, wy};
+    float *const wout[2] = {&w_.p->x, &w_.p->y};
+    rc = io_state_in(0, 2, win, wout, nullptr, 2, err);
+    if (rc) return rc;
     hipError_t he;
-    if ((he = hipMemcpyAsync(w_.p, wh.data(), N * sizeof(float2), hipMemcpyHostToDevice,
-                             stream_)) != hipSuccess)
-        return check(he, "upload w", err);
     if ((he = hipMemsetAsync(dE_.p, 0, dE_.n * sizeof(double), stream_)) != hipSuccess)
         return check(he, "memset", err);
     if ((he = hipMemsetAsync(pacc_.p, 0, pacc_.n * sizeof(double), stream_)) != hipSuccess)
@@ -177,28 +172,9 @@ int Engine::adjoint_op(const float *wx, const float *wy, float *jx, float *jy, d
     rc = adj_pass(err);
     if (rc) return rc;
     primed_ = false;  // the forward force buffers were not refreshed
-    if (launch_total_force(N, jx_.p, jy_.p, cfa_.p, gather_ ? goff_.p : nullptr, gent_.p,
-                           outx_.p, outy_.p, stream_) != hipSuccess)
-        return check(hipGetLastError(), "total", err);
-    std::vector<float> bx(N), by(N);
-    std::vector<double> de(dE_.n), pa(pacc_.n);
-    (void)hipMemcpyAsync(bx.data(), outx_.p, N * sizeof(float), hipMemcpyDeviceToHost, stream_);
-    (void)hipMemcpyAsync(by.data(), outy_.p, N * sizeof(float), hipMemcpyDeviceToHost, stream_);
-    (void)hipMemcpyAsync(de.data(), dE_.p, de.size() * sizeof(double), hipMemcpyDeviceToHost,
-                         stream_);
-    (void)hipMemcpyAsync(pa.data(), pacc_.p, pa.size() * sizeof(double), hipMemcpyDeviceToHost,
-                         stream_);
-    rc = sync(err);
+    rc = io_force_out(0, jx_.p, jy_.p, cfa_.p, gent_.p, jx, jy, err);
     if (rc) return rc;
-    for (int u = 0; u < N; ++u) {
-        if (jx) jx[u] = bx[iid[u]];
-        if (jy) jy[u] = by[iid[u]];
-    }
-    if (dE)
-        for (int e = 0; e < ntri_; ++e) dE[ecaller_h_[e]] = de[e];
-    if (deps) *deps = sum_pairs(pa, 0);
-    if (dsig) *dsig = sum_pairs(pa, 1);
-    return FM_OK;
+    return adj_grads(dE, deps, dsig, err);
 }
 
 // Graphs of recorded segments (adj_record_segment) carry this bit in their
@@ -217,8 +193,6 @@ int Engine::adjoint_forward(int nsteps, int ckpt, std::string &err) {
     if (nsteps < 1) { err = "nsteps must be >= 1"; return FM_ERR_ARG; }
     adj_.valid = false;
     int rc = check(hipSetDevice(device_), "hipSetDevice", err);
-    if (rc) return rc;
-    rc = ensure_order(err);
     if (rc) return rc;
     rc = adj_alloc(err);
     if (rc) return rc;
@@ -371,10 +345,11 @@ int Engine::adjoint_sweep(std::string &err) {
             // and wherever the rebuild rule fired
             rb.assign(len, 0);
             if (len > 1) {
-                rc = check(hipMemcpyAsync(rb.data() + 1, rblog_buf_.p + 1, (len - 1) * sizeof(int32_t),
-                                          hipMemcpyDeviceToHost, stream_), "rebuild log", err);
+                rc = check(launch_report(), "report", err);
                 if (rc) return rc;
-                rc = sync(err);
+                rc = io_out<int32_t>(len - 1, rblog_buf_.p + 1, nullptr, rb.data() + 1, err);
+                if (rc) return rc;
+                rc = sync(err, true);
                 if (rc) return rc;
             }
             rb[0] = 1;
@@ -414,13 +389,17 @@ int Engine::adjoint_sweep(std::string &err) {
 }
 
 int Engine::adj_grads(double *dE, double *deps, double *dsig, std::string &err) {
-    std::vector<double> de(dE_.n), pa(pacc_.n);
-    (void)hipMemcpyAsync(de.data(), dE_.p, de.size() * sizeof(double), hipMemcpyDeviceToHost, stream_);
-    (void)hipMemcpyAsync(pa.data(), pacc_.p, pa.size() * sizeof(double), hipMemcpyDeviceToHost, stream_);
-    const int rc = sync(err);
+    int rc = check(launch_report(), "report", err);
     if (rc) return rc;
-    if (dE)
-        for (int e = 0; e < ntri_; ++e) dE[ecaller_h_[e]] = de[e];
+    if (dE && ntri_ > 0) {
+        rc = io_out(ntri_, dE_.p, ecinv_.p, dE, err);
+        if (rc) return rc;
+    }
+    std::vector<double> pa(pacc_.n);
+    rc = io_out(pa.size(), pacc_.p, nullptr, pa.data(), err);
+    if (rc) return rc;
+    rc = sync(err, true);
+    if (rc) return rc;
     if (deps) *deps = sum_pairs(pa, 0);
     if (dsig) *dsig = sum_pairs(pa, 1);
     return FM_OK;
@@ -448,22 +427,16 @@ int Engine::adjoint_backward(const float *dx, const float *dy, double *dE, doubl
     }
     int rc = check(hipSetDevice(device_), "hipSetDevice", err);
     if (rc) return rc;
-    rc = ensure_order(err);
-    if (rc) return rc;
-    const int N = N_;
     if (adj_zero()) return check(hipGetLastError(), "memset", err);
-    const std::vector<int32_t> &iid = iid_h_[0];
-    std::vector<float> bx(N, 0.0f), by(N, 0.0f);
-    for (int u = 0; u < N; ++u) {
-        if (dx) bx[iid[u]] = dx[u];
-        if (dy) by[iid[u]] = dy[u];
+    const float *in[2];
+    float *out[2];
+    int k = 0;
+    if (dx) { in[k] = dx; out[k++] = xbx_.p; }
+    if (dy) { in[k] = dy; out[k++] = xby_.p; }
+    if (k) {
+        rc = io_state_in(0, k, in, out, nullptr, 1, err);
+        if (rc) return rc;
     }
-    const size_t fb = (size_t)N * sizeof(float);
-    if (hipMemcpyAsync(xbx_.p, bx.data(), fb, hipMemcpyHostToDevice, stream_) != hipSuccess ||
-        hipMemcpyAsync(xby_.p, by.data(), fb, hipMemcpyHostToDevice, stream_) != hipSuccess)
-        return check(hipGetLastError(), "cotangent", err);
-    rc = sync(err);  // the host buffers are reused
-    if (rc) return rc;
     rc = adjoint_sweep(err);
     if (rc) return rc;
     adj_.valid = false;
@@ -479,35 +452,30 @@ int Engine::adjoint_run(int nsteps, int ckpt, int nloss, const int32_t *ids, con
     }
     int rc = check(hipSetDevice(device_), "hipSetDevice", err);
     if (rc) return rc;
-    rc = ensure_order(err);
-    if (rc) return rc;
     const int N = N_;
     for (int k = 0; k < nloss; ++k)
         if (ids[k] < 0 || ids[k] >= N) { err = "loss particle out of range"; return FM_ERR_ARG; }
     rc = adjoint_forward(nsteps, ckpt, err);
     if (rc) return rc;
     // ---- the loss (1/K) sum |x_k - t_k|^2 and its gradient as the seed ----
-    const std::vector<int32_t> &iid = iid_h_[0];
-    std::vector<int32_t> lid(nloss);
     std::vector<float2> tgt(nloss);
-    for (int k = 0; k < nloss; ++k) {
-        lid[k] = iid[ids[k]];
-        tgt[k] = make_float2(tx[k], ty[k]);
-    }
+    for (int k = 0; k < nloss; ++k) tgt[k] = make_float2(tx[k], ty[k]);
     hipError_t he;
-    if ((he = loss_ids_.alloc(nloss)) != hipSuccess) return check(he, "alloc", err);
-    if ((he = loss_t_.alloc(nloss)) != hipSuccess) return check(he, "alloc", err);
     const int nlb = (nloss + 255) / 256;
-    if ((he = loss_part_.alloc(nlb)) != hipSuccess) return check(he, "alloc", err);
-    (void)hipMemcpyAsync(loss_ids_.p, lid.data(), nloss * sizeof(int32_t), hipMemcpyHostToDevice,
-                         stream_);
-    (void)hipMemcpyAsync(loss_t_.p, tgt.data(), nloss * sizeof(float2), hipMemcpyHostToDevice,
-                         stream_);
+    if ((loss_ids_.n < (size_t)nloss && (he = loss_ids_.alloc(nloss)) != hipSuccess) ||
+        (loss_t_.n < (size_t)nloss && (he = loss_t_.alloc(nloss)) != hipSuccess) ||
+        (loss_part_.n < (size_t)nlb && (he = loss_part_.alloc(nlb)) != hipSuccess))
+        return check(he, "alloc", err);
+    rc = io_in((size_t)nloss * sizeof(int32_t), ids, loss_ids_.p, err);
+    if (rc) return rc;
+    rc = io_in((size_t)nloss * sizeof(float2), tgt.data(), loss_t_.p, err);
+    if (rc) return rc;
     if (adj_zero()) return check(hipGetLastError(), "memset", err);
     LossArgs la{};
     la.reps = reps_.p;
     la.n = nloss;
     la.ids = loss_ids_.p;
+    la.iid = iid_.p;
     la.target = loss_t_.p;
     la.x = x_.p;
     la.y = y_.p;
@@ -517,9 +485,11 @@ int Engine::adjoint_run(int nsteps, int ckpt, int nloss, const int32_t *ids, con
     la.part = loss_part_.p;
     if (launch_adj_loss(la, stream_) != hipSuccess) return check(hipGetLastError(), "loss", err);
     std::vector<double> lp(nlb);
-    (void)hipMemcpyAsync(lp.data(), loss_part_.p, nlb * sizeof(double), hipMemcpyDeviceToHost,
-                         stream_);
-    rc = sync(err);  // (lid, tgt: host buffers of the uploads above)
+    rc = check(launch_report(), "report", err);
+    if (rc) return rc;
+    rc = io_out<double>(nlb, loss_part_.p, nullptr, lp.data(), err);
+    if (rc) return rc;
+    rc = sync(err, true);
     if (rc) return rc;
     rc = adjoint_sweep(err);
     if (rc) return rc;

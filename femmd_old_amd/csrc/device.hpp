@@ -371,7 +371,8 @@ struct AdjKickArgs {
 struct LossArgs {
     const RepDesc *reps;
     int32_t n;
-    const int32_t *ids;   // internal ids of the loss particles
+    const int32_t *ids;   // the loss particles (caller ids)
+    const int32_t *iid;   // caller id -> internal id
     const float2 *target;
     const float *x, *y;
     float *xbx, *xby;

@@ -389,7 +389,7 @@ int Engine::build(const std::vector<const HostSystem *> &reps, std::unique_ptr<E
     // (the guard, declared after them, is destroyed first).
     std::vector<int2> hbrep;
     std::vector<Span> hns;
-    std::vector<int32_t> hnr;
+    std::vector<int32_t> hnr, hiid, heinv;
     struct DrainGuard {
         hipStream_t s;
         ~DrainGuard() { (void)hipStreamSynchronize(s); }
@@ -426,6 +426,19 @@ int Engine::build(const std::vector<const HostSystem *> &reps, std::unique_ptr<E
     FM_UP(goff_, goff);
     FM_UP(gent_, gent);
     FM_UP(gpos_, gpos);
+    size_t most = 0;  // particles of the largest replica
+    hiid.reserve(N);
+    for (int r = 0; r < R; ++r) {
+        hiid.insert(hiid.end(), E->iid_h_[r].begin(), E->iid_h_[r].end());
+        most = std::max(most, E->iid_h_[r].size());
+    }
+    FM_UP(iid_, hiid);
+    heinv.resize(E->ntri_);
+    for (int e = 0; e < E->ntri_; ++e)  // (a single system's elements: the adjoint)
+        if (R == 1) heinv[E->ecaller_h_[e]] = e;
+    FM_UP(ecinv_, heinv);
+    if ((he = E->pin_.alloc(4 * most * sizeof(float))) != hipSuccess)
+        return E->check(he, "pinned memory", err);
     {
         // movable particles: no element, bond or cluster refers to them, so
         // a re-ordering may give them new internal ids
@@ -449,8 +462,6 @@ int Engine::build(const std::vector<const HostSystem *> &reps, std::unique_ptr<E
     if ((he = E->buf.alloc(cnt)) != hipSuccess) return E->check(he, "alloc " #buf, err)
     FM_AL(fx_, N);
     FM_AL(fy_, N);
-    FM_AL(outx_, N);
-    FM_AL(outy_, N);
     FM_AL(count_, (size_t)E->ncells_);
     FM_AL(tmp_, (size_t)E->ncells_ * E->cap_);
     E->nsort_ = (E->ncells_ + kSortCells - 1) / kSortCells;
@@ -1182,6 +1193,7 @@ int Engine::launch_reorder_now() {
         a.newof = ro_newof_.p;
     }
     if (launch_reorder(a, stream_) != hipSuccess) return -1;
+    if (launch_invert()) return -1;
     order_stale_ = true;
     ++nreorder_;
     if (!list_ && bins_pending_) {
@@ -1229,7 +1241,8 @@ int Engine::launch_bodies_eager(const BodyKind &k) {
     if (k.close) {
         // femmd2D/src/integrator.cpp:18-19: the observables of the last step
         // (Properties::compute)
-        return launch_observe(obs_args(), true, stream_) == hipSuccess ? 0 : -1;
+        return launch_observe(obs_args(), true, err_.p, &pin_.head()->err, stream_) == hipSuccess ? 0
+                                                                                              : -1;
     }
     return 0;
 }
@@ -1356,25 +1369,22 @@ int Engine::step(int nsteps, std::string &err) {
     steps_ += nsteps;
     ene_valid_ = true;  // the closing force pass formed the energies
     obs_valid_ = true;
-    return sync(err);
+    return sync(err, true);  // (the close reported the error word)
 }
 
-int Engine::sync(std::string &err) {
-    int rc = check(hipStreamSynchronize(stream_), "step", err);
+int Engine::sync(std::string &err, bool reported) {
+    const int rc = reported ? check(hipStreamSynchronize(stream_), "step", err) : io_report(nullptr, 0, err);
     if (rc) return rc;
-    uint32_t e = errors();
-    if (e) {
-        err = dev_error_text(e);
+    if (pin_.head()->err) {
+        err = dev_error_text(pin_.head()->err);
         return FM_ERR_DEVICE;
     }
     return FM_OK;
 }
 
 uint32_t Engine::errors() {
-    uint32_t e = 0;
-    (void)hipMemcpyAsync(&e, err_.p, sizeof(e), hipMemcpyDeviceToHost, stream_);
-    (void)hipStreamSynchronize(stream_);
-    return e;
+    std::string e;
+    return io_report(nullptr, 0, e) == FM_OK ? pin_.head()->err : 0u;
 }
 
 int Engine::clear_errors() {
@@ -1413,12 +1423,21 @@ int Engine::form_observables(std::string &err) {
         return check(hipGetLastError(), "ke", err);
     ObsArgs o = obs_args();
     o.ke_kick = 1;  // the partials k_ke just formed
-    if (launch_observe(o, false, stream_) != hipSuccess)
+    if (launch_observe(o, false, err_.p, &pin_.head()->err, stream_) != hipSuccess)
         return check(hipGetLastError(), "observe", err);
-    rc = sync(err);
+    rc = sync(err, true);
     if (rc) return rc;
     obs_valid_ = true;
     return FM_OK;
+}
+
+// Replica r's observables record, with the device's error word.
+int Engine::read_obs(int r, double *v, std::string &err) {
+    std::lock_guard<std::mutex> lock(pin_.mu);
+    const int rc = io_report(obs_.p + (size_t)kObsStride * r, kObsStride, err);
+    if (rc) return rc;
+    std::memcpy(v, pin_.head()->obs, kObsStride * sizeof(double));
+    return sync(err, true);
 }
 
 int Engine::energies(int r, fm_energies *out, std::string &err) {
@@ -1427,13 +1446,9 @@ int Engine::energies(int r, fm_energies *out, std::string &err) {
     if (rc) return rc;
     rc = form_observables(err);
     if (rc) return rc;
-    obs_h_.resize((size_t)kObsStride * R_);
-    rc = check(hipMemcpyAsync(obs_h_.data(), obs_.p, obs_h_.size() * sizeof(double),
-                              hipMemcpyDeviceToHost, stream_), "energy copy", err);
+    double v[kObsStride];
+    rc = read_obs(r, v, err);
     if (rc) return rc;
-    rc = sync(err);
-    if (rc) return rc;
-    const double *v = &obs_h_[(size_t)kObsStride * r];
     const RepDesc &D = reps_h_[r];
     const double n = D.p1 - D.p0, V = (double)D.Lx * D.Ly;
     std::memset(out, 0, sizeof(*out));
@@ -1458,13 +1473,9 @@ int Engine::averages(int r, fm_averages *out, std::string &err) {
     if (r < 0 || r >= R_) { err = "replica out of range"; return FM_ERR_ARG; }
     int rc = check(hipSetDevice(device_), "hipSetDevice", err);
     if (rc) return rc;
-    obs_h_.resize((size_t)kObsStride * R_);
-    rc = check(hipMemcpyAsync(obs_h_.data(), obs_.p, obs_h_.size() * sizeof(double),
-                              hipMemcpyDeviceToHost, stream_), "averages copy", err);
+    double v[kObsStride];
+    rc = read_obs(r, v, err);
     if (rc) return rc;
-    rc = sync(err);
-    if (rc) return rc;
-    const double *v = &obs_h_[(size_t)kObsStride * r];
     std::memset(out, 0, sizeof(*out));
     const double cnt = v[kObsRaw];
     out->count = (int64_t)cnt;
@@ -1499,53 +1510,37 @@ int Engine::set_observe_every(int every, std::string &err) {
 
 int Engine::get_state(int r, float *x, float *y, float *vx, float *vy, std::string &err) {
     if (r < 0 || r >= R_) { err = "replica out of range"; return FM_ERR_ARG; }
-    {
-        const int orc = ensure_order(err);
-        if (orc) return orc;
-    }
-    const RepDesc &D = reps_h_[r];
-    const int n = D.p1 - D.p0;
-    std::vector<float> buf(n);
+    const int rc = check(hipSetDevice(device_), "hipSetDevice", err);
+    if (rc) return rc;
     float *outs[4] = {x, y, vx, vy};
-    float *srcs[4] = {x_.p, y_.p, vx_.p, vy_.p};
-    const std::vector<int32_t> &iid = iid_h_[r];
+    const float *srcs[4] = {x_.p, y_.p, vx_.p, vy_.p};
+    int k = 0;
     for (int q = 0; q < 4; ++q) {
         if (!outs[q]) continue;
-        int rc = check(hipMemcpyAsync(buf.data(), srcs[q] + D.p0, n * sizeof(float),
-                                      hipMemcpyDeviceToHost, stream_), "get_state", err);
-        if (rc) return rc;
-        rc = check(hipStreamSynchronize(stream_), "get_state", err);
-        if (rc) return rc;
-        for (int u = 0; u < n; ++u) outs[q][u] = buf[iid[u] - D.p0];
+        outs[k] = outs[q];
+        srcs[k++] = srcs[q];
     }
-    return FM_OK;
+    return k ? io_state_out(r, k, srcs, outs, err) : FM_OK;
 }
 
 int Engine::set_state(int r, const float *x, const float *y, const float *vx, const float *vy,
                       std::string &err) {
     if (r < 0 || r >= R_) { err = "replica out of range"; return FM_ERR_ARG; }
-    {
-        const int orc = ensure_order(err);
-        if (orc) return orc;
-    }
+    int rc = check(hipSetDevice(device_), "hipSetDevice", err);
+    if (rc) return rc;
     const RepDesc &D = reps_h_[r];
-    const int n = D.p1 - D.p0;
-    std::vector<float> buf(n);
     const float *ins[4] = {x, y, vx, vy};
     float *dsts[4] = {x_.p, y_.p, vx_.p, vy_.p};
-    const std::vector<int32_t> &iid = iid_h_[r];
+    float wrap[4] = {D.Lx, D.Ly, 0.0f, 0.0f};
+    int k = 0;
     for (int q = 0; q < 4; ++q) {
         if (!ins[q]) continue;
-        for (int u = 0; u < n; ++u) {
-            float v = ins[q][u];
-            if (q == 0) v = wrap_host(v, D.Lx);
-            if (q == 1) v = wrap_host(v, D.Ly);
-            buf[iid[u] - D.p0] = v;
-        }
-        int rc = check(hipMemcpyAsync(dsts[q] + D.p0, buf.data(), n * sizeof(float),
-                                      hipMemcpyHostToDevice, stream_), "set_state", err);
-        if (rc) return rc;
-        rc = check(hipStreamSynchronize(stream_), "set_state", err);
+        ins[k] = ins[q];
+        dsts[k] = dsts[q];
+        wrap[k++] = wrap[q];
+    }
+    if (k) {
+        rc = io_state_in(r, k, ins, dsts, wrap, 1, err);
         if (rc) return rc;
     }
     if (x || y) primed_ = false;
@@ -1561,33 +1556,17 @@ int Engine::set_state(int r, const float *x, const float *y, const float *vx, co
 
 int Engine::get_forces(int r, float *fx, float *fy, std::string &err) {
     if (r < 0 || r >= R_) { err = "replica out of range"; return FM_ERR_ARG; }
-    {
-        const int orc = ensure_order(err);
-        if (orc) return orc;
-    }
-    int rc = ensure_primed(err);
+    int rc = check(hipSetDevice(device_), "hipSetDevice", err);
     if (rc) return rc;
-    // corner forces are held in gather order (no entry table)
-    if (launch_total_force(N_, fx_.p, fy_.p, cf_.p, gather_ ? goff_.p : nullptr, nullptr,
-                           outx_.p, outy_.p, stream_) != hipSuccess)
-        return check(hipGetLastError(), "total force", err);
-    const RepDesc &D = reps_h_[r];
-    const int n = D.p1 - D.p0;
-    std::vector<float> bx(n), by(n);
-    rc = check(hipMemcpyAsync(bx.data(), outx_.p + D.p0, n * sizeof(float), hipMemcpyDeviceToHost,
-                              stream_), "forces", err);
+    rc = ensure_primed(err);
     if (rc) return rc;
-    rc = check(hipMemcpyAsync(by.data(), outy_.p + D.p0, n * sizeof(float), hipMemcpyDeviceToHost,
-                              stream_), "forces", err);
+    // (corner forces are held in gather order: no entry table; the error word
+    // is reported before the forces are waited for)
+    hipError_t he = launch_report();
+    if (he != hipSuccess) return check(he, "report", err);
+    rc = io_force_out(r, fx_.p, fy_.p, cf_.p, nullptr, fx, fy, err);
     if (rc) return rc;
-    rc = sync(err);
-    if (rc) return rc;
-    const std::vector<int32_t> &iid = iid_h_[r];
-    for (int u = 0; u < n; ++u) {
-        if (fx) fx[u] = bx[iid[u] - D.p0];
-        if (fy) fy[u] = by[iid[u] - D.p0];
-    }
-    return FM_OK;
+    return sync(err, true);
 }
 
 int Engine::get_cells(int r, int32_t *ncx, int32_t *ncy, int32_t *key, int32_t *start,

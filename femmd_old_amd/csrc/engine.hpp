@@ -11,6 +11,7 @@
 
 #include <cstdint>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -72,10 +73,36 @@ struct DBuf {
     }
     hipError_t alloc(size_t count) {
         release();
-        n = count;
         if (count == 0) return hipSuccess;
-        return hipMalloc((void **)&p, count * sizeof(T));
+        const hipError_t e = hipMalloc((void **)&p, count * sizeof(T));
+        if (e != hipSuccess) p = nullptr;
+        n = p ? count : 0;
+        return e;
     }
+};
+
+// Pinned host memory of an engine (io.hip): a head the device reports into,
+// and the slots its transfers go through.
+constexpr size_t kIoSlotBytes = 1 << 20;
+constexpr int kIoSlots = 4;
+struct IoHead {
+    uint32_t err;             // the device's error word
+    uint32_t pad[15];
+    double obs[kObsStride];   // one replica's observables record
+};
+struct PinBuf {
+    unsigned char *p = nullptr;
+    size_t slot = 0;
+    int nslot = 0;
+    hipEvent_t ev[kIoSlots] = {};
+    std::mutex mu;  // one transfer at a time
+    PinBuf() = default;
+    PinBuf(const PinBuf &) = delete;
+    PinBuf &operator=(const PinBuf &) = delete;
+    ~PinBuf();
+    hipError_t alloc(size_t most);
+    IoHead *head() const { return reinterpret_cast<IoHead *>(p); }
+    void *data(int s) const { return p + sizeof(IoHead) + (size_t)s * slot; }
 };
 
 class Engine {
@@ -130,7 +157,9 @@ public:
     int64_t reorders() const { return nreorder_; }
     uint32_t errors();
     int clear_errors();
-    int sync(std::string &err);
+    // waits for the stream and reports the device's error word (reported: the
+    // stream's last work has already written it to pin_)
+    int sync(std::string &err, bool reported = false);
     int nrep() const { return R_; }
     int nparticles(int r) const { return reps_h_[r].p1 - reps_h_[r].p0; }
     int64_t steps() const { return steps_; }
@@ -261,6 +290,31 @@ private:
     int check(hipError_t e, const char *what, std::string &err);
     int drop_graph();
 
+    // io.hip: the caller's arrays (caller order) from and to the device's
+    // (internal order).  k <= 4 arrays of replica r's particles; stride: floats
+    // between a particle's values in dst; wrap: per array the box length that
+    // positions are wrapped into (0: as given; null: none)
+    template <class Fill, class Take>
+    int io_read(size_t count, size_t elem, Fill &&fill, Take &&take, std::string &err);
+    template <class Put, class Use>
+    int io_write(size_t count, size_t elem, Put &&put, Use &&use, std::string &err);
+    int io_state_out(int r, int k, const float *const *src, float *const *dst, std::string &err);
+    int io_state_in(int r, int k, const float *const *src, float *const *dst, const float *wrap,
+                    int stride, std::string &err);
+    int io_force_out(int r, const float *fx, const float *fy, const float2 *cf, const int32_t *gent,
+                     float *ox, float *oy, std::string &err);
+    // dst[i] = src[idx ? idx[i] : i] (idx: device)
+    template <class T>
+    int io_out(size_t n, const T *src, const int32_t *idx, T *dst, std::string &err);
+    int io_in(size_t bytes, const void *src, void *dst, std::string &err);
+    int io_report(const double *src, int n, std::string &err);
+    hipError_t launch_report(const double *src = nullptr, int n = 0);  // io_report without the wait
+    int read_obs(int r, double *v, std::string &err);
+    int launch_invert();
+    PinBuf pin_;
+    DBuf<int32_t> iid_;    // caller -> internal id (replica r's at p0)
+    DBuf<int32_t> ecinv_;  // caller -> internal element
+
     int device_ = 0;
     hipStream_t stream_ = nullptr;
     int R_ = 0, N_ = 0, ncells_ = 0, ntri_ = 0, nbond_ = 0, cap_ = 32, lds_cap_ = 2048;
@@ -338,10 +392,9 @@ private:
     std::vector<Span> nspans_h_;
     DBuf<double> ke_node_, ke_tile_;
     DBuf<double> obs_chunk_, obs_;  // observables: level-1 chunks, per-replica records
-    std::vector<double> obs_h_;
     DBuf<int32_t> rng_;
     DBuf<uint32_t> err_;
-    DBuf<float> outx_, outy_;
+    DBuf<float> outx_, outy_;  // unfolded positions (cluster_props)
     DBuf<int32_t> dbg_cnt_;
     DBuf<long long> dbg_s1_, dbg_s2_;
 
@@ -392,10 +445,9 @@ size_t list_build_lds_bytes(int lds_cap, int cell_cap, int nbr_cap, int block, b
 int list_build_resident(bool sigma, int block, const ForceArgs &a, int device);
 hipError_t launch_ctl_reset(Ctl *ctl, int nrep, uint32_t *dmax, int nslots, hipStream_t s);
 size_t forces_lds_bytes(int lds_cap, bool types, bool debug);
-hipError_t launch_total_force(int n, const float *fx, const float *fy, const float2 *cf,
-                              const int32_t *goff, const int32_t *gent, float *ox, float *oy,
-                              hipStream_t s);
-hipError_t launch_observe(const ObsArgs &o, bool accumulate, hipStream_t s);
+// err, report: if set, the error word is also written there (pinned memory)
+hipError_t launch_observe(const ObsArgs &o, bool accumulate, const uint32_t *err, uint32_t *report,
+                          hipStream_t s);
 hipError_t launch_fill_int(int32_t *p, int32_t v, size_t n, hipStream_t s);
 // dst[0, n) = x, dst[n, 2n) = y (graph-safe copy kernel)
 hipError_t launch_copy2(float *dst, const float *x, const float *y, int n, hipStream_t s);

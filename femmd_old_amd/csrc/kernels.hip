@@ -2468,28 +2468,6 @@ __host__ __device__ inline int forces_grid(const ForceArgs &a) {
     return ((forces_book(a) + 7) & ~7) + a.ntiles;
 }
 
-// Total force per particle (pair + gathered corners), internal order.
-__global__ __launch_bounds__(256) void k_total_force(int n, const float *fx,
-                                                     const float *fy,
-                                                     const float2 *cf,
-                                                     const int32_t *goff,
-                                                     const int32_t *gent,
-                                                     float *ox, float *oy) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= n) return;
-    float x = fx[p], y = fy[p];
-    if (goff) {
-        // gent null: cf is held in gather order
-        for (int e = goff[p]; e < goff[p + 1]; ++e) {
-            const float2 c = cf[gent ? gent[e] : e];
-            x += c.x;
-            y += c.y;
-        }
-    }
-    ox[p] = x;
-    oy[p] = y;
-}
-
 // Observables of the current step for every replica, with the same chunks
 // and order as the per-step path: level 1 (one workgroup per chunk), then
 // level 2 (one thread per replica); accumulate: add them to the running sums.
@@ -2497,16 +2475,20 @@ __global__ __launch_bounds__(256) void k_observe_l1(ObsArgs o) {
     __shared__ double red[kObsRed];
     obs_level1(o, blockIdx.x, gridDim.x, red);
 }
-__global__ __launch_bounds__(256) void k_observe_l2(ObsArgs o, int accumulate) {
+__global__ __launch_bounds__(256) void k_observe_l2(ObsArgs o, int accumulate, const uint32_t *err,
+                                                    uint32_t *report) {
+    if (report && blockIdx.x == 0 && threadIdx.x == 0) *report = *err;
     const int r = blockIdx.x * 4 + (int)(threadIdx.x >> 6);  // one wavefront per replica
     if (r < o.nrep) obs_finish(o, r, accumulate != 0);
 }
 
-hipError_t launch_observe(const ObsArgs &o, bool accumulate, hipStream_t s) {
+hipError_t launch_observe(const ObsArgs &o, bool accumulate, const uint32_t *err, uint32_t *report,
+                          hipStream_t s) {
     if (o.nrep <= 0) return hipSuccess;
     hipLaunchKernelGGL(k_observe_l1, dim3(std::min(o.nrep * o.nchunk, 4096)), dim3(256), 0, s,
                        o);
-    hipLaunchKernelGGL(k_observe_l2, dim3((o.nrep + 3) / 4), dim3(256), 0, s, o, accumulate ? 1 : 0);
+    hipLaunchKernelGGL(k_observe_l2, dim3((o.nrep + 3) / 4), dim3(256), 0, s, o, accumulate ? 1 : 0,
+                       err, report);
     return hipGetLastError();
 }
 
@@ -3018,7 +3000,7 @@ __global__ __launch_bounds__(256) void k_adj_loss(LossArgs a) {
     double l = 0.0, z = 0.0;
     if (k < a.n) {
         const RepDesc R = a.reps[0];
-        const int p = a.ids[k];
+        const int p = a.iid[a.ids[k]];
         const float2 t = a.target[k];
         float dx = a.x[p] - t.x, dy = a.y[p] - t.y;
         if (dx >= R.hLx) dx -= R.Lx; else if (dx < -R.hLx) dx += R.Lx;
@@ -3492,16 +3474,6 @@ hipError_t launch_list_build(bool sigma, int block, const ForceArgs &a, hipStrea
         FM_GO((k_list_build<true>), g, dim3(block), lds, s, a);
     else
         FM_GO((k_list_build<false>), g, dim3(block), lds, s, a);
-    return hipGetLastError();
-}
-
-hipError_t launch_total_force(int n, const float *fx, const float *fy,
-                              const float2 *cf, const int32_t *goff,
-                              const int32_t *gent, float *ox, float *oy,
-                              hipStream_t s) {
-    if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_total_force, dim3((n + 255) / 256), dim3(256), 0, s, n,
-                       fx, fy, cf, goff, gent, ox, oy);
     return hipGetLastError();
 }
 

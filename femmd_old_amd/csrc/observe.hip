@@ -83,12 +83,14 @@ int Engine::cluster_props(int r, double *out, float *ux, float *uy, std::string 
     if (r < 0 || r >= R_) { err = "replica out of range"; return FM_ERR_ARG; }
     int rc = check(hipSetDevice(device_), "hipSetDevice", err);
     if (rc) return rc;
-    rc = ensure_order(err);
-    if (rc) return rc;
     const bool unf = ux || uy;
     if (unf) {
         // unfolded positions of the cluster nodes, the wrapped positions of
         // every other particle
+        hipError_t he;
+        if ((!outx_.p && (he = outx_.alloc(N_)) != hipSuccess) ||
+            (!outy_.p && (he = outy_.alloc(N_)) != hipSuccess))
+            return check(he, "alloc", err);
         if (hipMemcpyAsync(outx_.p, x_.p, N_ * sizeof(float), hipMemcpyDeviceToDevice, stream_) !=
                 hipSuccess ||
             hipMemcpyAsync(outy_.p, y_.p, N_ * sizeof(float), hipMemcpyDeviceToDevice, stream_) !=
@@ -97,39 +99,26 @@ int Engine::cluster_props(int r, double *out, float *ux, float *uy, std::string 
     }
     if (run_cluster_props(unf ? outx_.p : nullptr, unf ? outy_.p : nullptr))
         return check(hipGetLastError(), "cluster props", err);
-    const int ncl = (int)cl_rep_h_.size();
-    std::vector<double> o((size_t)std::max(ncl, 1) * kClusterOut);
-    rc = check(hipMemcpyAsync(o.data(), cl_out_.p, o.size() * sizeof(double), hipMemcpyDeviceToHost,
-                              stream_), "cluster props", err);
+    rc = check(launch_report(), "report", err);
     if (rc) return rc;
-    const RepDesc &D = reps_h_[r];
-    const int n = D.p1 - D.p0;
-    std::vector<float> bx, by;
-    if (unf) {
-        bx.resize(n);
-        by.resize(n);
-        (void)hipMemcpyAsync(bx.data(), outx_.p + D.p0, n * sizeof(float), hipMemcpyDeviceToHost,
-                             stream_);
-        (void)hipMemcpyAsync(by.data(), outy_.p + D.p0, n * sizeof(float), hipMemcpyDeviceToHost,
-                             stream_);
-    }
-    rc = sync(err);
-    if (rc) return rc;
-    int k = 0;
-    for (int c = 0; c < ncl; ++c) {
-        if (cl_rep_h_[c] != r) continue;
-        if (out)
-            for (int q = 0; q < kClusterOut; ++q) out[(size_t)k * kClusterOut + q] = o[(size_t)c * kClusterOut + q];
-        ++k;
+    // replica r's clusters are consecutive
+    const int c0 = (int)(std::lower_bound(cl_rep_h_.begin(), cl_rep_h_.end(), r) - cl_rep_h_.begin());
+    const int c1 = (int)(std::upper_bound(cl_rep_h_.begin(), cl_rep_h_.end(), r) - cl_rep_h_.begin());
+    if (out && c1 > c0) {
+        rc = io_out((size_t)(c1 - c0) * kClusterOut, cl_out_.p + (size_t)c0 * kClusterOut, nullptr,
+                           out, err);
+        if (rc) return rc;
     }
     if (unf) {
-        const std::vector<int32_t> &iid = iid_h_[r];
-        for (int u = 0; u < n; ++u) {
-            if (ux) ux[u] = bx[iid[u] - D.p0];
-            if (uy) uy[u] = by[iid[u] - D.p0];
-        }
+        const float *src[2];
+        float *dst[2];
+        int k = 0;
+        if (ux) { src[k] = outx_.p; dst[k++] = ux; }
+        if (uy) { src[k] = outy_.p; dst[k++] = uy; }
+        rc = io_state_out(r, k, src, dst, err);
+        if (rc) return rc;
     }
-    return FM_OK;
+    return sync(err, true);
 }
 
 int Engine::cluster_virial(int r, double *vir, std::string &err) {
@@ -146,7 +135,8 @@ int Engine::cluster_virial(int r, double *vir, std::string &err) {
             return check(hipGetLastError(), "cluster virial", err);
         if (list_) primed_ = false;
         hipError_t he;
-        if ((he = cl_vir_.alloc(tiles_h_.size())) != hipSuccess) return check(he, "alloc", err);
+        if (cl_vir_.n != tiles_h_.size() && (he = cl_vir_.alloc(tiles_h_.size())) != hipSuccess)
+            return check(he, "alloc", err);
         ClusterVirialArgs A{};
         A.f = force_args();
         A.cid = cid_.p;
@@ -154,11 +144,12 @@ int Engine::cluster_virial(int r, double *vir, std::string &err) {
         A.out = cl_vir_.p;
         if (launch_cluster_virial(sigma_, types_, block_, A, stream_) != hipSuccess)
             return check(hipGetLastError(), "cluster virial", err);
-        std::vector<double> t(tiles_h_.size());
-        rc = check(hipMemcpyAsync(t.data(), cl_vir_.p, t.size() * sizeof(double),
-                                  hipMemcpyDeviceToHost, stream_), "cluster virial", err);
+        rc = check(launch_report(), "report", err);
         if (rc) return rc;
-        rc = sync(err);
+        std::vector<double> t(tiles_h_.size());
+        rc = io_out(t.size(), cl_vir_.p, nullptr, t.data(), err);
+        if (rc) return rc;
+        rc = sync(err, true);
         if (rc) return rc;
         for (size_t k = 0; k < t.size(); ++k)
             if (tiles_h_[k].rep == r) v += t[k];
