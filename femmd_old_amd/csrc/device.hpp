@@ -74,11 +74,19 @@ struct alignas(16) RepDesc {
 //            {uKinetic, uPotential, uTotal, pressure, virial, feaVirial,
 //            uBonded, uFea} (Prop::accum, femmd2D/src/properties.h:6-13)
 // A step's totals are formed in two levels with a fixed order (no float
-// atomics): kObsChunks chunks per replica, each the fixed-order sum of one
+// atomics): up to kObsChunks chunks per replica, each the fixed-order sum of one
 // slice of the per-workgroup partials (ke, lj, fea, bond), written by one
 // workgroup of 256 threads; then the chunks in chunk order.
 constexpr int kObsRaw = 8, kObsAvg = 8, kObsStride = 32, kObsChunks = 16;
 constexpr int kObsRed = 4 * kObsRaw;  // LDS doubles of a level-1 reduction
+// Level-1 chunks of a replica whose longest range holds n partials: one per
+// 256 (a pass of the workgroup that forms it), at most kObsChunks.  With 16 at
+// every size, the one binning workgroup of a 256-particle system formed 16 in
+// turn: 30 us of a 42 us step, now 4.
+__host__ __device__ inline int obs_chunks_of(int n) {
+    const int c = (n + 255) / 256;
+    return c < 1 ? 1 : c > kObsChunks ? kObsChunks : c;
+}
 struct ObsArgs {
     const RepDesc *reps;
     const int32_t *rng;        // 8 per replica: kick, tile, element, bond ranges
@@ -93,8 +101,7 @@ struct ObsArgs {
     const double *fea_part;    // 2 per element span: U, W
     const double *bond_part;   // 2 per bond span: U, W
     double *chunk;             // kObsChunks * kObsRaw per replica (level 1)
-    int32_t nchunk;            // level-1 chunks per replica (1..kObsChunks; of
-                               // the replica's partials in order)
+    int32_t nchunk;            // the largest replica's level-1 chunks
     double *obs;               // kObsStride per replica
     int32_t nrep;
 };

@@ -598,6 +598,7 @@ int Engine::build_tiles(const std::vector<int> &tile_w, std::string &err) {
     tiles_h_.clear();
     tile_w_.assign(R_, 0);
     rng_h_.assign(8 * R_, 0);
+    obs_nchunk_ = 1;
     int kb = 0, eb = 0, bb = 0;
     double worst = 0.0;
     for (int r = 0; r < R_; ++r) {
@@ -651,6 +652,8 @@ int Engine::build_tiles(const std::vector<int> &tile_w, std::string &err) {
         g[6] = bb;
         while (bb < (int)bspans_h_.size() && bspans_h_[bb].rep == r) ++bb;
         g[7] = bb;
+        obs_nchunk_ = std::max(obs_nchunk_, obs_chunks_of(std::max(std::max(g[1] - g[0], g[3] - g[2]),
+                                                                   std::max(g[5] - g[4], g[7] - g[6]))));
     }
     // LDS capacity: 1.3 x the close-packed count of the staged cells (an
     // elastomer under compression can exceed close packing a little), rounded
@@ -1062,10 +1065,7 @@ ObsArgs Engine::obs_args(bool prev) {
     o.chunk = obs_chunk_.p;
     o.obs = obs_.p;
     o.nrep = R_;
-    // a single system's partials in 16 chunks (one workgroup each); a batch
-    // of many replicas one chunk per replica (each replica's partials are
-    // few, and the jobs are many)
-    o.nchunk = R_ > 8 ? 1 : kObsChunks;
+    o.nchunk = obs_nchunk_;
     return o;
 }
 

@@ -350,6 +350,7 @@ private:
     std::vector<Span> kspans_h_, espans_h_, bspans_h_;
     std::vector<Tile> tiles_h_;
     std::vector<int32_t> rng_h_;  // per replica 8 ints (energy ranges)
+    int obs_nchunk_ = 1;          // level-1 chunks of the largest replica
 
     DBuf<RepDesc> reps_;
     DBuf<PairEntry> ptab_;

@@ -187,7 +187,7 @@ __device__ __forceinline__ void block_sum2(double &a, double &b, double *red) {
 // ranges (kick spans, tiles, element spans, bond spans), formed by one
 // workgroup of exactly 256 threads (the binning, sort and observe kernels all
 // run 256), so its bits do not depend on which kernel forms it.  Level 2:
-// one thread sums the replica's chunks in chunk order.
+// one wavefront sums the replica's chunks in a fixed order.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ void obs_slice(int b, int e, int c, int nc, int &lo, int &hi) {
     const long long len = e - b;
@@ -195,21 +195,28 @@ __device__ __forceinline__ void obs_slice(int b, int e, int c, int nc, int &lo, 
     hi = b + (int)(len * (c + 1) / nc);
 }
 
+// Level-1 chunks of replica r: see obs_chunks_of.
+__device__ __forceinline__ int obs_nchunk(const int32_t *g) {
+    return obs_chunks_of(max(max(g[1] - g[0], g[3] - g[2]), max(g[5] - g[4], g[7] - g[6])));
+}
+
 // Level 1 for chunk c of replica r: out[0, 8) of the chunk (see kObsRaw).
 // Called by every thread of a 256-thread workgroup (uniformly).
 __device__ void obs_chunk(const ObsArgs &o, int r, int c, double *red) {
     const int32_t *g = o.rng + 8 * r;
     const int tid = threadIdx.x;
+    const int nc = obs_nchunk(g);
+    if (c >= nc) return;  // (a larger replica's count; uniform)
     // the slices of the partials: kinetic energy of a query (k_ke, over the
     // kick spans) or of the particles the node kick integrated, tiles (U and
     // W; kinetic energy of the particles the pair pass integrated), elements,
     // bonds
     const int kb = o.ke_kick ? g[0] : o.nrng[2 * r], ke = o.ke_kick ? g[1] : o.nrng[2 * r + 1];
     int l0, h0, l1, h1, l2, h2, l3, h3;
-    obs_slice(kb, ke, c, o.nchunk, l0, h0);
-    obs_slice(g[2], g[3], c, o.nchunk, l1, h1);
-    obs_slice(g[4], g[5], c, o.nchunk, l2, h2);
-    obs_slice(g[6], g[7], c, o.nchunk, l3, h3);
+    obs_slice(kb, ke, c, nc, l0, h0);
+    obs_slice(g[2], g[3], c, nc, l1, h1);
+    obs_slice(g[4], g[5], c, nc, l2, h2);
+    obs_slice(g[6], g[7], c, nc, l3, h3);
     const double2 *kin = reinterpret_cast<const double2 *>(o.ke_kick ? o.ke_part : o.ke_node);
     const double2 *lj = reinterpret_cast<const double2 *>(o.lj_part);
     const double2 *kt = reinterpret_cast<const double2 *>(o.ke_tile);
@@ -274,8 +281,10 @@ __device__ void obs_finish(const ObsArgs &o, int r, bool accumulate) {
     static_assert(kObsRaw == 8 && kObsAvg == 8 && kObsChunks == 16, "lane layout of the totals");
     const int lane = threadIdx.x & 63, k = lane & 7, g = lane >> 3;
     const double *q = o.chunk + ((size_t)r * kObsChunks + g) * kObsRaw + k;
-    const double x = g < o.nchunk ? q[0] : 0.0;
-    const double y = g + 8 < o.nchunk ? q[8 * kObsRaw] : 0.0;
+    // (read before the count is known: a chunk past it is not used)
+    const double x0 = q[0], y0 = q[8 * kObsRaw];
+    const int nc = obs_nchunk(o.rng + 8 * r);
+    const double x = g < nc ? x0 : 0.0, y = g + 8 < nc ? y0 : 0.0;
     double t = k == 1 ? fmax(x, y) : x + y;
 #pragma unroll
     for (int m = 8; m < 64; m <<= 1) {
