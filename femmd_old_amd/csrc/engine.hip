@@ -464,7 +464,8 @@ int Engine::build(const std::vector<const HostSystem *> &reps, std::unique_ptr<E
     FM_AL(fy_, N);
     FM_AL(count_, (size_t)E->ncells_);
     FM_AL(tmp_, (size_t)E->ncells_ * E->cap_);
-    E->nsort_ = (E->ncells_ + kSortCells - 1) / kSortCells;
+    E->sort_cells_ = E->ncells_ <= kSortFewMax ? kSortCellsFew : kSortCells;
+    E->nsort_ = (E->ncells_ + E->sort_cells_ - 1) / E->sort_cells_;
     FM_AL(sort_status_, std::max(E->nsort_, 1));
     hbrep.assign(std::max(E->nsort_, 1), make_int2(0, 0));
     {
@@ -472,7 +473,7 @@ int Engine::build(const std::vector<const HostSystem *> &reps, std::unique_ptr<E
         // cells [cell0, cell0 + ncx * ncy + 1))
         int r = 0;
         for (int b = 0; b < E->nsort_; ++b) {
-            const int c0 = b * kSortCells, c1 = std::min(c0 + kSortCells, E->ncells_) - 1;
+            const int c0 = b * E->sort_cells_, c1 = std::min(c0 + E->sort_cells_, E->ncells_) - 1;
             while (r + 1 < R && rd[r + 1].cell0 <= c0) ++r;
             int r1 = r;
             while (r1 + 1 < R && rd[r1 + 1].cell0 <= c1) ++r1;
@@ -762,6 +763,7 @@ int Engine::launch_bin(bool gated) {
             d.ftile = ftile_.p;
             d.fblock = fblock_.p;
             d.nsort = nsort_;
+            d.sort_cells = sort_cells_;
             d.nf = nf_.p;
             d.rinfo = rinfo_.p;
             d.mark = mark_.p;
@@ -885,6 +887,7 @@ int Engine::launch_sort(bool gated, bool elems) {
     s.ncells = ncells_;
     s.cap = cap_;
     s.nsort = nsort_;
+    s.cells = sort_cells_;
     s.brep = brep_.p;
     s.count = count_.p;
     s.tmp = tmp_.p;

@@ -366,7 +366,7 @@ private:
     DBuf<uint32_t> ro_tmp_;
     DBuf<int32_t> count_, tmp_, start_, perm_, sorted_typ_;
     DBuf<unsigned long long> sort_status_, sort_ticket_;
-    int nsort_ = 0;
+    int nsort_ = 0, sort_cells_ = kSortCells;
     int lb_grid_ = 0;  // gated list-build grid (resident workgroups)
     DBuf<float4> sorted_;
     DBuf<Span> kspans_, espans_, bspans_;

@@ -608,8 +608,8 @@ __global__ __launch_bounds__(256) void k_flags(DecideArgs d) {
             info.y = d.rng[8 * r + 3] - d.rng[8 * r + 2];
             if (d.fblock) {
                 // the replica's cells, with its closing empty cell
-                const int b0 = R.cell0 / kSortCells;
-                const int b1 = (R.cell0 + R.ncx * R.ncy) / kSortCells;
+                const int b0 = R.cell0 / d.sort_cells;
+                const int b1 = (R.cell0 + R.ncx * R.ncy) / d.sort_cells;
                 for (int b = b0; b <= b1; ++b) d.mark[b] = 1;
             }
         }
@@ -907,13 +907,13 @@ __global__ __launch_bounds__(kKickThreads) void k_bin(KickArgs a, ElemArgs el) {
 // ---------------------------------------------------------------------------
 // Counting sort (femmd2D/src/nn.cpp:8-20 cell fill order, re-designed as a
 // single pass).  Workgroup b (taken in launch order from a ticket counter)
-// owns cells [b * kSortCells, (b + 1) * kSortCells): it reads and clears
+// owns cells [b * CELLS, (b + 1) * CELLS): it reads and clears
 // their capped counts, scans them, and publishes a status word before it
 // looks back: an inclusive prefix at once when the block holds the first
 // cell of a replica (every replica's sorted positions start at its own p0,
 // so the scan restarts there), else its aggregate, replaced by the inclusive
 // prefix once its look-back is done.  Look-back by the first wavefront
-// reads up to 64 predecessors at a time.  Each status word is one 64-bit
+// reads up to 256 predecessors at a time.  Each status word is one 64-bit
 // relaxed atomic (value, state, launch epoch), so no fences are needed;
 // the cell starts and the scattered particles are read by later kernels
 // only.  A workgroup waits only on lower tickets, whose workgroups are
@@ -923,10 +923,17 @@ __global__ __launch_bounds__(kKickThreads) void k_bin(KickArgs a, ElemArgs el) {
 // batches): the blocks to sort come from k_decide's list, taken in ticket
 // order from a per-step counter, with the step's epoch and a status array
 // of their own; workgroups beyond the list leave before taking a ticket.
+// Bound by its chain of dependent loads (ticket, counts, slot lists, caller
+// indices and rows, look-back): the rows are loaded once, with the caller
+// indices and before the look-back (they were loaded after it, from a second
+// read of the slot list).  Cell walk of 114,140 particles 18.6 -> 14.2 us a
+// step, a rebuild of 4,367 particles 20.7 -> 8.7, of 1.14 million 35.6 ->
+// 34.6, 512 replicas 28.5 -> 24.3.
 // ---------------------------------------------------------------------------
 constexpr unsigned long long kLbAggregate = 1ull, kLbInclusive = 2ull;
-constexpr int kSortIds = 4096;  // slot entries a sort workgroup copies to LDS
-constexpr int kSortBatch = 4;   // particles per lane in flight in the scatter
+constexpr int kSortThreads = 256;
+constexpr int kSortFill = 16;   // entries per cell a sort workgroup has LDS room for
+constexpr int kSortBatch = 4;   // particles per lane in flight
 constexpr int kLbSpinLimit = 1 << 22;
 
 __device__ __forceinline__ unsigned long long lb_word(uint32_t epoch, unsigned long long state,
@@ -946,15 +953,66 @@ __device__ __forceinline__ int rep_of_cell(const ScanArgs &a, int b, int c) {
     return lo;
 }
 
-__global__ __launch_bounds__(kSortCells) void k_sort(ScanArgs a, ElemArgs el) {
-    __shared__ int s_ex[kSortCells + 1];  // local exclusive prefix of the counts
-    __shared__ int s_st[kSortCells];      // cell starts
-    __shared__ int s_lim[kSortCells];     // end of each cell's replica range
-    __shared__ int s_w[kSortCells / 64];
+// The carry-in of sort block b, one wavefront (all lanes): the sum of its
+// predecessors' aggregates back to the nearest inclusive word, 256 words at a
+// time, four consecutive ones per lane.
+__device__ int sort_look_back(const unsigned long long *status, int b, uint32_t epoch, uint32_t *err) {
+    const int lane = threadIdx.x & 63;
+    int carry = 0, spins = 0;
+    for (int j = b - 1;;) {
+        int sum = 0;
+        bool inc = false, valid = true;  // an inclusive word met; every word up to it published
+        unsigned long long v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int q = j - 4 * lane - u;
+            v[u] = q >= 0 ? __hip_atomic_load(status + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            // q < 0 cannot be reached before an inclusive word (block 0
+            // always holds replica 0's first cell); treated as inclusive 0
+            const bool out = j - 4 * lane - u < 0;
+            const bool cur = (uint32_t)(v[u] >> 34) == (epoch & 0x3fffffffu);
+            const unsigned long long st = (v[u] >> 32) & 3ull;
+            if (!inc) {
+                valid = valid && (out || (cur && st != 0ull));
+                sum += out ? 0 : (int)(uint32_t)v[u];
+            }
+            inc = inc || out || (cur && st == kLbInclusive);
+        }
+        const unsigned long long im = __ballot(inc), vm = __ballot(valid);
+        const int k = im ? (__ffsll(im) - 1) : 63;
+        const unsigned long long want = (k == 63) ? ~0ull : ((2ull << k) - 1ull);
+        if ((vm & want) != want) {
+            if (++spins > kLbSpinLimit) {  // never expected: report, end the wait
+                if (lane == 0) atomicOr(err, 32u);  // FM_DEV_SORT_STALL
+                return carry;
+            }
+            continue;
+        }
+        carry += wave_sum_int(lane <= k ? sum : 0);
+        if (im) return carry;
+        j -= 256;
+    }
+}
+
+// A sort workgroup's entries in flight: kSortBatch per lane.
+struct SortEntries {
+    int i[kSortBatch], u[kSortBatch];  // particle (-1: none) and its caller index
+    uint8_t cl[kSortBatch];            // its cell (local index)
+};
+
+template <int CELLS>
+__global__ __launch_bounds__(kSortThreads) void k_sort(ScanArgs a, ElemArgs el) {
+    constexpr int kIds = CELLS * kSortFill;
+    __shared__ int s_ex[CELLS + 1];   // local exclusive prefix of the counts
+    __shared__ int s_st[CELLS];       // cell starts (-1: the carry-in + s_ex)
+    __shared__ int s_lim[CELLS];      // end of each cell's replica range
+    __shared__ int s_w[CELLS / 64];
     __shared__ unsigned long long s_tk;
-    __shared__ int s_carry, s_head;
-    __shared__ int s_ids[kSortIds];       // the block's slot entries' caller indices, cell order
-    __shared__ uint8_t s_cl[kSortIds];    // their cell (local index)
+    __shared__ int s_carry, s_head, s_flag;
+    __shared__ int s_ids[kIds];       // the block's slot entries' caller indices, cell order
     __shared__ double s_ored[kObsRed];
     // (cell walk) the step's element and bond forces, by the workgroups past
     // the sort's, and the previous step's observables, level 1, before the
@@ -979,197 +1037,193 @@ __global__ __launch_bounds__(kSortCells) void k_sort(ScanArgs a, ElemArgs el) {
     const uint32_t epoch =
         listed ? (uint32_t)a.nf[4] : (uint32_t)(tk / (unsigned long long)a.nsort);
     unsigned long long *const status = listed ? a.status2 : a.status;
-    const int c0 = b * kSortCells, c = c0 + t;
+    const int c0 = b * CELLS;
     if (a.ctl && !listed) {
         // gated (list mode): a block holding no cell of a rebuilding replica
         // has nothing to count, scan or scatter, and no rebuilding replica
         // looks back past its own first block, so it is skipped whole
-        __syncthreads();
         if (t == 0) {
             const int2 br = a.brep[b];
             int f = 0;
             for (int q = br.x; q <= br.y; ++q) f |= a.ctl[q].flag;
-            s_head = f;
+            s_flag = f;
         }
         __syncthreads();
-        if (!s_head) return;
+        if (!s_flag) return;
     }
+    // thread t counts cell c (the threads past the cells take the last one's
+    // replica and count nothing)
+    const int c = c0 + min(t, CELLS - 1);
+    const bool mine = t < CELLS && c < a.ncells;
     int n = 0;
-    if (c < a.ncells) {
+    if (mine) {
         n = min(a.count[c], a.cap);
         a.count[c] = 0;  // ready for the next binning
     }
     const int r = rep_of_cell(a, b, min(c, a.ncells - 1));
     const RepDesc &R = a.reps[r];
-    s_lim[t] = R.p1;
     const int hl = R.cell0 - c0;  // replica's first cell, local (< 0: earlier block)
     // block exclusive scan
     const int incl = wave_incl_scan(n);
-    if (lane == 63) s_w[w] = incl;
+    int ex = incl - n;
+    if (CELLS > 64) {
+        if (lane == 63) s_w[w] = incl;
+        __syncthreads();
+        for (int k = 0; k < w; ++k) ex += s_w[k];
+    }
+    if (t < CELLS) {
+        s_ex[t] = ex;
+        s_lim[t] = R.p1;
+    }
+    if (t == CELLS - 1) {
+        s_ex[CELLS] = ex + n;
+        s_head = hl >= 0;
+    }
     __syncthreads();
-    int wb = 0;
-    for (int k = 0; k < w; ++k) wb += s_w[k];
-    const int ex = wb + incl - n;
-    s_ex[t] = ex;
-    if (t == kSortCells - 1) s_ex[kSortCells] = ex + n;
-    __syncthreads();
-    const int tot = s_ex[kSortCells];
+    const int tot = s_ex[CELLS];
     // publish (the last cell's replica decides: its first cell in this block
     // means the block's end value is known without look-back)
-    if (t == kSortCells - 1) {
-        s_head = hl >= 0;
+    if (t == CELLS - 1) {
         const unsigned long long v = (hl >= 0)
             ? lb_word(epoch, kLbInclusive, R.p0 + tot - s_ex[hl])
             : lb_word(epoch, kLbAggregate, tot);
         __hip_atomic_store(status + b, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    // look-back, needed when the block's first cell continues a replica
-    // begun in an earlier block (uniform: read from the first cell)
-    // (not for a replica that does not rebuild: its starts are not written)
-    if (t == 0) s_carry = (hl >= 0 || (a.ctl && !a.ctl[r].flag)) ? -1 : 0;
-    __syncthreads();
-    const bool need = s_carry == 0;
-    if (need && w == 0) {
-        int carry = 0;
-        int j = b - 1;
-        int spins = 0;
-        while (true) {
-            const int q = j - lane;
-            unsigned long long v = 0;
-            if (q >= 0) v = __hip_atomic_load(status + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            const bool cur = (uint32_t)(v >> 34) == (epoch & 0x3fffffffu);
-            const unsigned long long st = (v >> 32) & 3ull;
-            // q < 0 cannot be reached before an inclusive word (block 0
-            // always holds replica 0's first cell); treated as inclusive 0
-            const bool valid = (q < 0) || (cur && st != 0ull);
-            const bool inc = (q < 0) || (cur && st == kLbInclusive);
-            const unsigned long long im = __ballot(inc), vm = __ballot(valid);
-            const int k = im ? (__ffsll(im) - 1) : 63;
-            const unsigned long long want = (k == 63) ? ~0ull : ((2ull << k) - 1ull);
-            if ((vm & want) != want) {
-                if (++spins > kLbSpinLimit) {  // never expected: report, end the wait
-                    if (lane == 0) atomicOr(a.err, 32u);  // FM_DEV_SORT_STALL
-                    break;
-                }
-                continue;
+    if (t < CELLS) s_st[t] = hl >= 0 ? R.p0 + ex - s_ex[hl] : -1;
+    // scatter: the block's particles in cell order; a particle's sorted
+    // position is its cell's start + its rank among the cell's members by
+    // their index in the caller's order, as the reference's cell fill walks
+    // the particles (femmd2D/src/nn.cpp:8-20), whatever the internal order.
+    // The caller indices of the block's slot entries are first gathered into
+    // LDS, so the ranks read LDS; a block with more particles than that holds
+    // reads the slot lists from memory.
+    const bool in_lds = tot <= kIds;
+    // the entries q0, q0 + kSortThreads, ... of this lane, loads batched
+    auto load = [&](int q0, SortEntries &s) {
+#pragma unroll
+        for (int u = 0; u < kSortBatch; ++u) {
+            const int q = q0 + u * kSortThreads;
+            s.i[u] = -1;
+            if (q < tot) {
+                int lo = 0;
+#pragma unroll
+                for (int h = CELLS / 2; h > 0; h >>= 1)
+                    if (s_ex[lo + h] <= q) lo += h;
+                s.cl[u] = (uint8_t)lo;
+                s.i[u] = a.tmp[(size_t)(c0 + lo) * a.cap + (q - s_ex[lo])];
             }
-            carry += wave_sum_int((lane <= k && q >= 0) ? (int)(uint32_t)v : 0);
-            if (im) break;
-            j -= 64;
         }
+#pragma unroll
+        for (int u = 0; u < kSortBatch; ++u) s.u[u] = s.i[u] >= 0 ? a.uid[s.i[u]] : 0;
+    };
+    // what a sorted entry holds of its particle
+    struct Row {
+        float4 e[kSortBatch];
+        int ty[kSortBatch];
+    };
+    auto load_row = [&](const SortEntries &s, Row &o) {
+#pragma unroll
+        for (int u = 0; u < kSortBatch; ++u) {
+            if (s.i[u] >= 0) {
+                const int i = s.i[u];
+                o.e[u].x = a.x[i];
+                o.e[u].y = a.y[i];
+                o.e[u].z = __int_as_float(a.grp[i]);
+                o.e[u].w = a.sig ? a.sig[i] : 0.0f;
+                o.ty[u] = a.typ ? a.typ[i] : 0;
+            }
+        }
+    };
+    // The first round's loads are issued before the look-back, whose wait
+    // they share; a lane's later rounds (denser blocks) load twice.
+    constexpr int kRound = kSortBatch * kSortThreads;
+    SortEntries s0;
+    Row w0;
+    load(t, s0);
+    load_row(s0, w0);
+    if (in_lds) {
+#pragma unroll
+        for (int u = 0; u < kSortBatch; ++u)
+            if (s0.i[u] >= 0) s_ids[t + u * kSortThreads] = s0.u[u];
+        for (int q0 = t + kRound; q0 < tot; q0 += kRound) {
+            SortEntries s;
+            load(q0, s);
+#pragma unroll
+            for (int u = 0; u < kSortBatch; ++u)
+                if (s.i[u] >= 0) s_ids[q0 + u * kSortThreads] = s.u[u];
+        }
+    }
+    if (w == 0) {
+        // look-back, needed when the block's first cell continues a replica
+        // begun in an earlier block (not for a replica that does not
+        // rebuild: its starts are not written)
+        const bool need = __builtin_amdgcn_readfirstlane((hl >= 0 || (a.ctl && !a.ctl[r].flag)) ? 0 : 1);
+        const int carry = need ? sort_look_back(status, b, epoch, a.err) : 0;
         if (lane == 0) {
             s_carry = carry;
-            if (!s_head)  // a block holding a replica's first cell published already
+            if (need && !s_head)  // a block holding a replica's first cell published already
                 __hip_atomic_store(status + b, lb_word(epoch, kLbInclusive, carry + tot),
                                    __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
     __syncthreads();
-    const int st = (hl >= 0) ? R.p0 + ex - s_ex[hl] : s_carry + ex;
-    s_st[t] = st;
-    if (c < a.ncells) {
+    const int carry = s_carry;
+    if (mine) {
+        const int st = s_st[t] >= 0 ? s_st[t] : carry + ex;
         // list mode: only the rebuilding replicas' cell starts change (the
         // others' lists index staging laid out by their own last starts)
         if (!a.ctl || a.ctl[r].flag) a.start[c] = st;
         if (c == a.ncells - 1) a.start[a.ncells] = st + n;
     }
-    __syncthreads();
-    // scatter: the block's particles in cell order; a particle's sorted
-    // position is its cell's start + its rank among the cell's members by
-    // their index in the caller's order, as the reference's cell fill walks
-    // the particles (femmd2D/src/nn.cpp:8-20), whatever the internal order.
-    // The block's slot entries' caller indices are first gathered into LDS
-    // (loads batched per lane), so the ranks read LDS; a block with more
-    // particles than the LDS copy holds reads the slot lists from memory.
-    const bool in_lds = tot <= kSortIds;
-    auto cell_of = [&](int q) {
-        int lo = 0, hi = kSortCells;
-        while (hi - lo > 1) {
-            const int mid = (lo + hi) >> 1;
-            if (s_ex[mid] <= q) lo = mid; else hi = mid;
-        }
-        return lo;
-    };
-    if (in_lds) {
-        for (int q0 = t; q0 < tot; q0 += kSortBatch * kSortCells) {
-            int v[kSortBatch], cl[kSortBatch];
-#pragma unroll
-            for (int u = 0; u < kSortBatch; ++u) {
-                const int q = q0 + u * kSortCells;
-                if (q < tot) {
-                    cl[u] = cell_of(q);
-                    v[u] = a.tmp[(size_t)(c0 + cl[u]) * a.cap + (q - s_ex[cl[u]])];
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < kSortBatch; ++u) {
-                const int q = q0 + u * kSortCells;
-                if (q < tot) {
-                    s_ids[q] = a.uid[v[u]];
-                    s_cl[q] = (uint8_t)cl[u];
-                }
-            }
-        }
-        __syncthreads();
-    }
-    for (int q0 = t; q0 < tot; q0 += kSortBatch * kSortCells) {
-        int ii[kSortBatch], pos[kSortBatch];
+    auto store = [&](int q0, SortEntries &s, const Row &o) {
+        int pos[kSortBatch];
 #pragma unroll
         for (int u = 0; u < kSortBatch; ++u) {
-            const int q = q0 + u * kSortCells;
-            ii[u] = -1;
-            if (q < tot) {
-                const int cl = in_lds ? (int)s_cl[q] : cell_of(q);
+            if (s.i[u] >= 0) {
+                const int q = q0 + u * kSortThreads, cl = s.cl[u];
                 const int b = s_ex[cl], m = s_ex[cl + 1] - b;
                 // (caller indices are unique within a replica, whose cells
                 // these are: a strict order)
-                const int *src = a.tmp + (size_t)(c0 + cl) * a.cap;
-                const int i = src[q - b];  // the particle (internal index)
+                const int ui = s.u[u];
                 int rank = 0;
                 if (in_lds) {
-                    const int ui = s_ids[q];
+#pragma unroll 4
                     for (int k = 0; k < m; ++k) rank += (s_ids[b + k] < ui);
                 } else {
-                    const int ui = a.uid[i];
+                    const int *src = a.tmp + (size_t)(c0 + cl) * a.cap;
                     for (int k = 0; k < m; ++k) rank += (a.uid[src[k]] < ui);
                 }
-                ii[u] = i;
-                pos[u] = s_st[cl] + rank;
+                pos[u] = (s_st[cl] >= 0 ? s_st[cl] : carry + b) + rank;
                 // counts that add up past the replica's particles (a binning
                 // on top of one not yet sorted) are reported, never written
                 if (pos[u] >= s_lim[cl]) {
                     atomicOr(a.err, 1u);  // FM_DEV_CELL_OVERFLOW
-                    ii[u] = -1;
+                    s.i[u] = -1;
                 }
             }
         }
-        float4 e[kSortBatch];
-        int ty[kSortBatch];
 #pragma unroll
         for (int u = 0; u < kSortBatch; ++u) {
-            if (ii[u] >= 0) {
-                const int i = ii[u];
-                e[u].x = a.x[i];
-                e[u].y = a.y[i];
-                e[u].z = __int_as_float(a.grp[i]);
-                e[u].w = a.sig ? a.sig[i] : 0.0f;
-                ty[u] = a.typ ? a.typ[i] : 0;
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < kSortBatch; ++u) {
-            if (ii[u] >= 0) {
-                const int i = ii[u], ps = pos[u];
+            if (s.i[u] >= 0) {
+                const int i = s.i[u], ps = pos[u];
                 a.perm[ps] = i;
-                a.sorted[ps] = e[u];
-                if (a.typ) a.sorted_typ[ps] = ty[u];
+                a.sorted[ps] = o.e[u];
+                if (a.typ) a.sorted_typ[ps] = o.ty[u];
                 if (a.spos) {  // list mode: the sorted-order state the list pass reads
                     a.spos[i] = ps;
-                    a.xys[ps] = make_float2(e[u].x, e[u].y);
-                    if (a.sigs) a.sigs[ps] = e[u].w;
+                    a.xys[ps] = make_float2(o.e[u].x, o.e[u].y);
+                    if (a.sigs) a.sigs[ps] = o.e[u].w;
                 }
             }
         }
+    };
+    store(t, s0, w0);
+    for (int q0 = t + kRound; q0 < tot; q0 += kRound) {
+        SortEntries s;
+        Row o;
+        load(q0, s);
+        load_row(s, o);
+        store(q0, s, o);
     }
 }
 
@@ -3371,7 +3425,9 @@ hipError_t launch_bin(const KickArgs &a, const ElemArgs &el, hipStream_t s) {
 
 hipError_t launch_sort(const ScanArgs &a, const ElemArgs &el, hipStream_t s) {
     if (a.nsort <= 0) return hipSuccess;
-    FM_GO(k_sort, dim3(a.nsort + el.nespans + el.nbspans), dim3(kSortCells), 0, s, a, el);
+    const dim3 grid(a.nsort + el.nespans + el.nbspans);
+    if (a.cells == kSortCellsFew) FM_GO(k_sort<kSortCellsFew>, grid, dim3(kSortThreads), 0, s, a, el);
+    else FM_GO(k_sort<kSortCells>, grid, dim3(kSortThreads), 0, s, a, el);
     return hipGetLastError();
 }
 
