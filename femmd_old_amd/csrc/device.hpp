@@ -286,6 +286,22 @@ struct ElemArgs {
     uint32_t *err;
 };
 
+// The one-kernel rebuild of a single replica (k_rebuild): its binning and
+// list-build workgroups, and its words, 128 bytes apart (a ticket counter, two
+// phase counters, eight go words per phase; never reset, every rebuild adds
+// the same counts).  At most kRebuildBins workgroups bin (more of them hold
+// each other's tickets up: 114,140 particles 446 workgroups 20.3 us a step,
+// 256 20.1, 160 19.9, 96 20.06).  Taken up to kRebuildMax workgroups, about
+// what is resident at once; a step against three kernels: 256 particles 16.1
+// -> 13.3 us, 4,367 16.9 -> 14.1, 30,011 16.3 -> 13.7, 56 k with elastomers
+// 18.9 -> 16.2, 114,140 (986 workgroups) 20.5 -> 19.9.
+constexpr int kRebuildSync = 16 * (3 + 2 * 8);
+constexpr int kRebuildBins = 160, kRebuildMax = 1024;
+struct RebuildArgs {
+    unsigned long long *sync;
+    int32_t nbin, nlist;
+};
+
 struct ForceArgs {
     const RepDesc *reps;
     const PairEntry *ptab;

@@ -481,6 +481,8 @@ int Engine::build(const std::vector<const HostSystem *> &reps, std::unique_ptr<E
         }
         if ((he = upload(E->brep_, hbrep, st)) != hipSuccess) return E->check(he, "upload brep", err);
     }
+    if (E->list_ && R == 1)  // (cleared by build_tiles)
+        FM_AL(rebuild_words_, (size_t)kRebuildSync + E->nsort_);
     if (E->list_ && R > kDecideMinReps) {
         FM_AL(fspan_, std::max<size_t>(ks.size(), 1));
         FM_AL(rinfo_, R);
@@ -666,6 +668,10 @@ int Engine::build_tiles(const std::vector<int> &tile_w, std::string &err) {
     if (list_) lb_grid_ = list_build_resident(sigma_, block_, force_args(), device_);
     if ((he = upload(tiles_, tiles_h_, stream_)) != hipSuccess) return check(he, "tiles", err);
     if ((he = upload(rng_, rng_h_, stream_)) != hipSuccess) return check(he, "ranges", err);
+    // (the counters assume the same workgroups at every rebuild)
+    if (rebuild_words_.p && (he = hipMemsetAsync(rebuild_words_.p, 0, rebuild_words_.n *
+                                                 sizeof(unsigned long long), stream_)) != hipSuccess)
+        return check(he, "rebuild counters", err);
     if (list_ && R_ > kDecideMinReps &&
         (he = ftile_.alloc(std::max<size_t>(tiles_h_.size(), 1))) != hipSuccess)
         return check(he, "tile list", err);
@@ -724,13 +730,7 @@ int Engine::set_tuning(int tile_w, int block, int use_graph, std::string &err) {
 // ---------------------------------------------------------------------------
 // Binning of the positions the force pass reads (xcur); gated = list mode,
 // only the replicas whose rebuild flag is set.
-int Engine::launch_bin(bool gated) {
-    if (!gated && bins_pending_) {
-        // a drift's binning no sort consumed (a run broken off after a body):
-        // start from empty cells
-        if (launch_fill_int(count_.p, 0, (size_t)ncells_, stream_) != hipSuccess) return -1;
-        bins_pending_ = false;
-    }
+KickArgs Engine::bin_args(bool gated) {
     KickArgs a{};
     a.reps = reps_.p;
     a.spans = kspans_.p;
@@ -743,36 +743,64 @@ int Engine::launch_bin(bool gated) {
     a.nspans = (int)kspans_h_.size();
     a.obs = obs_args(true);
     a.obs_l1 = (gated && l1_) ? 1 : 0;
-    ElemArgs el{};  // a step's element and bond forces beside its gated binning
-    if (gated) el = elem_args();
     if (gated) {  // list mode: decide and bin only the replicas that rebuild
         a.ctl = ctl_.p;
         a.any = any_.p;
         a.dmax = dmax_cur();  // the drift that produced the current positions
         a.one_rep = R_ == 1;
         a.rblog = R_ == 1 ? rblog_ : nullptr;
-        if (R_ > kDecideMinReps) {
-            DecideArgs d{};
-            d.reps = reps_.p;
-            d.ctl = ctl_.p;
-            d.dmax = dmax_cur();
-            d.rng = rng_.p;
-            d.nrep = R_;
-            d.any = any_.p;
-            d.fspan = fspan_.p;
-            d.ftile = ftile_.p;
-            d.fblock = fblock_.p;
-            d.nsort = nsort_;
-            d.sort_cells = sort_cells_;
-            d.nf = nf_.p;
-            d.rinfo = rinfo_.p;
-            d.mark = mark_.p;
-            if (launch_decide(d, stream_) != hipSuccess) return -1;
-            a.fspan = fspan_.p;
-            a.nfs = nf_.p;
-        }
+    }
+    return a;
+}
+
+int Engine::launch_bin(bool gated) {
+    if (!gated && bins_pending_) {
+        // a drift's binning no sort consumed (a run broken off after a body):
+        // start from empty cells
+        if (launch_fill_int(count_.p, 0, (size_t)ncells_, stream_) != hipSuccess) return -1;
+        bins_pending_ = false;
+    }
+    KickArgs a = bin_args(gated);
+    ElemArgs el{};  // a step's element and bond forces beside its gated binning
+    if (gated) el = elem_args();
+    if (gated && R_ > kDecideMinReps) {
+        DecideArgs d{};
+        d.reps = reps_.p;
+        d.ctl = ctl_.p;
+        d.dmax = dmax_cur();
+        d.rng = rng_.p;
+        d.nrep = R_;
+        d.any = any_.p;
+        d.fspan = fspan_.p;
+        d.ftile = ftile_.p;
+        d.fblock = fblock_.p;
+        d.nsort = nsort_;
+        d.sort_cells = sort_cells_;
+        d.nf = nf_.p;
+        d.rinfo = rinfo_.p;
+        d.mark = mark_.p;
+        if (launch_decide(d, stream_) != hipSuccess) return -1;
+        a.fspan = fspan_.p;
+        a.nfs = nf_.p;
     }
     return ::fm::launch_bin(a, el, stream_) == hipSuccess ? 0 : -1;
+}
+
+// Whether a step takes its gated binning, sort and list build as one kernel:
+// a single replica with 256-thread tiles and at most kRebuildMax workgroups
+// (profile() times the three apart).
+bool Engine::one_rebuild() const {
+    if (!list_ || R_ != 1 || block_ != 256 || sort_cells_ != kSortCellsFew || prof_ev_) return false;
+    const RebuildArgs r = rebuild_args();
+    return r.nbin + nsort_ + r.nlist <= kRebuildMax;
+}
+
+RebuildArgs Engine::rebuild_args() const {
+    RebuildArgs r{};
+    r.sync = rebuild_words_.p;
+    r.nbin = std::min((int)kspans_h_.size(), kRebuildBins);
+    r.nlist = (int)tiles_h_.size();
+    return r;
 }
 
 // The kick arguments shared by the first half-kick of a run (every
@@ -844,12 +872,20 @@ int Engine::launch_step_body(bool kick2, bool drift, bool energy, bool l1, bool 
     if (list_) {
         // binning, sort and list build run only for the replicas where some
         // particle moved more than skin / 2 since the last build
-        time_next(1);
-        const int bad = launch_bin(true);
-        arm_kernel_timer(nullptr, nullptr);
-        if (bad) return -1;
-        if (launch_sort(true)) return -1;
-        if (launch_list_build(true)) return -1;
+        if (one_rebuild()) {
+            ScanArgs sa = sort_args(true);
+            sa.status2 = rebuild_words_.p + kRebuildSync;
+            if (launch_rebuild(sigma_, bin_args(true), elem_args(), sa, force_args(), rebuild_args(),
+                               stream_) != hipSuccess)
+                return -1;
+        } else {
+            time_next(1);
+            const int bad = launch_bin(true);
+            arm_kernel_timer(nullptr, nullptr);
+            if (bad) return -1;
+            if (launch_sort(true)) return -1;
+            if (launch_list_build(true)) return -1;
+        }
     } else {
         if (launch_sort(false, true)) return -1;  // the binning of the last drift
     }
@@ -880,7 +916,7 @@ int Engine::launch_step_body(bool kick2, bool drift, bool energy, bool l1, bool 
 }
 
 // Counting sort of the last binning (single pass: scan and scatter).
-int Engine::launch_sort(bool gated, bool elems) {
+ScanArgs Engine::sort_args(bool gated) {
     ScanArgs s{};
     s.reps = reps_.p;
     s.nrep = R_;
@@ -911,6 +947,11 @@ int Engine::launch_sort(bool gated, bool elems) {
         s.xys = xys_cur();
         s.sigs = sigma_ ? sigs_.p : nullptr;
     }
+    return s;
+}
+
+int Engine::launch_sort(bool gated, bool elems) {
+    ScanArgs s = sort_args(gated);
     if (gated) {
         s.ctl = ctl_.p;
         s.any = any_.p;

@@ -195,6 +195,10 @@ private:
     // every sort writes the sorted-order state; a sort that no list build
     // follows must leave primed_ false.
     int launch_bin(bool gated = false);
+    KickArgs bin_args(bool gated);
+    ScanArgs sort_args(bool gated);
+    bool one_rebuild() const;
+    RebuildArgs rebuild_args() const;
     // One step body: kick2 (second half-kick of the previous step, with the
     // kinetic-energy partials when energy is set), drift (first half-kick,
     // drift, wrap), then the neighbour update and the force pass (pair
@@ -362,6 +366,7 @@ private:
     DBuf<int4> rinfo_;
     DBuf<uint8_t> mark_;
     DBuf<unsigned long long> sort_status2_;     // status words of the listed sort
+    DBuf<unsigned long long> rebuild_words_;    // one-kernel rebuild: RebuildArgs::sync, its sort's status words
     DBuf<int2> brep_;                   // per sort block: replica range
     DBuf<uint32_t> ro_tmp_;
     DBuf<int32_t> count_, tmp_, start_, perm_, sorted_typ_;
@@ -444,6 +449,8 @@ hipError_t launch_list_build(bool sigma, int block, const ForceArgs &a, hipStrea
 size_t list_build_lds_bytes(int lds_cap, int cell_cap, int nbr_cap, int block, bool sigma,
                             bool buffered);
 int list_build_resident(bool sigma, int block, const ForceArgs &a, int device);
+hipError_t launch_rebuild(bool sigma, const KickArgs &a, const ElemArgs &el, const ScanArgs &sa,
+                          const ForceArgs &f, const RebuildArgs &rb, hipStream_t s);
 hipError_t launch_ctl_reset(Ctl *ctl, int nrep, uint32_t *dmax, int nslots, hipStream_t s);
 size_t forces_lds_bytes(int lds_cap, bool types, bool debug);
 // err, report: if set, the error word is also written there (pinned memory)

@@ -315,6 +315,36 @@ __device__ void obs_finish(const ObsArgs &o, int r, bool accumulate) {
 // run and hand out slots by lane offset.  Slot order within a cell is not
 // deterministic; the scatter below orders each cell by particle index.
 // All 64 lanes of the wavefront must call this (ballot / shuffles).
+// A store for later kernels (kept in this XCD's L2 until they start), or
+// (kThrough) written through to where every XCD reads it, for workgroups of
+// the same kernel.
+template <bool kThrough>
+__device__ __forceinline__ void put(int32_t *p, int32_t v) {
+    if (kThrough) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else *p = v;
+}
+template <bool kThrough>
+__device__ __forceinline__ void put(float *p, float v) {
+    put<kThrough>(reinterpret_cast<int32_t *>(p), __float_as_int(v));
+}
+template <bool kThrough>
+__device__ __forceinline__ void put(float2 *p, float2 v) {
+    if (kThrough)
+        __hip_atomic_store(reinterpret_cast<unsigned long long *>(p),
+                           (unsigned long long)__float_as_uint(v.y) << 32 | __float_as_uint(v.x),
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else *p = v;
+}
+template <bool kThrough>
+__device__ __forceinline__ void put(float4 *p, float4 v) {
+    if (kThrough) {
+        float2 *q = reinterpret_cast<float2 *>(p);
+        put<true>(q, make_float2(v.x, v.y));
+        put<true>(q + 1, make_float2(v.z, v.w));
+    } else *p = v;
+}
+
+template <bool kThrough = false>
 __device__ __forceinline__ void bin_wave_to(int32_t *count, int32_t *tmp, int cap, uint32_t *err,
                                             bool active, int p, int c) {
     const int lane = threadIdx.x & 63;
@@ -331,12 +361,13 @@ __device__ __forceinline__ void bin_wave_to(int32_t *count, int32_t *tmp, int ca
     base = __shfl(base, h);
     if (active) {
         const int slot = base + (lane - h);
-        if (slot < cap) tmp[(size_t)c * cap + slot] = p;
+        if (slot < cap) put<kThrough>(tmp + (size_t)c * cap + slot, p);
         else atomicOr(err, 1u);  // FM_DEV_CELL_OVERFLOW (the particle is dropped)
     }
 }
+template <bool kThrough = false>
 __device__ __forceinline__ void bin_wave(const KickArgs &a, bool active, int p, int c) {
-    bin_wave_to(a.count, a.tmp, a.cap, a.err, active, p, c);
+    bin_wave_to<kThrough>(a.count, a.tmp, a.cap, a.err, active, p, c);
 }
 
 // The velocity-Verlet kick of one particle (femmd2D/src/integrator.cpp:
@@ -840,6 +871,40 @@ __global__ __launch_bounds__(kElemThreads) void k_elems(ElemArgs a) {
     elem_role(a, blockIdx.x, red);
 }
 
+// The particles of a span into their cells' slot lists.
+template <bool kThrough = false>
+__device__ __forceinline__ void bin_span(const KickArgs &a, const Span &sp, const RepDesc &R) {
+    const int p = sp.begin + (int)threadIdx.x;
+    const bool active = p < sp.end;
+    int c = 0;
+    if (active) {
+        float x = a.x[p], y = a.y[p];
+        if (!(isfinite(x) && isfinite(y))) {
+            atomicOr(a.err, 8u);
+            x = 0.0f;
+            y = 0.0f;
+        }
+        c = R.cell0 + cell_key(x, y, R);
+    }
+    bin_wave<kThrough>(a, active, p, c);
+}
+
+// A single replica's rebuild decision, from its descriptor and displacement
+// slots loaded together; `record` (one workgroup): as list_decide records it.
+__device__ __forceinline__ int one_rep_decide(const KickArgs &a, bool record) {
+    const RepDesc &R0 = a.reps[0];
+    const int flag = list_disp(a.dmax, a.ctl, 0, R0) > 0.5f * R0.skin;
+    if (record && threadIdx.x == 0) {
+        a.ctl->flag = flag;
+        if (flag) {
+            a.ctl->nbuild += 1u;
+            *a.any = 1;
+        }
+        if (a.rblog) *a.rblog = flag;  // (adjoint recording)
+    }
+    return flag;
+}
+
 __global__ __launch_bounds__(kKickThreads) void k_bin(KickArgs a, ElemArgs el) {
   __shared__ double ored[kObsRed];
   // the step's element and bond forces, by workgroups of their own: they
@@ -857,16 +922,7 @@ __global__ __launch_bounds__(kKickThreads) void k_bin(KickArgs a, ElemArgs el) {
       // a single replica: the decision comes first, from the replica's
       // descriptor and displacement slots loaded together (no span read
       // before them), so that a step without a rebuild leaves at once
-      const RepDesc &R0 = a.reps[0];
-      flag = list_disp(a.dmax, a.ctl, 0, R0) > 0.5f * R0.skin;
-      if (wb == 0 && threadIdx.x == 0) {  // as list_decide records it
-          a.ctl->flag = flag;
-          if (flag) {
-              a.ctl->nbuild += 1u;
-              *a.any = 1;
-          }
-          if (a.rblog) *a.rblog = flag;  // (adjoint recording)
-      }
+      flag = one_rep_decide(a, wb == 0);
       if (!flag) return;
       last_rep = 0;
   }
@@ -887,19 +943,7 @@ __global__ __launch_bounds__(kKickThreads) void k_bin(KickArgs a, ElemArgs el) {
             continue;
         }
     }
-    const int p = sp.begin + (int)threadIdx.x;
-    const bool active = p < sp.end;
-    int c = 0;
-    if (active) {
-        float x = a.x[p], y = a.y[p];
-        if (!(isfinite(x) && isfinite(y))) {
-            atomicOr(a.err, 8u);
-            x = 0.0f;
-            y = 0.0f;
-        }
-        c = R.cell0 + cell_key(x, y, R);
-    }
-    bin_wave(a, active, p, c);
+    bin_span(a, sp, R);
   }
 }
 
@@ -1003,54 +1047,27 @@ struct SortEntries {
     uint8_t cl[kSortBatch];            // its cell (local index)
 };
 
+// LDS of a sort workgroup.
 template <int CELLS>
-__global__ __launch_bounds__(kSortThreads) void k_sort(ScanArgs a, ElemArgs el) {
-    constexpr int kIds = CELLS * kSortFill;
-    __shared__ int s_ex[CELLS + 1];   // local exclusive prefix of the counts
-    __shared__ int s_st[CELLS];       // cell starts (-1: the carry-in + s_ex)
-    __shared__ int s_lim[CELLS];      // end of each cell's replica range
-    __shared__ int s_w[CELLS / 64];
-    __shared__ unsigned long long s_tk;
-    __shared__ int s_carry, s_head, s_flag;
-    __shared__ int s_ids[kIds];       // the block's slot entries' caller indices, cell order
-    __shared__ double s_ored[kObsRed];
-    // (cell walk) the step's element and bond forces, by the workgroups past
-    // the sort's, and the previous step's observables, level 1, before the
-    // ticket: no workgroup waits on one that has not taken its ticket
-    if ((int)blockIdx.x >= a.nsort) {
-        elem_role(el, (int)blockIdx.x - a.nsort, s_ored);
-        return;
-    }
-    if (a.obs_l1) obs_level1(a.obs, blockIdx.x, a.nsort, s_ored);
-    if (a.any && !*a.any) return;  // list mode, no replica rebuilds (uniform)
+struct SortLds {
+    static constexpr int kIds = CELLS * kSortFill;
+    int ex[CELLS + 1];  // local exclusive prefix of the counts
+    int st[CELLS];      // cell starts (-1: the carry-in + ex)
+    int lim[CELLS];     // end of each cell's replica range
+    int w[CELLS / 64];
+    int carry, head, flag;
+    unsigned long long tk;
+    int ids[kIds];      // the block's slot entries' caller indices, cell order
+};
+
+// Block b: counts, scans, publishes and scatters its cells (every thread of
+// a workgroup of kSortThreads).  kThrough: see put.
+template <int CELLS, bool kThrough = false>
+__device__ __forceinline__ void sort_block(const ScanArgs &a, int b, uint32_t epoch,
+                                           unsigned long long *status, SortLds<CELLS> &S) {
+    constexpr int kIds = SortLds<CELLS>::kIds;
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    // listed (gated batches): workgroups beyond the listed blocks leave at
-    // once, so only the listed blocks take tickets; they take the blocks in
-    // ticket order, with the step's epoch and a status array of their own
-    const bool listed = a.fblock != nullptr;
-    if (listed && (int)blockIdx.x >= a.nf[2]) return;
-    if (t == 0)
-        s_tk = listed ? (unsigned long long)atomicAdd(a.nf + 3, 1) : atomicAdd(a.ticket, 1ull);
-    __syncthreads();
-    const unsigned long long tk = s_tk;
-    const int b = listed ? a.fblock[tk] : (int)(tk % (unsigned long long)a.nsort);
-    const uint32_t epoch =
-        listed ? (uint32_t)a.nf[4] : (uint32_t)(tk / (unsigned long long)a.nsort);
-    unsigned long long *const status = listed ? a.status2 : a.status;
     const int c0 = b * CELLS;
-    if (a.ctl && !listed) {
-        // gated (list mode): a block holding no cell of a rebuilding replica
-        // has nothing to count, scan or scatter, and no rebuilding replica
-        // looks back past its own first block, so it is skipped whole
-        if (t == 0) {
-            const int2 br = a.brep[b];
-            int f = 0;
-            for (int q = br.x; q <= br.y; ++q) f |= a.ctl[q].flag;
-            s_flag = f;
-        }
-        __syncthreads();
-        if (!s_flag) return;
-    }
     // thread t counts cell c (the threads past the cells take the last one's
     // replica and count nothing)
     const int c = c0 + min(t, CELLS - 1);
@@ -1067,29 +1084,29 @@ __global__ __launch_bounds__(kSortThreads) void k_sort(ScanArgs a, ElemArgs el) 
     const int incl = wave_incl_scan(n);
     int ex = incl - n;
     if (CELLS > 64) {
-        if (lane == 63) s_w[w] = incl;
+        if (lane == 63) S.w[w] = incl;
         __syncthreads();
-        for (int k = 0; k < w; ++k) ex += s_w[k];
+        for (int k = 0; k < w; ++k) ex += S.w[k];
     }
     if (t < CELLS) {
-        s_ex[t] = ex;
-        s_lim[t] = R.p1;
+        S.ex[t] = ex;
+        S.lim[t] = R.p1;
     }
     if (t == CELLS - 1) {
-        s_ex[CELLS] = ex + n;
-        s_head = hl >= 0;
+        S.ex[CELLS] = ex + n;
+        S.head = hl >= 0;
     }
     __syncthreads();
-    const int tot = s_ex[CELLS];
+    const int tot = S.ex[CELLS];
     // publish (the last cell's replica decides: its first cell in this block
     // means the block's end value is known without look-back)
     if (t == CELLS - 1) {
         const unsigned long long v = (hl >= 0)
-            ? lb_word(epoch, kLbInclusive, R.p0 + tot - s_ex[hl])
+            ? lb_word(epoch, kLbInclusive, R.p0 + tot - S.ex[hl])
             : lb_word(epoch, kLbAggregate, tot);
         __hip_atomic_store(status + b, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    if (t < CELLS) s_st[t] = hl >= 0 ? R.p0 + ex - s_ex[hl] : -1;
+    if (t < CELLS) S.st[t] = hl >= 0 ? R.p0 + ex - S.ex[hl] : -1;
     // scatter: the block's particles in cell order; a particle's sorted
     // position is its cell's start + its rank among the cell's members by
     // their index in the caller's order, as the reference's cell fill walks
@@ -1108,9 +1125,9 @@ __global__ __launch_bounds__(kSortThreads) void k_sort(ScanArgs a, ElemArgs el) 
                 int lo = 0;
 #pragma unroll
                 for (int h = CELLS / 2; h > 0; h >>= 1)
-                    if (s_ex[lo + h] <= q) lo += h;
+                    if (S.ex[lo + h] <= q) lo += h;
                 s.cl[u] = (uint8_t)lo;
-                s.i[u] = a.tmp[(size_t)(c0 + lo) * a.cap + (q - s_ex[lo])];
+                s.i[u] = a.tmp[(size_t)(c0 + lo) * a.cap + (q - S.ex[lo])];
             }
         }
 #pragma unroll
@@ -1144,13 +1161,13 @@ __global__ __launch_bounds__(kSortThreads) void k_sort(ScanArgs a, ElemArgs el) 
     if (in_lds) {
 #pragma unroll
         for (int u = 0; u < kSortBatch; ++u)
-            if (s0.i[u] >= 0) s_ids[t + u * kSortThreads] = s0.u[u];
+            if (s0.i[u] >= 0) S.ids[t + u * kSortThreads] = s0.u[u];
         for (int q0 = t + kRound; q0 < tot; q0 += kRound) {
             SortEntries s;
             load(q0, s);
 #pragma unroll
             for (int u = 0; u < kSortBatch; ++u)
-                if (s.i[u] >= 0) s_ids[q0 + u * kSortThreads] = s.u[u];
+                if (s.i[u] >= 0) S.ids[q0 + u * kSortThreads] = s.u[u];
         }
     }
     if (w == 0) {
@@ -1160,43 +1177,43 @@ __global__ __launch_bounds__(kSortThreads) void k_sort(ScanArgs a, ElemArgs el) 
         const bool need = __builtin_amdgcn_readfirstlane((hl >= 0 || (a.ctl && !a.ctl[r].flag)) ? 0 : 1);
         const int carry = need ? sort_look_back(status, b, epoch, a.err) : 0;
         if (lane == 0) {
-            s_carry = carry;
-            if (need && !s_head)  // a block holding a replica's first cell published already
+            S.carry = carry;
+            if (need && !S.head)  // a block holding a replica's first cell published already
                 __hip_atomic_store(status + b, lb_word(epoch, kLbInclusive, carry + tot),
                                    __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
     __syncthreads();
-    const int carry = s_carry;
+    const int carry = S.carry;
     if (mine) {
-        const int st = s_st[t] >= 0 ? s_st[t] : carry + ex;
+        const int st = S.st[t] >= 0 ? S.st[t] : carry + ex;
         // list mode: only the rebuilding replicas' cell starts change (the
         // others' lists index staging laid out by their own last starts)
-        if (!a.ctl || a.ctl[r].flag) a.start[c] = st;
-        if (c == a.ncells - 1) a.start[a.ncells] = st + n;
+        if (!a.ctl || a.ctl[r].flag) put<kThrough>(a.start + c, st);
+        if (c == a.ncells - 1) put<kThrough>(a.start + a.ncells, st + n);
     }
-    auto store = [&](int q0, SortEntries &s, const Row &o) {
+    auto store = [&](SortEntries &s, const Row &o) {
         int pos[kSortBatch];
 #pragma unroll
         for (int u = 0; u < kSortBatch; ++u) {
             if (s.i[u] >= 0) {
-                const int q = q0 + u * kSortThreads, cl = s.cl[u];
-                const int b = s_ex[cl], m = s_ex[cl + 1] - b;
+                const int cl = s.cl[u];
+                const int b = S.ex[cl], m = S.ex[cl + 1] - b;
                 // (caller indices are unique within a replica, whose cells
                 // these are: a strict order)
                 const int ui = s.u[u];
                 int rank = 0;
                 if (in_lds) {
 #pragma unroll 4
-                    for (int k = 0; k < m; ++k) rank += (s_ids[b + k] < ui);
+                    for (int k = 0; k < m; ++k) rank += (S.ids[b + k] < ui);
                 } else {
                     const int *src = a.tmp + (size_t)(c0 + cl) * a.cap;
                     for (int k = 0; k < m; ++k) rank += (a.uid[src[k]] < ui);
                 }
-                pos[u] = (s_st[cl] >= 0 ? s_st[cl] : carry + b) + rank;
+                pos[u] = (S.st[cl] >= 0 ? S.st[cl] : carry + b) + rank;
                 // counts that add up past the replica's particles (a binning
                 // on top of one not yet sorted) are reported, never written
-                if (pos[u] >= s_lim[cl]) {
+                if (pos[u] >= S.lim[cl]) {
                     atomicOr(a.err, 1u);  // FM_DEV_CELL_OVERFLOW
                     s.i[u] = -1;
                 }
@@ -1206,25 +1223,67 @@ __global__ __launch_bounds__(kSortThreads) void k_sort(ScanArgs a, ElemArgs el) 
         for (int u = 0; u < kSortBatch; ++u) {
             if (s.i[u] >= 0) {
                 const int i = s.i[u], ps = pos[u];
-                a.perm[ps] = i;
-                a.sorted[ps] = o.e[u];
-                if (a.typ) a.sorted_typ[ps] = o.ty[u];
+                put<kThrough>(a.perm + ps, i);
+                put<kThrough>(a.sorted + ps, o.e[u]);
+                if (a.typ) put<kThrough>(a.sorted_typ + ps, o.ty[u]);
                 if (a.spos) {  // list mode: the sorted-order state the list pass reads
-                    a.spos[i] = ps;
-                    a.xys[ps] = make_float2(o.e[u].x, o.e[u].y);
-                    if (a.sigs) a.sigs[ps] = o.e[u].w;
+                    put<kThrough>(a.spos + i, ps);
+                    put<kThrough>(a.xys + ps, make_float2(o.e[u].x, o.e[u].y));
+                    if (a.sigs) put<kThrough>(a.sigs + ps, o.e[u].w);
                 }
             }
         }
     };
-    store(t, s0, w0);
+    store(s0, w0);
     for (int q0 = t + kRound; q0 < tot; q0 += kRound) {
         SortEntries s;
         Row o;
         load(q0, s);
         load_row(s, o);
-        store(q0, s, o);
+        store(s, o);
     }
+}
+template <int CELLS>
+__global__ __launch_bounds__(kSortThreads) void k_sort(ScanArgs a, ElemArgs el) {
+    __shared__ SortLds<CELLS> S;
+    __shared__ double s_ored[kObsRed];
+    // (cell walk) the step's element and bond forces, by the workgroups past
+    // the sort's, and the previous step's observables, level 1, before the
+    // ticket: no workgroup waits on one that has not taken its ticket
+    if ((int)blockIdx.x >= a.nsort) {
+        elem_role(el, (int)blockIdx.x - a.nsort, s_ored);
+        return;
+    }
+    if (a.obs_l1) obs_level1(a.obs, blockIdx.x, a.nsort, s_ored);
+    if (a.any && !*a.any) return;  // list mode, no replica rebuilds (uniform)
+    const int t = threadIdx.x;
+    // listed (gated batches): workgroups beyond the listed blocks leave at
+    // once, so only the listed blocks take tickets; they take the blocks in
+    // ticket order, with the step's epoch and a status array of their own
+    const bool listed = a.fblock != nullptr;
+    if (listed && (int)blockIdx.x >= a.nf[2]) return;
+    if (t == 0)
+        S.tk = listed ? (unsigned long long)atomicAdd(a.nf + 3, 1) : atomicAdd(a.ticket, 1ull);
+    __syncthreads();
+    const unsigned long long tk = S.tk;
+    const int b = listed ? a.fblock[tk] : (int)(tk % (unsigned long long)a.nsort);
+    const uint32_t epoch =
+        listed ? (uint32_t)a.nf[4] : (uint32_t)(tk / (unsigned long long)a.nsort);
+    unsigned long long *const status = listed ? a.status2 : a.status;
+    if (a.ctl && !listed) {
+        // gated (list mode): a block holding no cell of a rebuilding replica
+        // has nothing to count, scan or scatter, and no rebuilding replica
+        // looks back past its own first block, so it is skipped whole
+        if (t == 0) {
+            const int2 br = a.brep[b];
+            int f = 0;
+            for (int q = br.x; q <= br.y; ++q) f |= a.ctl[q].flag;
+            S.flag = f;
+        }
+        __syncthreads();
+        if (!S.flag) return;
+    }
+    sort_block<CELLS>(a, b, epoch, status, S);
 }
 
 // ---------------------------------------------------------------------------
@@ -2065,11 +2124,10 @@ __device__ void store_run(TileRun *o, const Tile &T, const RepDesc &R, int W, co
     o->d2[r] = b2 < row ? L.cstart[s0 + b2] - L.off[s0 + b2] : 0;
 }
 
+// The tiles b0, b0 + nb, ... of the list build (every thread of a workgroup).
 template <bool kSigma>
-__global__ __launch_bounds__(256) void k_list_build(ForceArgs a) {
-    extern __shared__ float4 dyn[];
-    __shared__ int s_cstart[kMaxSlots];
-    __shared__ int s_off[kMaxSlots + 1];
+__device__ __forceinline__ void list_tiles(const ForceArgs &a, int b0, int nb, float4 *dyn, int *s_cstart,
+                                           int *s_off) {
     PairLds L;
     L.ent = nullptr;
     L.typ = nullptr;
@@ -2087,10 +2145,9 @@ __global__ __launch_bounds__(256) void k_list_build(ForceArgs a) {
     B.sig = reinterpret_cast<float *>(B.grp + slots);
     uint32_t *mask = reinterpret_cast<uint32_t *>(B.grp + (kSigma ? 2 : 1) * slots);
     int *hist = reinterpret_cast<int *>(mask + 3 * list_build_words(a.cell_cap) * blockDim.x);
-    if (a.ctl && a.any && !*a.any) return;  // gated, and no replica rebuilds
     // gated batches walk the listed tiles of the rebuilding replicas
     const int nt = a.ftile ? *a.nft : a.ntiles;
-    for (int b = blockIdx.x; b < nt; b += gridDim.x) {
+    for (int b = b0; b < nt; b += nb) {
         const int tile = a.ftile ? a.ftile[xcd_remap(b, nt)] : xcd_remap(b, nt);
         const Tile T = a.tiles[tile];
         if (a.ctl && !a.ftile && !a.ctl[T.rep].flag) continue;  // uniform per workgroup
@@ -2121,6 +2178,107 @@ __global__ __launch_bounds__(256) void k_list_build(ForceArgs a) {
         }
         __syncthreads();  // the next tile restages the LDS
     }
+}
+template <bool kSigma>
+__global__ __launch_bounds__(256) void k_list_build(ForceArgs a) {
+    extern __shared__ float4 dyn[];
+    __shared__ int s_cstart[kMaxSlots];
+    __shared__ int s_off[kMaxSlots + 1];
+    if (a.ctl && a.any && !*a.any) return;  // gated, and no replica rebuilds
+    list_tiles<kSigma>(a, blockIdx.x, gridDim.x, dyn, s_cstart, s_off);
+}
+
+// ---------------------------------------------------------------------------
+// A single replica's rebuild in one kernel: workgroups of the binning, the
+// sort and the list build, taken in that order from a ticket counter, each
+// kind starting its work when the one before is done.  On a step without a
+// rebuild (most) every workgroup leaves at the decision, so such a step
+// launches one kernel where it launched three (each skipped one 1.5 us in a
+// replayed graph).  A workgroup waits only for lower tickets, whose
+// workgroups are already running, so no wait depends on how many are resident
+// at once; the waits are bounded all the same.  What one phase hands to the
+// next is written through (put): releasing it with a fence, which writes the
+// whole L2 back, took a rebuild of 23 k particles from 28 to 43 us, and of
+// 114,140 from 57 to 97.  The step's element and bond forces and the previous
+// step's level-1 observables, which the binning carries, come first and wait
+// for nothing.
+// ---------------------------------------------------------------------------
+// One more of the n workgroups of phase k done, once its writes for the next
+// phase (written through) have arrived: every wavefront waits for its own.
+// The last one gives the go, in eight words on lines of their own (the
+// workgroups that wait poll those: polled together with the counter, they
+// held its adds up).
+__device__ __forceinline__ void phase_done(unsigned long long *sync, int k, unsigned long long epoch, int n) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    const unsigned long long m = __hip_atomic_fetch_add(sync + 16 * (1 + k), 1ull, __ATOMIC_RELAXED,
+                                                        __HIP_MEMORY_SCOPE_AGENT);
+    if (m + 1 == (epoch + 1) * n)
+        for (int x = 0; x < 8; ++x)
+            __hip_atomic_store(sync + 16 * (3 + 8 * k + x), epoch + 1, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+}
+// Waits for phase k's go, then sees its writes.  False: the wait ran out
+// (uniform).
+__device__ __forceinline__ bool phase_wait(unsigned long long *sync, int k, unsigned long long epoch,
+                                           int *s_ok, uint32_t *err) {
+    if (threadIdx.x == 0) {
+        const unsigned long long *go = sync + 16 * (3 + 8 * k + (blockIdx.x & 7));
+        int spins = 0;
+        while (__hip_atomic_load(go, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) <= epoch &&
+               spins < kLbSpinLimit) {
+            ++spins;
+            __builtin_amdgcn_s_sleep(8);
+        }
+        *s_ok = spins < kLbSpinLimit;
+        if (!*s_ok) atomicOr(err, 32u);  // FM_DEV_SORT_STALL: never expected
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    }
+    __syncthreads();
+    return *s_ok != 0;
+}
+
+template <bool kSigma>
+__global__ __launch_bounds__(256) void k_rebuild(KickArgs a, ElemArgs el, ScanArgs sa, ForceArgs f,
+                                                 RebuildArgs rb) {
+    extern __shared__ float4 dyn[];
+    __shared__ double ored[kObsRed];
+    __shared__ int s_cstart[kMaxSlots];
+    __shared__ int s_off[kMaxSlots + 1];
+    __shared__ unsigned long long s_tk;
+    __shared__ int s_ok;
+    const int ne = el.nespans + el.nbspans;
+    if ((int)blockIdx.x < ne) {
+        elem_role(el, blockIdx.x, ored);
+        return;
+    }
+    const int wb = (int)blockIdx.x - ne;
+    if (a.obs_l1 && wb < rb.nbin) obs_level1(a.obs, wb, rb.nbin, ored);
+    if (!one_rep_decide(a, wb == 0)) return;
+    if (threadIdx.x == 0) s_tk = atomicAdd(rb.sync, 1ull);
+    __syncthreads();
+    const unsigned long long total = rb.nbin + sa.nsort + rb.nlist;
+    const unsigned long long epoch = s_tk / total;
+    int w = (int)(s_tk % total);
+    if (w < rb.nbin) {
+        const RepDesc R = a.reps[0];
+        for (int b = w; b < a.nspans; b += rb.nbin) bin_span<true>(a, a.spans[b], R);
+        phase_done(rb.sync, 0, epoch, rb.nbin);
+        return;
+    }
+    w -= rb.nbin;
+    if (w < sa.nsort) {
+        if (!phase_wait(rb.sync, 0, epoch, &s_ok, a.err)) return;
+        sort_block<kSortCellsFew, true>(sa, w, (uint32_t)epoch, sa.status2,
+                                  *reinterpret_cast<SortLds<kSortCellsFew> *>(dyn));
+        phase_done(rb.sync, 1, epoch, sa.nsort);
+        return;
+    }
+    w -= sa.nsort;
+    if (!phase_wait(rb.sync, 1, epoch, &s_ok, a.err)) return;
+    list_tiles<kSigma>(f, w, rb.nlist, dyn, s_cstart, s_off);
 }
 
 typedef uint32_t v2u __attribute__((ext_vector_type(2)));
@@ -3539,6 +3697,18 @@ hipError_t launch_list_build(bool sigma, int block, const ForceArgs &a, hipStrea
         FM_GO((k_list_build<true>), g, dim3(block), lds, s, a);
     else
         FM_GO((k_list_build<false>), g, dim3(block), lds, s, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_rebuild(bool sigma, const KickArgs &a, const ElemArgs &el, const ScanArgs &sa,
+                          const ForceArgs &f, const RebuildArgs &rb, hipStream_t s) {
+    const size_t lds = std::max(list_build_lds_bytes(f.lds_cap, f.cell_cap, f.nbr_cap, 256, sigma, f.lbuf != 0),
+                                sizeof(SortLds<kSortCellsFew>));
+    const dim3 g(el.nespans + el.nbspans + rb.nbin + sa.nsort + rb.nlist);
+    if (sigma)
+        FM_GO((k_rebuild<true>), g, dim3(256), lds, s, a, el, sa, f, rb);
+    else
+        FM_GO((k_rebuild<false>), g, dim3(256), lds, s, a, el, sa, f, rb);
     return hipGetLastError();
 }
 
