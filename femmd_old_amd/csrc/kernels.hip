@@ -3354,7 +3354,11 @@ __global__ __launch_bounds__(256) void k_cluster_props(ClusterArgs a) {
 // Cluster virial (femmd2D/src/interactions.cpp:370-382): over the pairs the
 // force pass takes (cell walk, same predicate and exclusions), for pairs
 // whose particles both belong to clusters, 1/2 f_ij . (R_ci - R_cj) with the
-// minimum image, summed per tile in FP64.
+// minimum image, summed per tile in FP64.  Bound by the serial loop over a
+// particle's three rows of cells: all of it reads LDS (a load of the cluster
+// per candidate and of its centre per pair held it: 56 k particles 66 -> 44
+// us).
+constexpr int kNoCluster = 0x7fc0c1a5;  // (a NaN no arithmetic makes)
 template <bool kSigma, bool kTypes>
 __global__ __launch_bounds__(256) void k_cluster_virial(ClusterVirialArgs A) {
     extern __shared__ float4 dyn[];
@@ -3376,13 +3380,27 @@ __global__ __launch_bounds__(256) void k_cluster_virial(ClusterVirialArgs A) {
     const Tile T = a.tiles[tile];
     const RepDesc R = a.reps[T.rep];
     const int W = T.w_flags & 0xffff;
-    if (stage_tile<kTypes, false, true>(a, T, R, W, L, nullptr, nullptr) < 0) {
+    const int M = stage_tile<kTypes, false, true>(a, T, R, W, L, nullptr, nullptr);
+    if (M < 0) {
         if (threadIdx.x == 0) {
             atomicOr(a.err, 2u);  // FM_DEV_TILE_OVERFLOW
             A.out[tile] = 0.0;
         }
         return;
     }
+    // each staged particle's cluster centre (kNoCluster: in none) in place of
+    // its id and, where none is staged, its sigma; with sigmas its cluster
+    for (int e = threadIdx.x; e < M; e += blockDim.x) {
+        const int c = A.cid[L.sp[e]];
+        if (kSigma) {
+            L.sp[e] = c;
+        } else {
+            const float2 m = c >= 0 ? A.cm[c] : make_float2(__int_as_float(kNoCluster), 0.0f);
+            L.ent[e].w = m.x;
+            L.sp[e] = __float_as_int(m.y);
+        }
+    }
+    __syncthreads();
     const bool wrapT = (T.w_flags >> 16) & 1;
     const int row = W + 2;
     const int c_lo = L.off[row + 1], c_hi = L.off[row + W + 1];
@@ -3392,27 +3410,27 @@ __global__ __launch_bounds__(256) void k_cluster_virial(ClusterVirialArgs A) {
     double acc = 0.0, dummy = 0.0;
     for (int k = threadIdx.x; k < nc; k += blockDim.x) {
         const int me = c_lo + k;
-        const int ci = A.cid[L.sp[me]];
-        if (ci < 0) continue;
+        const int ci = L.sp[me];
+        const float4 pi = L.ent[me];
+        if (kSigma ? ci < 0 : __float_as_int(pi.w) == kNoCluster) continue;
         int lo = row + 1, hi = row + W + 1;
         while (hi - lo > 1) {
             const int mid = (lo + hi) >> 1;
             if (L.off[mid] <= me) lo = mid; else hi = mid;
         }
         const int col = lo - row;
-        const float4 pi = L.ent[me];
         const float xi = pi.x, yi = pi.y, xim = xi - Lx, yim = yi - Ly;
         const int gi = __float_as_int(pi.z);
         const int gix = gi >= 0 ? gi : -2;
         const float si = pi.w;
         const int ti = kTypes ? L.typ[me] : 0;
-        const float2 Ri = A.cm[ci];
+        const float2 Ri = kSigma ? A.cm[ci] : make_float2(pi.w, __int_as_float(ci));
         for (int r = 0; r < 3; ++r) {
             const int j0 = L.off[r * row + col - 1], j1 = L.off[r * row + col + 2];
             for (int j = j0; j < j1; ++j) {
-                const int cj = A.cid[L.sp[j]];
-                if (cj < 0) continue;
+                const int cj = L.sp[j];
                 const float4 pj = L.ent[j];
+                if (kSigma ? cj < 0 : __float_as_int(pj.w) == kNoCluster) continue;
                 float dx = xi - pj.x, dy = yi - pj.y;
                 int sx = 0, sy = 0;
                 if (wrapT) {
@@ -3442,7 +3460,7 @@ __global__ __launch_bounds__(256) void k_cluster_virial(ClusterVirialArgs A) {
                 const float sr6 = sr2 * sr2 * sr2;
                 const float tv = __builtin_fmaf(-0.5f, sr6, sr6 * sr6);
                 const float fc = pe.e48 * tv * inv;
-                const float2 Rj = A.cm[cj];
+                const float2 Rj = kSigma ? A.cm[cj] : make_float2(pj.w, __int_as_float(cj));
                 float ddx = Ri.x - Rj.x, ddy = Ri.y - Rj.y;
                 ddx = (ddx >= hLx) ? ddx - Lx : ((ddx < -hLx) ? ddx + Lx : ddx);
                 ddy = (ddy >= hLy) ? ddy - Ly : ((ddy < -hLy) ? ddy + Ly : ddy);
