@@ -114,7 +114,6 @@ int Engine::adj_kick(bool accumulate, bool drift, bool make_w, float c) {
     k.jy = jy_.p;
     k.cfa = cfa_.p;
     k.goff = gather_ ? goff_.p : nullptr;
-    k.gent = gent_.p;
     k.inv_m = inv_m_.p;
     k.w = w_.p;
     k.c = c;
@@ -172,7 +171,7 @@ int Engine::adjoint_op(const float *wx, const float *wy, float *jx, float *jy, d
     rc = adj_pass(err);
     if (rc) return rc;
     primed_ = false;  // the forward force buffers were not refreshed
-    rc = io_force_out(0, jx_.p, jy_.p, cfa_.p, gent_.p, jx, jy, err);
+    rc = io_force_out(0, jx_.p, jy_.p, cfa_.p, jx, jy, err);
     if (rc) return rc;
     return adj_grads(dE, deps, dsig, err);
 }

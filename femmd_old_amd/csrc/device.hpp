@@ -375,7 +375,7 @@ struct AdjArgs {
     ForceArgs f;          // forward inputs (binning, tiles, elements, bonds)
     const float2 *w;      // w per particle, internal order
     float *jx, *jy;       // pair part of J w, internal order
-    float2 *cfa;          // element / bond corner parts of J w
+    float2 *cfa;          // element / bond corner parts of J w, in gather order
     const float *eE;      // Young's modulus per element (forces are linear in E)
     double *dE;           // per element: += w . f_e / E_e
     double *pacc;         // per tile: += sum_i w_i . f_i / eps, += w . df/dsigma
@@ -389,7 +389,7 @@ struct AdjKickArgs {
     float *xbx, *xby, *vbx, *vby;
     const float *jx, *jy;
     const float2 *cfa;
-    const int32_t *goff, *gent;
+    const int32_t *goff;
     const float *inv_m;
     float2 *w;
     float c;

@@ -424,7 +424,6 @@ int Engine::build(const std::vector<const HostSystem *> &reps, std::unique_ptr<E
     FM_UP(bk_, hbk);
     FM_UP(br0_, hbr0);
     FM_UP(goff_, goff);
-    FM_UP(gent_, gent);
     FM_UP(gpos_, gpos);
     size_t most = 0;  // particles of the largest replica
     hiid.reserve(N);
@@ -532,8 +531,8 @@ int Engine::build(const std::vector<const HostSystem *> &reps, std::unique_ptr<E
     FM_AL(err_, 1);
     if (E->list_) {
         FM_AL(nbr_, (size_t)E->nbr_cap_ * N / 2);  // uint16 entries
-        FM_AL(nnum_, N);
-        FM_AL(lid_, N);
+        FM_AL(nnum_, N + 1);  // (a last tile without particles reads its first slot)
+        FM_AL(lid_, N + 1);
         FM_AL(ctl_, R);
         FM_AL(any_, 1);
         // two sets of displacement slots and two sorted-order position
@@ -1604,11 +1603,10 @@ int Engine::get_forces(int r, float *fx, float *fy, std::string &err) {
     if (rc) return rc;
     rc = ensure_primed(err);
     if (rc) return rc;
-    // (corner forces are held in gather order: no entry table; the error word
-    // is reported before the forces are waited for)
+    // (the error word is reported before the forces are waited for)
     hipError_t he = launch_report();
     if (he != hipSuccess) return check(he, "report", err);
-    rc = io_force_out(r, fx_.p, fy_.p, cf_.p, nullptr, fx, fy, err);
+    rc = io_force_out(r, fx_.p, fy_.p, cf_.p, fx, fy, err);
     if (rc) return rc;
     return sync(err, true);
 }

@@ -305,8 +305,8 @@ private:
     int io_state_out(int r, int k, const float *const *src, float *const *dst, std::string &err);
     int io_state_in(int r, int k, const float *const *src, float *const *dst, const float *wrap,
                     int stride, std::string &err);
-    int io_force_out(int r, const float *fx, const float *fy, const float2 *cf, const int32_t *gent,
-                     float *ox, float *oy, std::string &err);
+    int io_force_out(int r, const float *fx, const float *fy, const float2 *cf, float *ox, float *oy,
+                     std::string &err);
     // dst[i] = src[idx ? idx[i] : i] (idx: device)
     template <class T>
     int io_out(size_t n, const T *src, const int32_t *idx, T *dst, std::string &err);
@@ -383,7 +383,7 @@ private:
     DBuf<int32_t> spos_;
     DBuf<float2> xys_;
     DBuf<Tile> tiles_;
-    DBuf<int32_t> t0_, t1_, t2_, bi_, bj_, goff_, gent_, gpos_;
+    DBuf<int32_t> t0_, t1_, t2_, bi_, bj_, goff_, gpos_;
     DBuf<float4> dmbm_;
     DBuf<float2> alm_, cf_;
     DBuf<float> bk_, br0_;

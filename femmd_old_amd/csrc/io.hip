@@ -70,12 +70,11 @@ __global__ __launch_bounds__(kIoThreads) void k_state_in(StateInArgs a, uint64_t
 }
 
 // Total force per particle, caller order: pair force plus its corner forces
-// in gather order (gent null: cf is held in gather order), x then y.
+// (held in gather order), x then y.
 __global__ __launch_bounds__(kIoThreads) void k_force_out(const float *fx, const float *fy,
                                                           const float2 *cf, const int32_t *goff,
-                                                          const int32_t *gent, const int32_t *iid,
-                                                          uint32_t n, uint64_t t0, uint32_t m,
-                                                          float *out) {
+                                                          const int32_t *iid, uint32_t n, uint64_t t0,
+                                                          uint32_t m, float *out) {
     const uint32_t t = blockIdx.x * kIoThreads + threadIdx.x;
     if (t >= m) return;
     const uint64_t i = t0 + t;
@@ -84,7 +83,7 @@ __global__ __launch_bounds__(kIoThreads) void k_force_out(const float *fx, const
     float v = y ? fy[q] : fx[q];
     if (goff)
         for (int e = goff[q]; e < goff[q + 1]; ++e) {
-            const float2 c = cf[gent ? gent[e] : e];
+            const float2 c = cf[e];
             v += y ? c.y : c.x;
         }
     out[t] = v;
@@ -258,14 +257,14 @@ int Engine::io_state_in(int r, int k, const float *const *src, float *const *dst
 }
 
 int Engine::io_force_out(int r, const float *fx, const float *fy, const float2 *cf,
-                         const int32_t *gent, float *ox, float *oy, std::string &err) {
+                         float *ox, float *oy, std::string &err) {
     const size_t n = (size_t)nparticles(r);
     float *const dst[2] = {ox, oy};
     return io_read(
         2 * n, sizeof(float),
         [&](uint64_t i, uint32_t m, void *slot) {
             hipLaunchKernelGGL(k_force_out, dim3(blocks(m)), dim3(kIoThreads), 0, stream_, fx, fy, cf,
-                               gather_ ? goff_.p : nullptr, gent, iid_.p + reps_h_[r].p0, (uint32_t)n,
+                               gather_ ? goff_.p : nullptr, iid_.p + reps_h_[r].p0, (uint32_t)n,
                                i, m, static_cast<float *>(slot));
             return hipGetLastError() != hipSuccess;
         },

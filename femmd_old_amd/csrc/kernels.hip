@@ -3017,11 +3017,12 @@ __device__ void adj_list_tile(const AdjArgs &A, int tile, PairLds &L, float2 *lp
 // Piola-Kirchhoff stress along dF = dDs Bm) pushed through H = -A0 P Bm^T;
 // and dL/dE_e += w . f_e / E_e (P is linear in (lambda, mu), both
 // proportional to E at fixed nu).
-__device__ void adj_elem_block(const AdjArgs &A, int b, double *red) {
+__device__ void adj_elem_block(const AdjArgs &A, int b) {
     const ForceArgs &a = A.f;
     const Span sp = a.el.espans[b];
     const RepDesc R = a.reps[sp.rep];
     for (int e = sp.begin + (int)threadIdx.x; e < sp.end; e += blockDim.x) {
+        const int g0 = a.el.gpos[3 * e], g1 = a.el.gpos[3 * e + 1], g2 = a.el.gpos[3 * e + 2];
         const int n0 = a.el.t0[e], n1 = a.el.t1[e], n2 = a.el.t2[e];
         const float x0 = a.x[n0], y0 = a.y[n0];
         const float x1 = a.x[n1], y1 = a.y[n1];
@@ -3107,14 +3108,13 @@ __device__ void adj_elem_block(const AdjArgs &A, int b, double *red) {
         const float f1x = -(P00 * B.z + P01 * B.w), f1y = -(P10 * B.z + P11 * B.w);
         const float g0x = -(Q00 * B.x + Q01 * B.y), g0y = -(Q10 * B.x + Q11 * B.y);
         const float g1x = -(Q00 * B.z + Q01 * B.w), g1y = -(Q10 * B.z + Q11 * B.w);
-        A.cfa[3 * e] = make_float2(g0x, g0y);
-        A.cfa[3 * e + 1] = make_float2(g1x, g1y);
-        A.cfa[3 * e + 2] = make_float2(-g0x - g1x, -g0y - g1y);
+        A.cfa[g0] = make_float2(g0x, g0y);
+        A.cfa[g1] = make_float2(g1x, g1y);
+        A.cfa[g2] = make_float2(-g0x - g1x, -g0y - g1y);
         const double wf = (double)(w0.x * f0x + w0.y * f0y) + (double)(w1.x * f1x + w1.y * f1y) -
                           (double)(w2.x * (f0x + f1x) + w2.y * (f0y + f1y));
         A.dE[e] += wf / (double)A.eE[e];
     }
-    (void)red;
 }
 
 // Bond part of J w: g = -k (r - r0) / r, g' = dg/ds = -k r0 / (2 r^3).
@@ -3139,8 +3139,8 @@ __device__ void adj_bond_block(const AdjArgs &A, int b) {
         const float dwx = wi.x - wj.x, dwy = wi.y - wj.y;
         const float g2 = 2.0f * gp * (dx * dwx + dy * dwy);
         const float jx = g * dwx + g2 * dx, jy = g * dwy + g2 * dy;
-        A.cfa[a.el.cf_bond0 + 2 * l] = make_float2(jx, jy);
-        A.cfa[a.el.cf_bond0 + 2 * l + 1] = make_float2(-jx, -jy);
+        A.cfa[a.el.gpos[a.el.cf_bond0 + 2 * l]] = make_float2(jx, jy);
+        A.cfa[a.el.gpos[a.el.cf_bond0 + 2 * l + 1]] = make_float2(-jx, -jy);
     }
 }
 
@@ -3175,13 +3175,16 @@ __global__ __launch_bounds__(256) void k_adj_forces(AdjArgs A) {
     }
     b -= a.ntiles;
     if (b < a.el.nespans) {
-        adj_elem_block(A, b, s_red);
+        adj_elem_block(A, b);
         return;
     }
     b -= a.el.nespans;
     if (b < a.el.nbspans) adj_bond_block(A, b);
 }
 
+// Bound by its chain of loads: the corner parts are held in gather order and
+// read four at a time (an entry table before each, one after another: 23 k
+// particles 4.2 -> 3.2 us, 233 k 5.9 -> 5.4).
 __global__ __launch_bounds__(kKickThreads) void k_adj_kick(AdjKickArgs a) {
     const Span sp = a.spans[blockIdx.x];
     const RepDesc R = a.reps[sp.rep];
@@ -3191,10 +3194,18 @@ __global__ __launch_bounds__(kKickThreads) void k_adj_kick(AdjKickArgs a) {
     if (a.accumulate) {
         float jx = a.jx[p], jy = a.jy[p];
         if (a.goff) {
-            for (int e = a.goff[p]; e < a.goff[p + 1]; ++e) {
-                const float2 c = a.cfa[a.gent[e]];
-                jx += c.x;
-                jy += c.y;
+            // (four corners' loads in flight, added in order)
+            const int e1 = a.goff[p + 1];
+            for (int e = a.goff[p]; e < e1; e += 4) {
+                float2 c[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) c[u] = a.cfa[min(e + u, e1 - 1)];
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    if (e + u < e1) {
+                        jx += c[u].x;
+                        jy += c[u].y;
+                    }
             }
         }
         xbx += jx;
