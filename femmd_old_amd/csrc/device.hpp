@@ -60,9 +60,9 @@ struct alignas(16) RepDesc {
     float dslack;      // rounding allowance of the displacement test
     float im_uniform;  // 1/m shared by every particle of the replica (the
                        // kick then loads no inv_m); 0: masses differ
-    int32_t pg;        // particles [pg, p1) have element or bond corners (or
-                       // the replica has no pair forces: no tile integrates
-                       // them, the node kick does)
+    int32_t pg;        // particles [pg, p1) have element or bond corners (all
+                       // of them where the replica has no pair forces: no tile
+                       // integrates them, the node kick does)
     float rc_list;     // list mode: the largest cutoff of the pair table (in
                        // sigma units); lists hold every pair within
                        // rc_list * sigma_ij + skin

@@ -3,9 +3,8 @@
 // Replaces the reference's per-step host loop (femmd2D/src/integrator.cpp:
 // 8-57) and its upload / topology setup (femmd2D/src/particles.cpp:105-199,
 // femmd2D/src/bonds.cpp:31-83, femmd2D/src/nn.cpp:192-250).  One step is
-// five kernels on one stream (kick+bin, scan reduce, scan apply, scatter,
-// forces) with no host synchronisation; the step loop is replayed from a
-// captured HIP graph.
+// two to four kernels on one stream (kernels.hip) with no host
+// synchronisation; the step loop is replayed from a captured HIP graph.
 #include "engine.hpp"
 
 #include <algorithm>

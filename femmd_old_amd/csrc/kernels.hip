@@ -12,6 +12,7 @@
 //                look-back): cell starts, sorted order, sorted copies (cell
 //                walk: the elements and bonds beside it)
 //   k_list_build list mode: Verlet lists of the rebuilding replicas' tiles
+//   k_rebuild    the three above as one launch, for a single replica that fits
 //   k_forces     LJ cell tiles (LDS-staged neighbours, lists or the 3x3 cell
 //                walk); each tile then gives its centre particles, with their
 //                corner forces gathered through a per-particle CSR in a fixed
@@ -22,7 +23,8 @@
 //                (no tiles)
 // and at the end of a run the second half-kick only, then the observables.
 // Energies, virials and the kinetic energy are per-workgroup FP64 partials
-// summed in a fixed order (k_bin / k_sort level 1, k_forces level 2).
+// summed in a fixed order (k_rebuild / k_bin / k_sort level 1, k_forces level
+// 2).
 //
 // The file is compiled with -ffp-contract=off: every FP32 expression that
 // must agree bit for bit with the reference's real=float arithmetic (wrap,
@@ -2691,7 +2693,16 @@ __host__ __device__ inline int forces_grid(const ForceArgs &a) {
 
 // Observables of the current step for every replica, with the same chunks
 // and order as the per-step path: level 1 (one workgroup per chunk), then
-// level 2 (one thread per replica); accumulate: add them to the running sums.
+// level 2 (one wavefront per replica); accumulate: add them to the running
+// sums.  Where every replica has one chunk, its workgroup does both (one
+// launch: a one-step run of 256 particles with its queries 78.0 -> 75.9 us).
+__global__ __launch_bounds__(256) void k_observe(ObsArgs o, int accumulate, const uint32_t *err,
+                                                 uint32_t *report) {
+    __shared__ double red[kObsRed];
+    if (report && blockIdx.x == 0 && threadIdx.x == 0) *report = *err;
+    obs_chunk(o, blockIdx.x, 0, red);  // (ends with a barrier)
+    if (threadIdx.x < 64) obs_finish(o, blockIdx.x, accumulate != 0);
+}
 __global__ __launch_bounds__(256) void k_observe_l1(ObsArgs o) {
     __shared__ double red[kObsRed];
     obs_level1(o, blockIdx.x, gridDim.x, red);
@@ -2706,6 +2717,10 @@ __global__ __launch_bounds__(256) void k_observe_l2(ObsArgs o, int accumulate, c
 hipError_t launch_observe(const ObsArgs &o, bool accumulate, const uint32_t *err, uint32_t *report,
                           hipStream_t s) {
     if (o.nrep <= 0) return hipSuccess;
+    if (o.nchunk == 1) {
+        hipLaunchKernelGGL(k_observe, dim3(o.nrep), dim3(256), 0, s, o, accumulate ? 1 : 0, err, report);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(k_observe_l1, dim3(std::min(o.nrep * o.nchunk, 4096)), dim3(256), 0, s,
                        o);
     hipLaunchKernelGGL(k_observe_l2, dim3((o.nrep + 3) / 4), dim3(256), 0, s, o, accumulate ? 1 : 0,
