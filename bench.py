@@ -10,8 +10,8 @@ A step is one pass of the hot path over the whole system: half-kick + drift
 on the steps where some particle has moved more than skin / 2 since the
 last build, the reference's rule; skin 0.6, the engine default), LJ / CST
 forces, and the second
-half-kick with its kinetic-energy reduction (fused into the next step's
-first kernel).  --skin 0 walks the cells every step instead.  Inputs are
+half-kick with its kinetic-energy reduction (fused with the next step's
+first half-kick into the force pass).  --skin 0 walks the cells every step instead.  Inputs are
 resident in HBM when the timed region starts.
 
 Prints one JSON line: value = particle-steps/s; roofline for the dominant
@@ -51,54 +51,59 @@ def _eager(obj):
 def algorithmic_bytes(n, ncells, ntri, nbond, list_len=None, uniform_mass=False, n_corner=0):
     """Bytes each kernel moves per executed launch in this layout (each
     input array read once, each output written once; FP32 values, int32
-    indices).  The force pass also integrates the n - n_corner particles
-    without element or bond corners; the node kick integrates the n_corner
-    others.  uniform_mass: the kick takes the mass from the replica's
-    descriptor (no inv_m read).
+    indices).  The force pass also integrates its particles; the node kick
+    integrates n_corner others (those of replicas without pair forces: 0 in
+    every workload here).  uniform_mass: the kick takes the mass from the
+    replica's descriptor (no inv_m read).  The element and bond forces are
+    formed beside the binning (the cell walk's sort) every step.
 
     Per-step cell walk (list_len None):
-    forces   r sorted (16), perm: 20/particle; w fx,fy: 8/corner particle;
-             kicked particles r vx,vy, w x,y,vx,vy, slot: +28 (+4 inv_m);
-             r start 4/cell, counter read-modify-write 8/cell;
-             CST: r 3 ids, Dm, Bm, A0*lambda, A0*mu, 3 node x,y; w 3 corners:
-             100/element; bond: r ids, k, r0, 2 node x,y; w 2 ends: 48/bond
+    forces   r sorted (16), perm: 20/particle; kicked particles r vx,vy,
+             w x,y,vx,vy, slot: +28 (+4 inv_m); r corner forces: 24/element,
+             16/bond; r start 4/cell, counter read-modify-write 8/cell
+    elements CST: r 3 ids, 3 gather places, Dm, Bm, A0*lambda, A0*mu, 3 node
+             x,y; w 3 corners: 112/element; bond: r ids, places, k, r0, 2 node
+             x,y; w 2 ends: 56/bond
     kick     (node kick) r fx,fy,x,y,vx,vy,goff; w x,y,vx,vy,slot: 48 (+4
-             inv_m)/corner particle; gather 12/corner
+             inv_m)/particle, w fx,fy by the force pass: +8
     sort     r count, w count (zeroed), w start: 12/cell; r own slot entry,
              x,y,group; w perm, sorted (16): 36/particle
     Neighbour lists (list_len = mean list length L, padded to groups of 4:
     about L + 1.5 slots of 2 bytes):
     forces   r sorted x,y (8), length, slots, internal id (4): 16 + 2(L+1.5)
-             /particle; w fx,fy: 8/corner particle; kicked particles r vx,vy,
-             w x,y,vx,vy and the sorted-order copy of x,y: +32 (+4 inv_m);
-             r start: 4/cell; elements and bonds as above
+             /particle; kicked particles r vx,vy, w x,y,vx,vy and the
+             sorted-order copy of x,y: +32 (+4 inv_m); corner forces as above;
+             tile records: under 4/cell
+    elements as above
     kick     (node kick) r fx,fy,x,y,vx,vy,spos,goff; w x,y,vx,vy and the
-             sorted-order x,y: 56 (+4 inv_m)/corner particle; gather 12/corner
+             sorted-order x,y: 56 (+4 inv_m)/particle, w fx,fy: +8
     bin      r x,y; w slot: 12/particle; counters 8/cell     (rebuild steps)
     sort     as above plus spos and the sorted x,y: 48/particle (rebuild steps)
     list     r sorted (16); w slots, length: 20 + 2(L+1.5)/particle;
              r start: 4/cell                                   (rebuild steps)
     """
-    corners = 36 * ntri + 24 * nbond
-    elems = 100 * ntri + 48 * nbond
+    corners = 24 * ntri + 16 * nbond
+    elems = 112 * ntri + 56 * nbond
     im = 0 if uniform_mass else 4
     nk = n - n_corner  # integrated by the force pass
     if list_len is None:
         b = {
-            "kick": (48 + im) * n_corner + corners,
+            "kick": (48 + im) * n_corner,
+            "elements": elems,
             "bin": 0,
             "sort": 36 * n + 12 * ncells,
             "list_build": 0,
-            "forces": 20 * n + 8 * n_corner + (28 + im) * nk + 12 * ncells + elems,
+            "forces": 20 * n + 8 * n_corner + (28 + im) * nk + 12 * ncells + corners,
         }
     else:
         slots = 2.0 * (float(list_len) + 1.5)
         b = {
-            "kick": (56 + im) * n_corner + corners,
+            "kick": (56 + im) * n_corner,
+            "elements": elems,
             "bin": 12 * n + 8 * ncells,
             "sort": 48 * n + 12 * ncells,
             "list_build": int((20 + slots) * n) + 4 * ncells,
-            "forces": int((16 + slots) * n) + 8 * n_corner + (32 + im) * nk + 4 * ncells + elems,
+            "forces": int((16 + slots) * n) + 8 * n_corner + (32 + im) * nk + 4 * ncells + corners,
         }
     return b
 
@@ -114,10 +119,11 @@ def compulsory_bytes(n, ncells, ntri, nbond, n_fea_nodes, n_bonded_nodes, excl=T
     force pass: LJ r sorted x,y, perm (+ exclusion id), w fx,fy: 20 (+4)/particle,
                 r start 4/cell; CST r 3 ids, Bm, A0, E, 3 node x,y, w 3 corners:
                 84/triangle; bond r ids, k, r0, 2 node x,y, w 2 ends: 40/bond
-    fused force pass (the kernel launched): the same, except that for each
-    of the n - n_corner particles without element or bond corners it also
-                kicks and drifts: instead of w fx,fy it r vx,vy (+ inv_m when
-                masses differ), w x,y,vx,vy: +16 (+4)/particle
+    fused force pass: the same, except that for each of n - n_corner particles
+                it also kicks and drifts: instead of w fx,fy it r vx,vy (+
+                inv_m when masses differ), w x,y,vx,vy: +16 (+4)/particle
+    pass:       the fused pass without its elements and bonds (formed beside
+                the binning): the bytes of the k_forces launch
     step:       128/particle (124 without exclusions) + 12/cell + 120/triangle
                 + 20/element node + 64/bond + 20/bonded node"""
     per_p = 24 if excl else 20
@@ -125,18 +131,8 @@ def compulsory_bytes(n, ncells, ntri, nbond, n_fea_nodes, n_bonded_nodes, excl=T
     fused = forces + (n - n_corner) * (16 if uniform_mass else 20)
     step = ((128 if excl else 124) * n + 12 * ncells + 120 * ntri + 20 * n_fea_nodes
             + 64 * nbond + 20 * n_bonded_nodes)
-    return {"forces": forces, "forces_fused": fused, "step": step}
-
-
-def fused_corner_particles(w) -> int:
-    """Particles with element or bond corners (integrated by the node kick,
-    not by the force pass)."""
-    import numpy as np
-    ga = w.global_arrays()
-    u = [np.asarray(ga["tri"], np.int64).ravel()]
-    if w.n_bonds:
-        u += [np.asarray(w.bonds[0], np.int64), np.asarray(w.bonds[1], np.int64)]
-    return int(np.unique(np.concatenate(u)).size) if sum(a.size for a in u) else 0
+    return {"forces": forces, "forces_fused": fused, "pass": fused - 84 * ntri - 40 * nbond,
+            "step": step}
 
 
 def measured_traffic(kernel: str, mode: str):
@@ -237,7 +233,7 @@ def c3_leg(steps: int, warmup: int, skin: float):
     bonded = len(set(np.asarray(w.bonds[0], int).tolist()) |
                  set(np.asarray(w.bonds[1], int).tolist())) if w.n_bonds else 0
     cb = compulsory_bytes(w.n_total, ncx * ncy, w.n_tri, w.n_bonds, int(w.n_nodes), bonded,
-                          excl=True, n_corner=fused_corner_particles(w))
+                          excl=True)
     ms_step = 1e3 * secs / steps
     # run twice: two fresh systems, the same steps, bitwise the same state
     a = _eager(configs.build_system(w, skin=skin))
@@ -260,8 +256,8 @@ def c3_leg(steps: int, warmup: int, skin: float):
             "steps_per_rebuild": round(steps / max(ls1["rebuilds"] - ls0["rebuilds"], 1), 2)
             if list_mode else None,
             "step_kernels_ms": {k: round(v, 5) for k, v in prof.items()},
-            "forces_compulsory_bytes": cb["forces_fused"],
-            "forces_frac": round(cb["forces_fused"] / (prof["forces"] * 1e-3) / 1e9 / HBM_PEAK_GBS,
+            "forces_compulsory_bytes": cb["pass"],
+            "forces_frac": round(cb["pass"] / (prof["forces"] * 1e-3) / 1e9 / HBM_PEAK_GBS,
                                  4),
             "step_compulsory_bytes": cb["step"],
             "step_frac": round(cb["step"] / (ms_step * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
@@ -515,8 +511,7 @@ def main():
     m = w.global_arrays()["mass"]
     ab = algorithmic_bytes(w.n_total, ncx * ncy, w.n_tri, w.n_bonds,
                            ls1["mean"] if list_mode else None,
-                           uniform_mass=bool(np.isfinite(m[0]) and m[0] > 0 and np.all(m == m[0])),
-                           n_corner=fused_corner_particles(w))
+                           uniform_mass=bool(np.isfinite(m[0]) and m[0] > 0 and np.all(m == m[0])))
     kern = "forces"
     ga = w.global_arrays()
     n_nodes = int(w.n_nodes)
@@ -524,22 +519,22 @@ def main():
                  set(np.asarray(w.bonds[1], int).tolist())) if w.n_bonds else 0
     uniform = bool(np.isfinite(m[0]) and m[0] > 0 and np.all(m == m[0]))
     cb = compulsory_bytes(w.n_total, ncx * ncy, w.n_tri, w.n_bonds, n_nodes, bonded,
-                          excl=bool(w.elastomers), n_corner=fused_corner_particles(w),
-                          uniform_mass=uniform)
-    achieved = cb["forces_fused"] / (prof[kern] * 1e-3) / 1e9
+                          excl=bool(w.elastomers), uniform_mass=uniform)
+    achieved = cb["pass"] / (prof[kern] * 1e-3) / 1e9
     model_achieved = ab[kern] / (prof[kern] * 1e-3) / 1e9
-    step_bytes = ab["kick"] + ab["forces"] + rebuild_frac * sum(ab[k] for k in REBUILD_KERNELS)
+    step_bytes = ab["kick"] + ab["elements"] + ab["forces"] + rebuild_frac * sum(ab[k] for k in REBUILD_KERNELS)
     mode = "list" if list_mode else "cells"
     ms_step = 1e3 * secs / args.steps
     roof = {"bound": "hbm", "kernel": f"k_{kern}", "achieved": round(achieved, 1),
             "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
             "traffic": measured_traffic(f"k_{kern}", mode) if args.scale == 1.0 else None,
             "traffic_source": "rocprofv3 --pmc FETCH_SIZE, WRITE_SIZE (profiles/)",
-            "bytes_per_launch": cb["forces_fused"],
-            "bytes_rule": "compulsory bytes of the fused force pass (each input read once, "
-                          "each output written once, no neighbour list): 24/particle + "
-                          "4/cell + 84/triangle + 40/bond, + 16 per particle it kicks and "
-                          "drifts (r vx,vy, w x,y,vx,vy in place of w fx,fy)",
+            "bytes_per_launch": cb["pass"],
+            "bytes_rule": "compulsory bytes of the force pass with its kick (each input read "
+                          "once, each output written once, no neighbour list): 24/particle "
+                          "+ 4/cell, + 16 per particle it kicks and drifts (r vx,vy, w "
+                          "x,y,vx,vy in place of w fx,fy); the element and bond forces are "
+                          "another launch's",
             "launch_ms": round(prof[kern], 5),
             "layout_bytes_per_launch": ab[kern],
             "layout_achieved": round(model_achieved, 1),
