@@ -20,10 +20,11 @@ constexpr int kMaxSlots = 3 * (kMaxTileW + 2);
 // cells the smaller blocks are taken: they put more loads in flight while the
 // chip is not full, but each workgroup takes a ticket and looks back.
 // Measured, blocks of 64 against 256 cells: 4,367 particles (0.5 k cells) 8.5
-// against 18 us per sort, 114,140 (14.6 k cells) 14.2 against 15.3, 512
-// replicas (73.7 k cells) 24.3 against 25.8, 1.14 million (143 k cells) 54.7
-// against 34.6.
-constexpr int kSortCells = 256, kSortCellsFew = 64, kSortFewMax = 1536 * kSortCellsFew;
+// against 18 us per sort, 114,140 (14.4 k cells, lists) 20.1 against 21.5 us per
+// step, (22.2 k cells, cell walk) 41.7 against 41.7; then the other way, cell
+// walk of 228 k particles (44.1 k cells) 56.5 against 50.4 us per step, 457 k
+// (88.8 k cells) 87.4 against 71.5.
+constexpr int kSortCells = 256, kSortCellsFew = 64, kSortFewMax = 384 * kSortCellsFew;
 constexpr int kKickThreads = 256;
 constexpr int kElemThreads = 256;
 constexpr int kMaxPairTypes = 16;  // particle types of a pair table

@@ -988,7 +988,7 @@ __global__ __launch_bounds__(kKickThreads) void k_bin(KickArgs a, ElemArgs el) {
 // indices and before the look-back (they were loaded after it, from a second
 // read of the slot list).  Cell walk of 114,140 particles 18.6 -> 14.2 us a
 // step, a rebuild of 4,367 particles 20.7 -> 8.7, of 1.14 million 35.6 ->
-// 34.6, 512 replicas 28.5 -> 24.3.
+// 34.6, 512 replicas 28.5 -> 25.8.
 // ---------------------------------------------------------------------------
 constexpr unsigned long long kLbAggregate = 1ull, kLbInclusive = 2ull;
 constexpr int kSortThreads = 256;

@@ -10,7 +10,8 @@ from femmd_old_amd import System, configs
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("nc,skin", [(3, 0.6), (7, 0.6), (8, 0.6), (11, 0.6), (16, 0.6), (313, 0.6),
+@pytest.mark.parametrize("nc,skin", [(3, 0.6), (7, 0.6), (8, 0.6), (11, 0.6), (16, 0.6), (156, 0.6),
+                                     (157, 0.6), (313, 0.6),
                                      (314, 0.6), (8, 3.4), (25, 3.4)])
 def test_sorted_order(nc, skin):
     L = float(np.float32((nc + 0.5) * (configs.RC_WCA + skin)))
