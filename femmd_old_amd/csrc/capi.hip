@@ -524,6 +524,17 @@ int fm_clear_errors(fm_system *h) {
     FM_END(h)
 }
 
+// For the tests of what is never expected (not declared in include/femmd.h):
+// the polls after which a wait inside the one-kernel rebuild is given up
+// (< 0: the default).
+int fm_test_rebuild_spins(fm_system *h, int32_t spins) {
+    FM_GUARD(h)
+    h->hs.rebuild_spins = spins < 0 ? fm::kRebuildSpins : spins;
+    if (h->eng) h->eng->set_rebuild_spins(h->hs.rebuild_spins);
+    return FM_OK;
+    FM_END(h)
+}
+
 int fm_get_cells(fm_system *h, int32_t *ncx, int32_t *ncy, int32_t *key, int32_t *start,
                  int32_t *perm) {
     FM_GUARD(h)

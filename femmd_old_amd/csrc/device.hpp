@@ -298,9 +298,11 @@ struct ElemArgs {
 // 18.9 -> 16.2, 114,140 (986 workgroups) 20.5 -> 19.9.
 constexpr int kRebuildSync = 16 * (3 + 2 * 8);
 constexpr int kRebuildBins = 160, kRebuildMax = 1024;
+constexpr int kRebuildSpins = 1 << 22;  // seconds: a wait takes under 0.1 ms
 struct RebuildArgs {
     unsigned long long *sync;
     int32_t nbin, nlist;
+    int32_t spins;             // polls after which a wait is given up
 };
 
 struct ForceArgs {

@@ -66,7 +66,7 @@ std::string dev_error_text(uint32_t e) {
     if (e & FM_DEV_INVERTED) s += " inverted element (det F <= 0);";
     if (e & FM_DEV_NONFINITE) s += " non-finite coordinate;";
     if (e & FM_DEV_LIST_OVERFLOW) s += " neighbour list capacity exceeded;";
-    if (e & FM_DEV_SORT_STALL) s += " counting sort look-back timed out;";
+    if (e & FM_DEV_SORT_STALL) s += " counting sort or list rebuild timed out;";
     return s;
 }
 
@@ -112,6 +112,7 @@ int Engine::build(const std::vector<const HostSystem *> &reps, std::unique_ptr<E
     E->block_ = reps[0]->block;
     E->use_graph_ = reps[0]->use_graph;
     E->reorder_every_ = reps[0]->reorder_every;
+    E->rebuild_spins_ = reps[0]->rebuild_spins;
     E->obs_every_ = reps[0]->observe_every;
 
     // neighbour-list mode: one skin for the batch
@@ -798,6 +799,7 @@ RebuildArgs Engine::rebuild_args() const {
     r.sync = rebuild_words_.p;
     r.nbin = std::min((int)kspans_h_.size(), kRebuildBins);
     r.nlist = (int)tiles_h_.size();
+    r.spins = rebuild_spins_;
     return r;
 }
 
@@ -1429,10 +1431,29 @@ uint32_t Engine::errors() {
     return io_report(nullptr, 0, e) == FM_OK ? pin_.head()->err : 0u;
 }
 
+// A stalled one-kernel rebuild leaves its phase counters short and its
+// particles binned but not sorted: the words and the counts start again, and
+// the next call builds the lists anew.  (The host's copy of the error word is
+// current: the call that stalled has reported it.)
 int Engine::clear_errors() {
+    if (rebuild_words_.p && (pin_.head()->err & FM_DEV_SORT_STALL)) {
+        if (hipMemsetAsync(rebuild_words_.p, 0, rebuild_words_.n * sizeof(unsigned long long), stream_) !=
+                hipSuccess ||
+            launch_fill_int(count_.p, 0, (size_t)ncells_, stream_) != hipSuccess)
+            return FM_ERR_HIP;
+        primed_ = false;
+        ene_valid_ = false;
+        obs_valid_ = false;
+    }
     (void)hipMemsetAsync(err_.p, 0, sizeof(uint32_t), stream_);
     (void)hipStreamSynchronize(stream_);
+    pin_.head()->err = 0;
     return FM_OK;
+}
+
+void Engine::set_rebuild_spins(int spins) {
+    rebuild_spins_ = spins;
+    drop_graph();  // (an argument of its captured launches)
 }
 
 int Engine::compute_forces(std::string &err) {

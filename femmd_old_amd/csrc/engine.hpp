@@ -52,6 +52,8 @@ struct HostSystem {
     float skin = 0.6f;
     // launch tuning
     int32_t tile_w = 0, block = 256, use_graph = 1;
+    // polls after which a wait inside the one-kernel rebuild is given up
+    int32_t rebuild_spins = kRebuildSpins;
     // steps between re-orderings of the internal order (0: never)
     int32_t reorder_every = 1000;
     // observables formed and accumulated every step (1) or per run (0)
@@ -157,6 +159,7 @@ public:
     int64_t reorders() const { return nreorder_; }
     uint32_t errors();
     int clear_errors();
+    void set_rebuild_spins(int spins);
     // waits for the stream and reports the device's error word (reported: the
     // stream's last work has already written it to pin_)
     int sync(std::string &err, bool reported = false);
@@ -366,6 +369,7 @@ private:
     DBuf<int4> rinfo_;
     DBuf<uint8_t> mark_;
     DBuf<unsigned long long> sort_status2_;     // status words of the listed sort
+    int rebuild_spins_ = kRebuildSpins;
     DBuf<unsigned long long> rebuild_words_;    // one-kernel rebuild: RebuildArgs::sync, its sort's status words
     DBuf<int2> brep_;                   // per sort block: replica range
     DBuf<uint32_t> ro_tmp_;

@@ -2237,25 +2237,27 @@ __device__ __forceinline__ void phase_done(unsigned long long *sync, int k, unsi
                                __HIP_MEMORY_SCOPE_AGENT);
 }
 // Waits for phase k's go, then sees its writes.  False: the wait ran out
-// (uniform).
-__device__ __forceinline__ bool phase_wait(unsigned long long *sync, int k, unsigned long long epoch,
+// (uniform).  A workgroup that gives up leaves its phase's counter short, so
+// no later go comes until Engine::clear_errors has put the words back.
+__device__ __forceinline__ bool phase_wait(const RebuildArgs &rb, int k, unsigned long long epoch,
                                            int *s_ok, uint32_t *err) {
     if (threadIdx.x == 0) {
-        const unsigned long long *go = sync + 16 * (3 + 8 * k + (blockIdx.x & 7));
-        int spins = 0;
-        while (__hip_atomic_load(go, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) <= epoch &&
-               spins < kLbSpinLimit) {
-            ++spins;
+        const unsigned long long *go = rb.sync + 16 * (3 + 8 * k + (blockIdx.x & 7));
+        bool ok = false;
+        for (int spins = 0; spins < rb.spins; ++spins) {
+            ok = __hip_atomic_load(go, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) > epoch;
+            if (ok) break;
             __builtin_amdgcn_s_sleep(8);
         }
-        *s_ok = spins < kLbSpinLimit;
-        if (!*s_ok) atomicOr(err, 32u);  // FM_DEV_SORT_STALL: never expected
+        *s_ok = ok;
+        if (!ok) atomicOr(err, 32u);  // FM_DEV_SORT_STALL: never expected
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     }
     __syncthreads();
     return *s_ok != 0;
 }
 
+constexpr unsigned long long kNoTicket = ~0ull;
 template <bool kSigma>
 __global__ __launch_bounds__(256) void k_rebuild(KickArgs a, ElemArgs el, ScanArgs sa, ForceArgs f,
                                                  RebuildArgs rb) {
@@ -2277,8 +2279,15 @@ __global__ __launch_bounds__(256) void k_rebuild(KickArgs a, ElemArgs el, ScanAr
         return;
     }
     if (!one_rep_decide(a, wb == 0)) return;
-    if (threadIdx.x == 0) s_tk = atomicAdd(rb.sync, 1ull);
+    if (threadIdx.x == 0) {
+        // after a stall (reported, not yet cleared) no rebuild is tried: its
+        // waits would run to their bound, its binning add to one not sorted
+        const uint32_t e = __hip_atomic_load(a.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const unsigned long long tk = atomicAdd(rb.sync, 1ull);
+        s_tk = e & 32u ? kNoTicket : tk;
+    }
     __syncthreads();
+    if (s_tk == kNoTicket) return;
     const unsigned long long total = rb.nbin + sa.nsort + rb.nlist;
     const unsigned long long epoch = s_tk / total;
     int w = (int)(s_tk % total);
@@ -2290,14 +2299,14 @@ __global__ __launch_bounds__(256) void k_rebuild(KickArgs a, ElemArgs el, ScanAr
     }
     w -= rb.nbin;
     if (w < sa.nsort) {
-        if (!phase_wait(rb.sync, 0, epoch, &s_ok, a.err)) return;
+        if (!phase_wait(rb, 0, epoch, &s_ok, a.err)) return;
         sort_block<kSortCellsFew, true>(sa, w, (uint32_t)epoch, sa.status2,
                                   *reinterpret_cast<SortLds<kSortCellsFew> *>(dyn));
         phase_done(rb.sync, 1, epoch, sa.nsort);
         return;
     }
     w -= sa.nsort;
-    if (!phase_wait(rb.sync, 1, epoch, &s_ok, a.err)) return;
+    if (!phase_wait(rb, 1, epoch, &s_ok, a.err)) return;
     list_tiles<kSigma>(f, w, rb.nlist, dyn, s_cstart, s_off);
 }
 

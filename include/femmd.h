@@ -49,7 +49,7 @@ typedef struct fm_batch fm_batch;   /* many independent replicas */
 #define FM_DEV_INVERTED 4u       /* an element with det F <= 0             */
 #define FM_DEV_NONFINITE 8u      /* a non-finite coordinate after a drift  */
 #define FM_DEV_LIST_OVERFLOW 16u /* more neighbours than the list capacity */
-#define FM_DEV_SORT_STALL 32u    /* the counting sort's look-back timed out */
+#define FM_DEV_SORT_STALL 32u    /* a wait of the sort or rebuild timed out */
 
 /* ---- material models (femmd2D/src/interactions.cpp:411-689) ---- */
 #define FM_NEO_HOOKEAN 0 /* calcFeaForcesCPU2, svk = 0 (reference CPU) */
