@@ -1951,6 +1951,16 @@ __device__ __forceinline__ uint32_t shift_in8(uint32_t m, H &&h) {
     return m;
 }
 
+// The word of n candidates (a multiple of 8 up to 32; 0 in a wavefront without
+// lists): predicate t, the t-th shifted in, at bit t.
+__host__ __device__ constexpr uint32_t mask_word(uint32_t m, int n) {
+    return __builtin_bitreverse32(m) >> ((32 - n) & 31);
+}
+static_assert(mask_word(0u, 0) == 0u && mask_word(1u, 8) == 0x80u && mask_word(0x80u, 8) == 1u &&
+                  mask_word(1u, 24) == 0x800000u && mask_word(1u, 32) == 0x80000000u &&
+                  mask_word(0x80000001u, 32) == 0x80000001u,
+              "no shift by the width of the word; the first candidate lowest");
+
 // List build of one staged tile; bound by vector issue.  Each row's
 // candidates (cells col-1 .. col+1, one contiguous run) are tested 32 at a
 // time into a bit mask per lane, with a wavefront-uniform trip count (the
@@ -2018,7 +2028,7 @@ __device__ void list_tile_body_mask(const ForceArgs &a, const Tile &T, const Rep
                 else
                     m = shift_in8(m, near);
             }
-            m = __brev(m) >> (32 - n8);  // bit t: candidate jr[r] + b + t
+            m = mask_word(m, n8);  // bit t: candidate jr[r] + b + t
             const int left = len[r] - b;  // candidates of the lane's own run
             m &= left >= 32 ? ~0u : (left > 0 ? (1u << left) - 1u : 0u);
             if (r == 1) {
