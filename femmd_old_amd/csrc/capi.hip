@@ -535,6 +535,15 @@ int fm_test_rebuild_spins(fm_system *h, int32_t spins) {
     FM_END(h)
 }
 
+// The same, before fm_commit: whether pinned memory is taken to be had.
+int fm_test_pinned(fm_system *h, int32_t on) {
+    FM_GUARD(h)
+    if (h->eng) return fail(h, FM_ERR_STATE, "system already committed");
+    h->hs.pinned = on != 0;
+    return FM_OK;
+    FM_END(h)
+}
+
 int fm_get_cells(fm_system *h, int32_t *ncx, int32_t *ncy, int32_t *key, int32_t *start,
                  int32_t *perm) {
     FM_GUARD(h)

@@ -436,8 +436,8 @@ int Engine::build(const std::vector<const HostSystem *> &reps, std::unique_ptr<E
     for (int e = 0; e < E->ntri_; ++e)  // (a single system's elements: the adjoint)
         if (R == 1) heinv[E->ecaller_h_[e]] = e;
     FM_UP(ecinv_, heinv);
-    if ((he = E->pin_.alloc(4 * most * sizeof(float))) != hipSuccess)
-        return E->check(he, "pinned memory", err);
+    if ((he = E->pin_.alloc(4 * most * sizeof(float), reps[0]->pinned)) != hipSuccess)
+        return E->check(he, "transfer memory", err);
     {
         // movable particles: no element, bond or cluster refers to them, so
         // a re-ordering may give them new internal ids
@@ -1285,7 +1285,7 @@ int Engine::launch_bodies_eager(const BodyKind &k) {
     if (k.close) {
         // femmd2D/src/integrator.cpp:18-19: the observables of the last step
         // (Properties::compute)
-        return launch_observe(obs_args(), true, err_.p, &pin_.head()->err, stream_) == hipSuccess ? 0
+        return launch_observe(obs_args(), true, err_.p, &pin_.dhead()->err, stream_) == hipSuccess ? 0
                                                                                               : -1;
     }
     return 0;
@@ -1417,7 +1417,7 @@ int Engine::step(int nsteps, std::string &err) {
 }
 
 int Engine::sync(std::string &err, bool reported) {
-    const int rc = reported ? check(hipStreamSynchronize(stream_), "step", err) : io_report(nullptr, 0, err);
+    const int rc = reported ? io_wait(err) : io_report(nullptr, 0, err);
     if (rc) return rc;
     if (pin_.head()->err) {
         err = dev_error_text(pin_.head()->err);
@@ -1486,7 +1486,7 @@ int Engine::form_observables(std::string &err) {
         return check(hipGetLastError(), "ke", err);
     ObsArgs o = obs_args();
     o.ke_kick = 1;  // the partials k_ke just formed
-    if (launch_observe(o, false, err_.p, &pin_.head()->err, stream_) != hipSuccess)
+    if (launch_observe(o, false, err_.p, &pin_.dhead()->err, stream_) != hipSuccess)
         return check(hipGetLastError(), "observe", err);
     rc = sync(err, true);
     if (rc) return rc;

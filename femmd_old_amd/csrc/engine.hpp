@@ -54,6 +54,7 @@ struct HostSystem {
     int32_t tile_w = 0, block = 256, use_graph = 1;
     // polls after which a wait inside the one-kernel rebuild is given up
     int32_t rebuild_spins = kRebuildSpins;
+    bool pinned = true;  // transfers through pinned memory where it can be had
     // steps between re-orderings of the internal order (0: never)
     int32_t reorder_every = 1000;
     // observables formed and accumulated every step (1) or per run (0)
@@ -83,8 +84,10 @@ struct DBuf {
     }
 };
 
-// Pinned host memory of an engine (io.hip): a head the device reports into,
-// and the slots its transfers go through.
+// Host memory of an engine (io.hip): a head the device reports into, and the
+// slots its transfers go through.  Pinned, the kernels reading and writing it
+// in place (d = p); where none can be had, ordinary memory of one slot with a
+// copy on the device (d) that the kernels use (staged).
 constexpr size_t kIoSlotBytes = 1 << 20;
 constexpr int kIoSlots = 4;
 struct IoHead {
@@ -93,7 +96,7 @@ struct IoHead {
     double obs[kObsStride];   // one replica's observables record
 };
 struct PinBuf {
-    unsigned char *p = nullptr;
+    unsigned char *p = nullptr, *d = nullptr;  // the host's, the kernels'
     size_t slot = 0;
     int nslot = 0;
     hipEvent_t ev[kIoSlots] = {};
@@ -102,9 +105,12 @@ struct PinBuf {
     PinBuf(const PinBuf &) = delete;
     PinBuf &operator=(const PinBuf &) = delete;
     ~PinBuf();
-    hipError_t alloc(size_t most);
+    hipError_t alloc(size_t most, bool pinned);
+    bool staged() const { return d != p; }
     IoHead *head() const { return reinterpret_cast<IoHead *>(p); }
+    IoHead *dhead() const { return reinterpret_cast<IoHead *>(d); }
     void *data(int s) const { return p + sizeof(IoHead) + (size_t)s * slot; }
+    void *ddata(int s) const { return d + sizeof(IoHead) + (size_t)s * slot; }
 };
 
 class Engine {
@@ -315,6 +321,7 @@ private:
     int io_out(size_t n, const T *src, const int32_t *idx, T *dst, std::string &err);
     int io_in(size_t bytes, const void *src, void *dst, std::string &err);
     int io_report(const double *src, int n, std::string &err);
+    int io_wait(std::string &err);  // the stream's work done, the head current
     hipError_t launch_report(const double *src = nullptr, int n = 0);  // io_report without the wait
     int read_obs(int r, double *v, std::string &err);
     int launch_invert();

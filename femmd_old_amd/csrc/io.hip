@@ -8,7 +8,8 @@
 // one wait; the host only copies contiguous runs between that memory and the
 // caller's arrays.  Large transfers go through a ring of kIoSlots slots, the
 // device filling (or emptying) some while the host copies another: the pinned
-// memory of an engine is bounded by kIoSlots * kIoSlotBytes.
+// memory of an engine is bounded by kIoSlots * kIoSlotBytes.  Where no pinned
+// memory can be had, a slot on the device takes its place and is copied.
 //
 // Bound by the latency of one kernel and one wait (13 us) for small systems
 // and by the host link for large ones.  Before, each array was copied to
@@ -115,20 +116,32 @@ unsigned blocks(uint32_t m) { return (m + kIoThreads - 1) / kIoThreads; }
 }  // namespace
 
 PinBuf::~PinBuf() {
-    if (p) (void)hipHostFree(p);
+    if (staged()) {
+        delete[] p;
+        if (d) (void)hipFree(d);
+    } else if (p) {
+        (void)hipHostFree(p);
+    }
     for (auto &e : ev)
         if (e) (void)hipEventDestroy(e);
 }
 
-// Pinned memory for the largest replica's state, at most a ring of slots.
-hipError_t PinBuf::alloc(size_t most) {
+// Memory for the largest replica's state, at most a ring of slots.
+hipError_t PinBuf::alloc(size_t most, bool pinned) {
     slot = std::min<size_t>(std::max<size_t>((most + 255) / 256 * 256, 1024), kIoSlotBytes);
     nslot = most > slot ? kIoSlots : 1;
-    hipError_t e = hipHostMalloc(reinterpret_cast<void **>(&p), sizeof(IoHead) + slot * nslot,
-                                 hipHostMallocDefault);
-    if (e != hipSuccess) {
-        p = nullptr;
-        return e;
+    hipError_t e = hipSuccess;
+    if (pinned && hipHostMalloc(reinterpret_cast<void **>(&p), sizeof(IoHead) + slot * nslot,
+                                hipHostMallocDefault) == hipSuccess) {
+        d = p;
+    } else {
+        (void)hipGetLastError();
+        nslot = 1;
+        p = new unsigned char[sizeof(IoHead) + slot];
+        if ((e = hipMalloc(reinterpret_cast<void **>(&d), sizeof(IoHead) + slot)) != hipSuccess) {
+            d = nullptr;
+            return e;
+        }
     }
     std::memset(p, 0, sizeof(IoHead));
     for (int k = 0; k < (nslot > 1 ? nslot : 0); ++k)
@@ -137,15 +150,21 @@ hipError_t PinBuf::alloc(size_t most) {
 }
 
 // `count` items of `elem` bytes to the host: fill(first, n, slot) launches
-// the kernel that writes items [first, first + n) into a slot, take(first, n,
-// slot) consumes them on the host, in order.
+// the kernel that writes items [first, first + n) into a slot (and, staged,
+// its copy follows on the stream), take(first, n, slot) consumes them on the
+// host, in order.
 template <class Fill, class Take>
 int Engine::io_read(size_t count, size_t elem, Fill &&fill, Take &&take, std::string &err) {
     std::lock_guard<std::mutex> lock(pin_.mu);
     const size_t per = pin_.slot / elem;
+    auto put = [&](size_t i, size_t m, int s) -> bool {  // true: failed
+        return fill((uint64_t)i, (uint32_t)m, pin_.ddata(s)) ||
+               (pin_.staged() && hipMemcpyAsync(pin_.data(s), pin_.ddata(s), m * elem,
+                                                hipMemcpyDeviceToHost, stream_) != hipSuccess);
+    };
     if (count == 0) return FM_OK;
     if (count <= per) {
-        if (fill((uint64_t)0, (uint32_t)count, pin_.data(0))) return check(hipGetLastError(), "read", err);
+        if (put(0, count, 0)) return check(hipErrorUnknown, "read", err);
         const int rc = check(hipStreamSynchronize(stream_), "read", err);
         if (rc) return rc;
         take((uint64_t)0, (uint32_t)count, pin_.data(0));
@@ -157,7 +176,7 @@ int Engine::io_read(size_t count, size_t elem, Fill &&fill, Take &&take, std::st
         for (; issued < nchunk && issued < c + (size_t)pin_.nslot; ++issued) {
             const size_t i = issued * per;
             const int s = (int)(issued % pin_.nslot);
-            if (fill((uint64_t)i, (uint32_t)std::min(per, count - i), pin_.data(s)) ||
+            if (put(i, std::min(per, count - i), s) ||
                 (pin_.nslot > 1 && hipEventRecord(pin_.ev[s], stream_) != hipSuccess)) {
                 (void)hipStreamSynchronize(stream_);
                 return check(hipErrorUnknown, "read", err);
@@ -190,7 +209,9 @@ int Engine::io_write(size_t count, size_t elem, Put &&put, Use &&use, std::strin
         }
         const uint32_t m = (uint32_t)std::min(per, count - i);
         put((uint64_t)i, m, pin_.data(s));
-        if (use((uint64_t)i, m, pin_.data(s)) ||
+        if ((pin_.staged() && hipMemcpyAsync(pin_.ddata(s), pin_.data(s), m * elem,
+                                             hipMemcpyHostToDevice, stream_) != hipSuccess) ||
+            use((uint64_t)i, m, pin_.ddata(s)) ||
             (pin_.nslot > 1 && hipEventRecord(pin_.ev[s], stream_) != hipSuccess)) {
             (void)hipStreamSynchronize(stream_);
             return check(hipErrorUnknown, "write", err);
@@ -299,7 +320,7 @@ int Engine::io_in(size_t bytes, const void *src, void *dst, std::string &err) {
             std::memcpy(slot, static_cast<const unsigned char *>(src) + i, m);
         },
         [&](uint64_t i, uint32_t m, void *slot) {
-            return hipMemcpyAsync(static_cast<unsigned char *>(dst) + i, slot, m, hipMemcpyHostToDevice,
+            return hipMemcpyAsync(static_cast<unsigned char *>(dst) + i, slot, m, hipMemcpyDefault,
                                   stream_) != hipSuccess;
         },
         err);
@@ -308,14 +329,22 @@ int Engine::io_in(size_t bytes, const void *src, void *dst, std::string &err) {
 // The error word, and n <= kObsStride doubles of src, read with one kernel
 // and one wait.
 hipError_t Engine::launch_report(const double *src, int n) {
-    hipLaunchKernelGGL(k_report, dim3(1), dim3(64), 0, stream_, err_.p, src, n, pin_.head());
+    hipLaunchKernelGGL(k_report, dim3(1), dim3(64), 0, stream_, err_.p, src, n, pin_.dhead());
     return hipGetLastError();
 }
 
 int Engine::io_report(const double *src, int n, std::string &err) {
     const int rc = check(launch_report(src, n), "report", err);
-    if (rc) return rc;
-    return check(hipStreamSynchronize(stream_), "report", err);
+    return rc ? rc : io_wait(err);
+}
+
+int Engine::io_wait(std::string &err) {
+    if (pin_.staged()) {
+        const int rc = check(hipMemcpyAsync(pin_.p, pin_.d, sizeof(IoHead), hipMemcpyDeviceToHost, stream_),
+                             "report", err);
+        if (rc) return rc;
+    }
+    return check(hipStreamSynchronize(stream_), "step", err);
 }
 
 int Engine::launch_invert() {
