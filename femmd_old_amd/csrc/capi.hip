@@ -535,7 +535,17 @@ int fm_test_rebuild_spins(fm_system *h, int32_t spins) {
     FM_END(h)
 }
 
-// The same, before fm_commit: whether pinned memory is taken to be had.
+// Whether a step takes its rebuild as one kernel, and the rebuild's workgroups.
+int fm_test_one_rebuild(fm_system *h, int32_t *one, int32_t *workgroups) {
+    FM_GUARD(h)
+    FM_NEED_ENGINE(h);
+    *one = h->eng->one_rebuild();
+    *workgroups = h->eng->rebuild_workgroups();
+    return FM_OK;
+    FM_END(h)
+}
+
+// Before fm_commit: whether pinned memory is taken to be had.
 int fm_test_pinned(fm_system *h, int32_t on) {
     FM_GUARD(h)
     if (h->eng) return fail(h, FM_ERR_STATE, "system already committed");

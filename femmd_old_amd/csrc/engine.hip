@@ -790,8 +790,12 @@ int Engine::launch_bin(bool gated) {
 // (profile() times the three apart).
 bool Engine::one_rebuild() const {
     if (!list_ || R_ != 1 || block_ != 256 || sort_cells_ != kSortCellsFew || prof_ev_) return false;
+    return rebuild_workgroups() <= kRebuildMax;
+}
+
+int Engine::rebuild_workgroups() const {
     const RebuildArgs r = rebuild_args();
-    return r.nbin + nsort_ + r.nlist <= kRebuildMax;
+    return r.nbin + nsort_ + r.nlist;
 }
 
 RebuildArgs Engine::rebuild_args() const {

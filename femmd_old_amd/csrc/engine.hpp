@@ -166,6 +166,8 @@ public:
     uint32_t errors();
     int clear_errors();
     void set_rebuild_spins(int spins);
+    bool one_rebuild() const;
+    int rebuild_workgroups() const;
     // waits for the stream and reports the device's error word (reported: the
     // stream's last work has already written it to pin_)
     int sync(std::string &err, bool reported = false);
@@ -206,7 +208,6 @@ private:
     int launch_bin(bool gated = false);
     KickArgs bin_args(bool gated);
     ScanArgs sort_args(bool gated);
-    bool one_rebuild() const;
     RebuildArgs rebuild_args() const;
     // One step body: kick2 (second half-kick of the previous step, with the
     // kinetic-energy partials when energy is set), drift (first half-kick,
