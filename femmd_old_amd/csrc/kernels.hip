@@ -2246,28 +2246,34 @@ __device__ __forceinline__ void phase_done(unsigned long long *sync, int k, unsi
             __hip_atomic_store(sync + 16 * (3 + 8 * k + x), epoch + 1, __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_AGENT);
 }
-// Waits for phase k's go, then sees its writes.  False: the wait ran out
-// (uniform).  A workgroup that gives up leaves its phase's counter short, so
-// no later go comes until Engine::clear_errors has put the words back.
+// Waits for phase k's go, then sees its writes.  False: the wait was given up
+// (uniform).  It runs out after rb.spins polls; a workgroup that gives up
+// leaves its phase's counter short, so no later go of that phase comes until
+// Engine::clear_errors has put the words back, and a later rebuild of the run
+// gives up once it finds the stall reported (looked for every 4096 polls, some
+// milliseconds, where the bound takes seconds; a look at the ticket instead
+// cost every rebuild of 114,140 particles 2 us).  Its binning adds to one not
+// sorted: counts past a cell's or replica's room are reported, never written.
 __device__ __forceinline__ bool phase_wait(const RebuildArgs &rb, int k, unsigned long long epoch,
                                            int *s_ok, uint32_t *err) {
     if (threadIdx.x == 0) {
         const unsigned long long *go = rb.sync + 16 * (3 + 8 * k + (blockIdx.x & 7));
-        bool ok = false;
-        for (int spins = 0; spins < rb.spins; ++spins) {
-            ok = __hip_atomic_load(go, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) > epoch;
-            if (ok) break;
+        int left = rb.spins;
+        while (__hip_atomic_load(go, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) <= epoch && left > 0) {
+            --left;
+            if ((left & 4095) == 0 &&
+                (__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & 32u))
+                left = 0;
             __builtin_amdgcn_s_sleep(8);
         }
-        *s_ok = ok;
-        if (!ok) atomicOr(err, 32u);  // FM_DEV_SORT_STALL: never expected
+        *s_ok = left > 0;
+        if (left <= 0) atomicOr(err, 32u);  // FM_DEV_SORT_STALL: never expected
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     }
     __syncthreads();
     return *s_ok != 0;
 }
 
-constexpr unsigned long long kNoTicket = ~0ull;
 template <bool kSigma>
 __global__ __launch_bounds__(256) void k_rebuild(KickArgs a, ElemArgs el, ScanArgs sa, ForceArgs f,
                                                  RebuildArgs rb) {
@@ -2289,15 +2295,8 @@ __global__ __launch_bounds__(256) void k_rebuild(KickArgs a, ElemArgs el, ScanAr
         return;
     }
     if (!one_rep_decide(a, wb == 0)) return;
-    if (threadIdx.x == 0) {
-        // after a stall (reported, not yet cleared) no rebuild is tried: its
-        // waits would run to their bound, its binning add to one not sorted
-        const uint32_t e = __hip_atomic_load(a.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const unsigned long long tk = atomicAdd(rb.sync, 1ull);
-        s_tk = e & 32u ? kNoTicket : tk;
-    }
+    if (threadIdx.x == 0) s_tk = atomicAdd(rb.sync, 1ull);
     __syncthreads();
-    if (s_tk == kNoTicket) return;
     const unsigned long long total = rb.nbin + sa.nsort + rb.nlist;
     const unsigned long long epoch = s_tk / total;
     int w = (int)(s_tk % total);

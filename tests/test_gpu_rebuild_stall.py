@@ -42,7 +42,7 @@ def test_a_stalled_rebuild_is_recovered(build):
             a.run(5)
     assert a.device_errors() & STALL
     # more rebuilds before the error is cleared, at the usual bound (seconds):
-    # none is tried
+    # each gives up long before it
     assert lib.fm_test_rebuild_spins(a.handle, -1) == 0
     t = time.perf_counter()
     with pytest.raises(FemmdError, match="timed out"):
