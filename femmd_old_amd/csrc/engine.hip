@@ -1425,6 +1425,17 @@ int Engine::sync(std::string &err, bool reported) {
     if (rc) return rc;
     if (pin_.head()->err) {
         err = dev_error_text(pin_.head()->err);
+        if (rebuild_words_.p && (pin_.head()->err & FM_DEV_SORT_STALL)) {
+            // a stalled one-kernel rebuild leaves its phase counters short and
+            // its particles binned but not sorted: the words and the counts
+            // start again, and the next call builds the lists anew
+            (void)hipMemsetAsync(rebuild_words_.p, 0, rebuild_words_.n * sizeof(unsigned long long),
+                                 stream_);
+            (void)launch_fill_int(count_.p, 0, (size_t)ncells_, stream_);
+            primed_ = false;
+            ene_valid_ = false;
+            obs_valid_ = false;
+        }
         return FM_ERR_DEVICE;
     }
     return FM_OK;
@@ -1435,23 +1446,9 @@ uint32_t Engine::errors() {
     return io_report(nullptr, 0, e) == FM_OK ? pin_.head()->err : 0u;
 }
 
-// A stalled one-kernel rebuild leaves its phase counters short and its
-// particles binned but not sorted: the words and the counts start again, and
-// the next call builds the lists anew.  (The host's copy of the error word is
-// current: the call that stalled has reported it.)
 int Engine::clear_errors() {
-    if (rebuild_words_.p && (pin_.head()->err & FM_DEV_SORT_STALL)) {
-        if (hipMemsetAsync(rebuild_words_.p, 0, rebuild_words_.n * sizeof(unsigned long long), stream_) !=
-                hipSuccess ||
-            launch_fill_int(count_.p, 0, (size_t)ncells_, stream_) != hipSuccess)
-            return FM_ERR_HIP;
-        primed_ = false;
-        ene_valid_ = false;
-        obs_valid_ = false;
-    }
     (void)hipMemsetAsync(err_.p, 0, sizeof(uint32_t), stream_);
     (void)hipStreamSynchronize(stream_);
-    pin_.head()->err = 0;
     return FM_OK;
 }
 

@@ -1202,11 +1202,13 @@ __device__ __forceinline__ void sort_block(const ScanArgs &a, int b, uint32_t ep
     __syncthreads();
     const int carry = S.carry;
     if (mine) {
-        const int st = S.st[t] >= 0 ? S.st[t] : carry + ex;
+        // (counts that add up past the replica's particles, reported below:
+        // no start beyond its last)
+        const int st = min(S.st[t] >= 0 ? S.st[t] : carry + ex, R.p1);
         // list mode: only the rebuilding replicas' cell starts change (the
         // others' lists index staging laid out by their own last starts)
         if (!a.ctl || a.ctl[r].flag) put<kThrough>(a.start + c, st);
-        if (c == a.ncells - 1) put<kThrough>(a.start + a.ncells, st + n);
+        if (c == a.ncells - 1) put<kThrough>(a.start + a.ncells, min(st + n, R.p1));
     }
     auto store = [&](SortEntries &s, const Row &o) {
         int pos[kSortBatch];
@@ -2249,7 +2251,7 @@ __device__ __forceinline__ void phase_done(unsigned long long *sync, int k, unsi
 // Waits for phase k's go, then sees its writes.  False: the wait was given up
 // (uniform).  It runs out after rb.spins polls; a workgroup that gives up
 // leaves its phase's counter short, so no later go of that phase comes until
-// Engine::clear_errors has put the words back, and a later rebuild of the run
+// the host, told of it, has put the words back, and a later rebuild of the run
 // gives up once it finds the stall reported (looked for every 4096 polls, some
 // milliseconds, where the bound takes seconds; a look at the ticket instead
 // cost every rebuild of 114,140 particles 2 us).  Its binning adds to one not

@@ -1,6 +1,6 @@
 """A rebuild whose waits are given up (the bound set to no polls at all, so
-every kernel ends at once): the run reports it, further runs of the handle end
-without waiting to their bound, and after clear_errors the handle steps as one
+every kernel ends at once): the run reports it, further runs of the handle give
+up without waiting to their bound, and after clear_errors the handle steps as one
 that never stalled, bitwise, through many more rebuilds."""
 import time
 
@@ -50,6 +50,14 @@ def test_a_stalled_rebuild_is_recovered(build):
     assert time.perf_counter() - t < 1.0
     a.clear_errors()
     assert a.device_errors() == 0
+    # a stall in the first of a recorded trajectory's segments, whose next
+    # ones bin and sort without the host between
+    assert lib.fm_test_rebuild_spins(a.handle, 0) == 0
+    a.set_state(*start)
+    with pytest.raises(FemmdError, match="timed out"):
+        a.adjoint_forward(160, 40)
+    assert lib.fm_test_rebuild_spins(a.handle, -1) == 0
+    a.clear_errors()
     a.set_state(*start)
     for s in (a, b):
         n0 = s.list_stats()["rebuilds"]
