@@ -455,7 +455,9 @@ class System:
 
     def profile(self, nsteps: int = 10) -> dict:
         """Per-step device ms of each kernel (its dispatch's start and end
-        timestamps) and of the whole step body."""
+        timestamps) and of the whole step body.  Binning, sort and list build
+        are launched apart here, also for a small single system, whose run()
+        takes them as one kernel: "step" is then longer than run()'s."""
         ms = (C.c_double * 6)()
         self._check(self._lib.fm_profile_step(self._h, int(nsteps), ms))
         return dict(zip(("kick", "bin", "sort", "list_build", "forces", "step"), list(ms)))

@@ -103,7 +103,7 @@ struct ObsArgs {
                                // and ke_node over the node-kick spans (steps)
     const double *ke_part;     // 2 per kick span: sum m v^2, max v^2
     const double *ke_tile;     // 2 per tile: the same, particles kicked by the pair pass
-    const double *ke_node;     // 2 per node-kick span: the same, element / bond particles
+    const double *ke_node;     // 2 per node-kick span: the same, replicas without tiles
     const double *lj_part;     // 2 per tile: U, W
     const double *fea_part;    // 2 per element span: U, W
     const double *bond_part;   // 2 per bond span: U, W
@@ -223,9 +223,9 @@ struct DecideArgs {
 // systems let every binning workgroup take it for the replicas it meets.
 constexpr int kDecideMinReps = 8;
 
-// Single-pass counting sort: workgroup b scans cells [b * kSortCells, ...),
-// takes its carry-in from its predecessors' status words (decoupled
-// look-back) and scatters the particles of its own cells.
+// Single-pass counting sort: workgroup b scans cells [b * cells, ...), takes
+// its carry-in from its predecessors' status words (decoupled look-back) and
+// scatters the particles of its own cells.
 struct ScanArgs {
     const RepDesc *reps;
     int32_t nrep;
@@ -289,13 +289,17 @@ struct ElemArgs {
 
 // The one-kernel rebuild of a single replica (k_rebuild): its binning and
 // list-build workgroups, and its words, 128 bytes apart (a ticket counter, two
-// phase counters, eight go words per phase; never reset, every rebuild adds
-// the same counts).  At most kRebuildBins workgroups bin (more of them hold
-// each other's tickets up: 114,140 particles 446 workgroups 20.3 us a step,
-// 256 20.1, 160 19.9, 96 20.06).  Taken up to kRebuildMax workgroups, about
-// what is resident at once; a step against three kernels: 256 particles 16.1
-// -> 13.3 us, 4,367 16.9 -> 14.1, 30,011 16.3 -> 13.7, 56 k with elastomers
-// 18.9 -> 16.2, 114,140 (986 workgroups) 20.5 -> 19.9.
+// phase counters, eight go words per phase; every rebuild adds the same counts,
+// so they start again only with new tiles or after a stall).  At most
+// kRebuildBins workgroups bin (more of them hold each other's tickets up:
+// 114,140 particles 446 workgroups 20.3 us a step, 256 20.1, 160 19.9, 96
+// 20.06).  Taken up to kRebuildMax workgroups, about what is resident at once;
+// a step against three kernels: 256 particles 16.1 -> 13.3 us, 4,367 16.9 ->
+// 14.1, 30,011 16.3 -> 13.7, 56 k with elastomers 18.9 -> 16.2, 91,348 (767
+// workgroups) 18.8 -> 17.8, 114,140 (986) 20.6 -> 20.0.  Past the limit it was
+// still the faster one where measured, by as much (1039 workgroups 21.15 ->
+// 20.5, 1139 21.8 -> 21.2, 1466 23.9 -> 23.3): the limit is not where it stops
+// paying.
 constexpr int kRebuildSync = 16 * (3 + 2 * 8);
 constexpr int kRebuildBins = 160, kRebuildMax = 1024;
 constexpr int kRebuildSpins = 1 << 22;  // seconds: a wait takes under 0.1 ms

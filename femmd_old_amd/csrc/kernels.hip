@@ -320,13 +320,6 @@ __device__ void obs_finish(const ObsArgs &o, int r, bool accumulate) {
     ob[kObsRaw + 1 + kObsAvg + lane] += a * a;
 }
 
-// Bin one particle per lane into its cell's slot list (the reference's
-// atomic cell fill, femmd2D/src/nnCuda.cu:69-82, re-designed): runs of
-// equal cells among consecutive lanes -- the common case, since particles
-// are stored near their cell -- take one integer atomicAdd for the whole
-// run and hand out slots by lane offset.  Slot order within a cell is not
-// deterministic; the scatter below orders each cell by particle index.
-// All 64 lanes of the wavefront must call this (ballot / shuffles).
 // A store for later kernels (kept in this XCD's L2 until they start), or
 // (kThrough) written through to where every XCD reads it, for workgroups of
 // the same kernel.
@@ -356,6 +349,13 @@ __device__ __forceinline__ void put(float4 *p, float4 v) {
     } else *p = v;
 }
 
+// Bin one particle per lane into its cell's slot list (the reference's
+// atomic cell fill, femmd2D/src/nnCuda.cu:69-82, re-designed): runs of
+// equal cells among consecutive lanes -- the common case, since particles
+// are stored near their cell -- take one integer atomicAdd for the whole
+// run and hand out slots by lane offset.  Slot order within a cell is not
+// deterministic; the scatter below orders each cell by particle index.
+// All 64 lanes of the wavefront must call this (ballot / shuffles).
 template <bool kThrough = false>
 __device__ __forceinline__ void bin_wave_to(int32_t *count, int32_t *tmp, int cap, uint32_t *err,
                                             bool active, int p, int c) {
@@ -441,9 +441,10 @@ __device__ __forceinline__ void kick_particle(const RepDesc &R, float ax, float 
 // coalesced chunks through LDS and each lane adds its own particle's
 // entries in order (the same sums in the same order as reading its run
 // directly, which leaves each lane a strided walk of its own).  It pays
-// where the node kick is throughput-bound (many workgroups); with few, the
-// two barriers per chunk lengthen each workgroup's path and the direct
-// walk is faster.
+// where the node kick is throughput-bound (many workgroups, kGatherLdsSpans);
+// with few, the two barriers per chunk lengthen each workgroup's path and the
+// direct walk is faster.  (Its 16 KB of LDS hold no launch back: eight
+// workgroups of 256 threads fill a CU, 128 of 160 KB.)
 constexpr int kGatherChunk = 2048;
 __device__ __forceinline__ void gather_corners(const KickArgs &a, const Span &sp, int p,
                                                bool active, float &fx, float &fy) {
@@ -1963,13 +1964,17 @@ static_assert(mask_word(0u, 0) == 0u && mask_word(1u, 8) == 0x80u && mask_word(0
                   mask_word(0x80000001u, 32) == 0x80000001u,
               "no shift by the width of the word; the first candidate lowest");
 
-// List build of one staged tile; bound by vector issue.  Each row's
-// candidates (cells col-1 .. col+1, one contiguous run) are tested 32 at a
+// List build of one staged tile; bound by vector issue (38.9 M wavefront
+// instructions a rebuild of 1.14 million particles, 63 of its 85 us; under a
+// third of them test candidates, the rest rank and take out the lists and
+// bring spilled scalars back) with the latency it does not cover at five
+// wavefronts per SIMD.  Each row's candidates (cells col-1 .. col+1, one contiguous run) are tested 32 at a
 // time into a bit mask per lane, with a wavefront-uniform trip count (the
 // longest run among the lanes; bits past a lane's own run and of the centre
 // itself are cleared afterwards): six vector instructions per candidate (8
-// with an exclusion group in the wavefront), where a compaction store per
-// candidate took 14 and conflicted in LDS.  The masks wait until the chunk's
+// with an exclusion group in the wavefront).  A compaction store per candidate
+// took 14 of 37.1 M in all, so the gain lies in LDS: 2.5 instead of 4.9 M
+// instructions, 2.2 instead of 14.7 M cycles of conflicts.  The masks wait until the chunk's
 // lists are ranked -- in registers while every run of the wavefront is at
 // most 32 long, else in LDS (word w of lane t at mask[w * blockDim + t]) --
 // then each lane takes its set bits in order and stores its list in groups
@@ -2341,7 +2346,8 @@ typedef uint32_t v2u __attribute__((ext_vector_type(2)));
 // (femmd2D/src/interactionsCuda.cu:91-96), scaled per tile.
 // The loop over the list's groups runs to the longest list of the wavefront
 // (lists are ranked by length; a lane past its own list takes the padding
-// slot four times), so its control and the group addresses are scalar.
+// slot four times), so its control and the group addresses are scalar.  Two
+// groups past it are loaded and not used: 16 bytes a particle of its traffic.
 // What a lane needs of its list slot, loaded before the staging is waited
 // for: length word, internal id, the first two groups of entries.
 struct ListSlot {
@@ -2674,10 +2680,15 @@ __device__ void step_book(const ForceArgs &a, int b, int nb) {
 // closing second half-kick of a run; 2 forces, the second half-kick of this
 // step and the first half-kick, drift and wrap of the next
 // (femmd2D/src/integrator.cpp:8-29), for every particle (tile_kick).
-// Wavefronts per SIMD: the list pass 6 (5 with a type table), where what it
-// keeps in flight needs no spilled register (1.14 million particles: 38 us;
-// 39 at 7, 45 at 8 with 14 spilled, 42 at 5; 30,011 particles of six types:
-// 10.8 us at 5, 12.1 at 6); the cell walk 8.
+// Wavefronts per SIMD: the list pass 6 (5 with a type table), where a uniform
+// sigma needs no spilled register (1.14 million particles: 38 us; 39 at 7, 45
+// at 8 with 14 spilled, 42 at 5; 30,011 particles of six types: 10.8 us at 5,
+// 12.1 at 6).  One type with mixed sigmas spills 6 at 6 and is better at 5
+// (100,000 particles 17.9 us a step against 16.1, 1 million 52.3 against
+// 51.4), the cell walk spills 11 at 8 (mixed sigmas 9) and is better at 7 with
+// a uniform sigma only (114,140 particles 41.3 us a step against 39.7, 1.14
+// million 123.8 against 120.0; 1 million of mixed sigmas 153.4 against 155.3,
+// 163.8 at 6).  Neither line is drawn by these figures yet.
 template <bool kList, bool kTypes>
 constexpr int kForceWaves = kList ? (kTypes ? 5 : 6) : 8;
 template <bool kSigma, bool kTypes, bool kDebug, bool kList, bool kEnergy, int kKick>

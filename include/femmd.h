@@ -246,7 +246,11 @@ int fm_time_forces(fm_system *h, int32_t reps, double *ms);
  * force pass, except for replicas without pair forces), binning (list mode;
  * with the element and bond forces), counting sort (cell walk: with the
  * element and bond forces), list build, force pass (0 for a kernel the mode
- * does not launch), whole step with its share of the opening half-kick. */
+ * does not launch), whole step with its share of the opening half-kick.  A
+ * single list-mode system of up to about 115,000 particles takes binning, sort
+ * and list build as one kernel when it steps; here the three are launched and
+ * timed apart, and the whole step is theirs (skipped launches and boundaries
+ * included): what fm_step takes is timed around it. */
 int fm_profile_step(fm_system *h, int32_t nsteps, double *ms);
 /* Elastomer clusters (one per fm_add_elastomer call, in call order). */
 int fm_cluster_count(fm_system *h, int32_t *nc);
